@@ -1462,13 +1462,21 @@ int mmnb_decoder_prefill(mmnb_decoder *d, const int64_t *tokens, int64_t n,
   if ((rc = launch(ctx, kKernDecOps, k_embed_rows, dim3((unsigned)n), dim3(256), 0,
                    (const int64_t *)d->tok, (const float *)d->embed, H, d->x)))
     return rc;
-  // With more than 8 rows the projections take the MFMA GEMM; the norms and
-  // SwiGLU that feed them then write its prepared activations themselves
-  // (k_rmsnorm_prep, k_swiglu_prep) instead of fp32 rows for k_prep_a.
-  const bool fuse = ctx->prep_fuse && n > 8 && H <= kPrepMaxDim && I <= kPrepMaxDim;
+  // Projections of up to 32 rows read fp32 rows (the few-row kernel, or the
+  // GEMVs); beyond, they take the MFMA GEMM, and the norms and SwiGLU that feed
+  // it write its prepared activations themselves (k_rmsnorm_prep,
+  // k_swiglu_prep) instead of fp32 rows for k_prep_a.
+  const bool can_fuse = ctx->prep_fuse && H <= kPrepMaxDim && I <= kPrepMaxDim;
+  auto gemm = [&](const mmnb_pack *pk) { return n > 32 || (n > 8 && nbits_takes_gemm(ctx, pk, n)); };
+  auto fused = [&](const mmnb_pack *pk) { return can_fuse && gemm(pk); };
+  auto from_rows = [&](const mmnb_pack *pk, const float *a, int64_t lda, float *y) -> int {
+    return gemm(pk) ? launch_nbits_gemm(ctx, pk, a, lda, n, y)
+                    : launch_matmul_nbits(ctx, pk, a, lda, n, y);
+  };
   // x (+= add) normalised with gamma, as the input of the projection `next`
   auto norm_into = [&](const float *gamma, const float *add, const mmnb_pack *next) -> int {
-    if (!fuse) return launch_rmsnorm(ctx, d->x, n, H, gamma, eps, d->h, add, add ? d->x : nullptr);
+    if (!fused(next))
+      return launch_rmsnorm(ctx, d->x, n, H, gamma, eps, d->h, add, add ? d->x : nullptr);
     int64_t segsp = 0, mpad = 0;
     void *ap = nullptr;
     int *ex = nullptr;
@@ -1479,8 +1487,8 @@ int mmnb_decoder_prefill(mmnb_decoder *d, const int64_t *tokens, int64_t n,
                   segsp * kSegK, ex, (uint4 *)ap);
   };
   auto gemm_from_norm = [&](const mmnb_pack *pk, float *y) -> int {
-    return fuse ? launch_matmul_nbits_prepared(ctx, pk, n, y)
-                : launch_matmul_nbits(ctx, pk, d->h, H, n, y);
+    return fused(pk) ? launch_matmul_nbits_prepared(ctx, pk, n, y)
+                     : from_rows(pk, d->h, H, y);
   };
   if ((rc = norm_into(d->layers[0].ln1, nullptr, d->layers[0].qkv))) return rc;
   for (int64_t li = 0; li < c.layers; li++) {
@@ -1495,11 +1503,11 @@ int mmnb_decoder_prefill(mmnb_decoder *d, const int64_t *tokens, int64_t n,
     if ((rc = launch_attn_rows(ctx, d->q, nh * hd, 1, n, (int)nh, (int)kvh, (int)hd, ck, cv,
                                Lmax, P, scale, nullptr, 1, d->attn, nh * hd)))
       return rc;
-    if ((rc = launch_matmul_nbits(ctx, L.o, d->attn, nh * hd, n, d->tmp))) return rc;
+    if ((rc = from_rows(L.o, d->attn, nh * hd, d->tmp))) return rc;
     // x += o; h = rmsnorm(x)
     if ((rc = norm_into(L.ln2, d->tmp, L.gu))) return rc;
     if ((rc = gemm_from_norm(L.gu, d->gu))) return rc;
-    if (fuse) {
+    if (fused(L.down)) {
       int64_t segsp = 0, mpad = 0;
       void *ap = nullptr;
       int *ex = nullptr;
@@ -1513,7 +1521,7 @@ int mmnb_decoder_prefill(mmnb_decoder *d, const int64_t *tokens, int64_t n,
                        dim3((unsigned)((I + 255) / 256), (unsigned)n), dim3(256), 0,
                        (const float *)d->gu, I, d->act)))
         return rc;
-      if ((rc = launch_matmul_nbits(ctx, L.down, d->act, I, n, d->tmp))) return rc;
+      if ((rc = from_rows(L.down, d->act, I, d->tmp))) return rc;
     }
     // x += down, and (but after the last layer) the next layer's input norm
     if (li + 1 < c.layers) {

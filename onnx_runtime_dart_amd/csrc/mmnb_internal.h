@@ -39,6 +39,9 @@ constexpr int kSegK = 64;        // k per 32-byte segment
 constexpr int kSegBytes = 32;
 constexpr size_t kTailPad = 1024;  // bytes of slack after every device buffer
 constexpr int kGemmMaxSplitTiles = 1024;  // tiles of a K-sliced prefill GEMM
+constexpr int kSkMaxSlices = 8;      // K slices of a few-row product
+constexpr int kSkMaxGroups = 1024;   // its workgroups when it has K slices, at most
+constexpr int kSkTile = 32 * 64;     // floats of one workgroup's partial tile
 
 enum PackKind { kPackNBits = 1, kPackInteger = 2, kPackConv = 3 };
 
@@ -78,6 +81,9 @@ struct mmnb_ctx {
   // Per-tile arrival counters of the prefill GEMM's K slices (kGemmMaxSplitTiles
   // ints, zero at rest: the last slice of a tile resets its counter).
   int *d_gemm_cnt = nullptr;
+  // K-slice partials of the few-row products (kSkMaxGroups tiles of kSkTile
+  // floats, 8 MB), allocated with the context: those calls never grow scratch.
+  float *d_sk_part = nullptr;
   // Tuning override of the GEMV columns-per-lane R (MMNB_GEMV_R; 0 = auto).
   int gemv_r = 0;
   // Tuning override of the multi-row GEMV column groups per workgroup
@@ -119,6 +125,12 @@ struct mmnb_pack {
   int64_t k64 = 0;        // k padded to a multiple of 64 (and >= n_blocks*block)
   int64_t col_bytes = 0;  // bytes per column in d_w (= k64 / 2)
   uint8_t *d_w = nullptr;
+  // the same weights for the matrix-core kernels, a second copy in their
+  // operand order: 1 KB units [ceil(n / 32)][k64 / 64], lane l of a unit
+  // holding the 16-byte half l / 32 of column l % 32's segment (zeros past
+  // column n).  In d_w, where a column is one run, a wave's operand load
+  // touches 64 lines for 16 bytes each.
+  uint8_t *d_wt = nullptr;
   float *d_scales = nullptr;
   uint8_t *d_zp = nullptr;  // packed uint4; 0x88 filler when the op has none
   // block-major copies for the prefill GEMM, one allocation of rows
@@ -283,6 +295,12 @@ int pack_nbits_any(mmnb_ctx *ctx, const uint8_t *b_q, const float *scales,
                    mmnb_pack **out);
 // Block sizes the fast kernels take as they are (powers of two >= 16).
 bool nbits_block_native(int64_t bs);
+// MatMulNBits of a few rows in one launch (no scratch; K-slice partials and
+// counters of the context): whether a call should take it, with its column
+// waves cw and K slices nsl, and the launch.
+bool nbits_skinny_plan(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, int *cw, int *nsl);
+int launch_nbits_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
+                        int64_t m, float *d_y, int cw, int nsl);
 // MatMulNBits on a generic pack (no scratch; the reference's order and bits).
 int launch_nbits_generic(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
                          int64_t m, float *d_y);
@@ -296,6 +314,11 @@ int run_matmul_nbits(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_
 // MatMulNBits: y[m, n] = a[m, k] * W;  lda = row stride of a (elements).
 int launch_matmul_nbits(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a,
                         int64_t lda, int64_t m, float *d_y);
+// Whether launch_matmul_nbits takes the prefill GEMM for m rows, and that path
+// (activation prep, GEMM) whatever it would take.
+bool nbits_takes_gemm(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m);
+int launch_nbits_gemm(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
+                      int64_t m, float *d_y);
 // The prefill GEMM (M > 8) with its activations prepared by the caller's own
 // kernel instead of k_prep_a: gemm_prepared_a returns where to write them
 // (scratch: the hi/lo fp16 units, [mpad / 32][segsp][4][2] x 1 KB, and the
@@ -365,7 +388,7 @@ int launch_probe_read(mmnb_ctx *ctx, const void *d_buf, size_t bytes);
 int build_gemm_sz(mmnb_ctx *ctx, mmnb_pack *p);
 int repack_nbits_weights(mmnb_ctx *ctx, const uint8_t *d_src, int64_t n,
                          int64_t k, int64_t src_col_bytes,
-                         int64_t dst_col_bytes, uint8_t *d_dst);
+                         int64_t dst_col_bytes, uint8_t *d_dst, uint8_t *d_dst_t);
 // B [batch, k, n] row-major, or [batch, n, k] with b_trans (a convolution
 // weight, output channel major).  Zero points: bzp_len 0, 1, n (per column,
 // shared by the batches) or batch*n (per column of each batch; d_ecol then

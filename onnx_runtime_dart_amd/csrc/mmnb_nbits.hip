@@ -22,23 +22,6 @@ static int ilog2(int64_t v) {
   return r;
 }
 
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef float float16_t __attribute__((ext_vector_type(16)));
-typedef float f4vec __attribute__((ext_vector_type(4)));
-typedef int i4vec __attribute__((ext_vector_type(4)));
-typedef unsigned u4vec __attribute__((ext_vector_type(4)));
-
-// 16 bytes of a packed weight column for the GEMVs, which read every weight
-// once per call: a non-temporal load (nt), so the stream does not displace
-// the lines that are read again (activations, scales, zero points) and is
-// not kept where the next call's weights would have to evict it.  Against
-// plain loads, the M = 1 GEMV at K = N = 4096 (block 128, packs rotated past
-// the caches) went from 4.60 to 4.40 us per call, at K = N = 16384 from 33.8
-// to 32.8 us; the scales loaded the same way were slower (4.42 us).
-__device__ __forceinline__ u4vec ld_weights16(const uint8_t *p) {
-  return __builtin_nontemporal_load((const u4vec *)p);
-}
 __device__ __forceinline__ uint4 ld_weights16_u4(const uint8_t *p) {
   const u4vec v = ld_weights16(p);
   return make_uint4(v.x, v.y, v.z, v.w);
@@ -61,18 +44,19 @@ __device__ __forceinline__ int zp_of(const uint8_t *__restrict__ Z, int64_t zi) 
 // ---------------------------------------------------------------------------
 __global__ void k_repack_nbits(const uint8_t *__restrict__ src, int64_t n,
                                int64_t src_col, int64_t dst_col, int64_t K,
-                               uint8_t *__restrict__ dst) {
+                               uint8_t *__restrict__ dst, uint8_t *__restrict__ dst_t) {
   const int64_t segs = dst_col / kSegBytes;
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= n * segs) return;
+  if (idx >= (n + 31) / 32 * 32 * segs) return;
   const int64_t col = idx / segs, s = idx % segs;
+  if (col >= n && !dst_t) return;
   const uint8_t *cs = src + col * src_col;
   uint32_t d[8];
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     const int64_t off = s * kSegBytes + 4 * i;
     uint32_t v = 0;
-    if (off + 4 <= src_col) {
+    if (off + 4 <= src_col && col < n) {
       v = (uint32_t)cs[off] | ((uint32_t)cs[off + 1] << 8) |
           ((uint32_t)cs[off + 2] << 16) | ((uint32_t)cs[off + 3] << 24);
     }
@@ -82,25 +66,27 @@ __global__ void k_repack_nbits(const uint8_t *__restrict__ src, int64_t n,
     else if (valid < 8) v &= (1u << (4 * valid)) - 1u;
     d[i] = v;
   }
-  uint32_t *o = (uint32_t *)(dst + col * dst_col + s * kSegBytes);
-  o[0] = d[0];
-  o[1] = d[2];
-  o[2] = d[4];
-  o[3] = d[6];
-  o[4] = d[1];
-  o[5] = d[3];
-  o[6] = d[5];
-  o[7] = d[7];
+  const u4vec lo = {d[0], d[2], d[4], d[6]}, hi = {d[1], d[3], d[5], d[7]};
+  if (col < n) {
+    u4vec *o = (u4vec *)(dst + col * dst_col + s * kSegBytes);
+    o[0] = lo;
+    o[1] = hi;
+  }
+  if (dst_t) {
+    u4vec *o = (u4vec *)dst_t + ((col >> 5) * segs + s) * 64 + (col & 31);
+    o[0] = lo;
+    o[32] = hi;
+  }
 }
 
 int repack_nbits_weights(mmnb_ctx *ctx, const uint8_t *d_src, int64_t n, int64_t k,
-                         int64_t src_col, int64_t dst_col, uint8_t *d_dst) {
+                         int64_t src_col, int64_t dst_col, uint8_t *d_dst, uint8_t *d_dst_t) {
   const int64_t segs = dst_col / kSegBytes;
-  const int64_t total = n * segs;
+  const int64_t total = (n + 31) / 32 * 32 * segs;
   const int threads = 256;
   const int64_t blocks = (total + threads - 1) / threads;
   return launch(ctx, kKernRepack, k_repack_nbits, dim3((unsigned)blocks), dim3(threads), 0,
-                d_src, n, src_col, dst_col, k, d_dst);
+                d_src, n, src_col, dst_col, k, d_dst, d_dst_t);
 }
 
 // ---------------------------------------------------------------------------
@@ -137,39 +123,6 @@ int build_gemm_sz(mmnb_ctx *ctx, mmnb_pack *p) {
   return launch(ctx, kKernRepack, k_sz_block_major, dim3((unsigned)blocks), dim3(threads), 0,
                 (const float *)p->d_scales, (const uint8_t *)p->d_zp, p->n, p->n_blocks,
                 p->ldsz, (uint32_t *)p->d_st);
-}
-
-// (a & mask) | orv in one VALU op.  gfx9 VOP3 takes no literal, so the
-// compiler splits this into v_and + v_or; with the mask in an SGPR and the
-// magic in a VGPR it is one v_and_or_b32.
-__device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t mask, uint32_t orv) {
-  uint32_t r;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(mask), "v"(orv));
-  return r;
-}
-
-// 8 nibbles of one dword -> 8 fp16 values (q - zp), exact.  (q | 0x6400)
-// as fp16 is 1024 + q; (16q | 0x6400) is 1024 + 16q, so
-//   lo nibble pairs: (1024 + q) - (1024 + zp)
-//   hi nibble pairs: (1024 + 16q) / 16 - (64 + zp)
-// Output order {n0, n4, n1, n5, n2, n6, n3, n7}; the prepared activations
-// use the same k permutation.
-__device__ __forceinline__ half8_t dequant8(uint32_t w, int zp, uint32_t magic) {
-  const uint32_t t0 = and_or(w, 0x000F000Fu, magic);
-  const uint32_t t1 = and_or(w, 0x00F000F0u, magic);
-  const uint32_t w8 = w >> 8;
-  const uint32_t t2 = and_or(w8, 0x000F000Fu, magic);
-  const uint32_t t3 = and_or(w8, 0x00F000F0u, magic);
-  // 1024 + zp and 64 + zp (zp <= 15) as fp16 bits: ulp 1 at 1024, 1/16 at 64
-  const half2_t zz = __builtin_bit_cast(half2_t, (uint32_t)(0x6400 + zp) * 0x10001u);
-  const half2_t zs = __builtin_bit_cast(half2_t, (uint32_t)(0x5400 + (zp << 4)) * 0x10001u);
-  const half2_t sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
-  const half2_t h0 = __builtin_bit_cast(half2_t, t0) - zz;
-  const half2_t h1 = __builtin_bit_cast(half2_t, t1) * sixteenth - zs;
-  const half2_t h2 = __builtin_bit_cast(half2_t, t2) - zz;
-  const half2_t h3 = __builtin_bit_cast(half2_t, t3) * sixteenth - zs;
-  half8_t r = {h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
-  return r;
 }
 
 // ---------------------------------------------------------------------------
@@ -678,7 +631,8 @@ int launch_dec_gemv_attn(mmnb_ctx *ctx, const mmnb_pack *p, const DecAttnPartial
 }
 
 // ---------------------------------------------------------------------------
-// Decode-shape GEMV for 2 <= M <= 8, activations staged in LDS.
+// Decode-shape GEMV for 2 <= M <= 4 and small weights (gemv_multi_takes),
+// activations staged in LDS.
 //
 // Holding a chunk's 32 activations per row in registers (the M = 1 kernel)
 // costs 32*M VGPRs and re-reads A through L1 for every pair of columns; at
@@ -929,9 +883,6 @@ static int launch_gemv_lds_m(mmnb_ctx *ctx, int R, int nbpc, dim3 grid, dim3 blo
 }
 
 
-static int launch_gemm(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
-                       int64_t m, float *d_y);
-
 // Waves splitting K (kw), chunk iterations and staged-activation LDS bytes
 // of the multi-row GEMV for M rows.
 static size_t gemv_multi_lds(const mmnb_pack *p, int64_t m, int *kw_out, int *iters_out) {
@@ -947,20 +898,29 @@ static size_t gemv_multi_lds(const mmnb_pack *p, int64_t m, int *kw_out, int *it
   return (size_t)m * 8 * (cs + 1) * 16;
 }
 
-// Whether 2 <= M <= 8 rows of A fit the multi-row GEMV's LDS (the kernel
-// also holds a static 8 x M x 8 float reduction buffer).
+// Whether the M rows of A fit the multi-row GEMV's LDS (the kernel also holds
+// a static 8 x M x 8 float reduction buffer).
 static bool gemv_multi_fits(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m) {
   return gemv_multi_lds(p, m, nullptr, nullptr) + 8 * 8 * 8 * 4 <= (size_t)ctx->lds_max;
 }
 
-// 2 <= M <= 8: the LDS-staged kernel, or the MFMA GEMM when A does not fit
-// the workgroup's LDS.
+// Whether a call of 2 <= M <= 4 rows takes the multi-row GEMV: its rows fit
+// LDS and the weight is small but K longer than two chunks of the matrix-core kernel
+// (us there and here: M = 2, (2048, 4096) 6.7 and 5.1, (4096, 4096) 8.5 and
+// 7.5; M = 4, (2048, 2048) 5.8 and 5.5; but M = 3, (1024, 4096) 4.5 and 4.6,
+// (3072, 8192) 9.5 and 11.4; M = 4, 4096^2 8.5 and 9.7).
+static bool gemv_multi_takes(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m) {
+  return m >= 2 && m <= 4 && p->k64 > 1024 &&
+         p->n * p->col_bytes <= (int64_t)(m <= 3 ? 8 : 4) << 20 &&
+         gemv_multi_fits(ctx, p, m);
+}
+
+// 2 <= M <= 4 (gemv_multi_takes).
 static int launch_gemv_multi(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a,
                              int64_t lda, int64_t m, float *d_y) {
   const int C = (int)(p->col_bytes / 16);
   int kw, iters;
   const size_t shmem = gemv_multi_lds(p, m, &kw, &iters);
-  if (!gemv_multi_fits(ctx, p, m)) return launch_gemm(ctx, p, d_a, lda, m, d_y);
   const int64_t n = p->n;
   // Every workgroup stages all of A, so fewer, wider workgroups win: up to
   // 8 waves (cg column groups of kw waves), then the most columns per lane
@@ -984,10 +944,6 @@ static int launch_gemv_multi(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a
     MMNB_CASE(2)
     MMNB_CASE(3)
     MMNB_CASE(4)
-    MMNB_CASE(5)
-    MMNB_CASE(6)
-    MMNB_CASE(7)
-    MMNB_CASE(8)
 #undef MMNB_CASE
     default:
       return fail(MMNB_ERR_ARG, "GEMV: M out of range");
@@ -995,8 +951,7 @@ static int launch_gemv_multi(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a
 }
 
 static int launch_gemv(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
-                       int64_t m, float *d_y) {
-  if (m > 1) return launch_gemv_multi(ctx, p, d_a, lda, m, d_y);
+                       float *d_y) {
   const int C = (int)(p->col_bytes / 16);  // chunks per column
   // waves splitting K: one chunk per lane up to 4 waves, then iterate
   int nw = (C + 31) / 32;
@@ -1806,8 +1761,8 @@ static int gemm_ctx_part(mmnb_ctx *ctx, const GemmPlan &pl, void **d_part) {
   return pb ? scratch_get(ctx, 10, pb, d_part) : MMNB_OK;
 }
 
-static int launch_gemm(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
-                       int64_t m, float *d_y) {
+int launch_nbits_gemm(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
+                      int64_t m, float *d_y) {
   GemmPlan pl;
   int rc;
   if ((rc = gemm_plan(ctx, p, m, pl))) return rc;
@@ -1845,19 +1800,50 @@ int launch_matmul_nbits_prepared(mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, f
   return gemm_run(ctx, p, m, pl, d_ap, d_exp, d_y, d_part, ctx->d_gemm_cnt);
 }
 
+// Which kernel takes a call.  The GEMM's tuning overrides send every call of
+// several rows to it.
+enum NbitsRoute { kRouteGeneric, kRouteGemv, kRouteGemvMulti, kRouteSkinny, kRouteGemm };
+static NbitsRoute nbits_route(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, int *cw,
+                              int *nsl) {
+  if (p->generic) return kRouteGeneric;
+  if (m == 1) return kRouteGemv;
+  if (ctx->gemm_cb || ctx->gemm_ksplit || ctx->gemm_stages != 2) return kRouteGemm;
+  if (gemv_multi_takes(ctx, p, m)) return kRouteGemvMulti;
+  return nbits_skinny_plan(ctx, p, m, cw, nsl) ? kRouteSkinny : kRouteGemm;
+}
+
+bool nbits_takes_gemm(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m) {
+  int cw, nsl;
+  return nbits_route(ctx, p, m, &cw, &nsl) == kRouteGemm;
+}
+
+// The kernels that need no scratch (everything but the prefill GEMM): launches
+// and returns true with the status in *rc, or returns false.
+static bool launch_no_scratch(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
+                              int64_t m, float *d_y, int *rc) {
+  int cw, nsl;
+  switch (nbits_route(ctx, p, m, &cw, &nsl)) {
+    case kRouteGeneric: *rc = launch_nbits_generic(ctx, p, d_a, lda, m, d_y); return true;
+    case kRouteGemv: *rc = launch_gemv(ctx, p, d_a, lda, d_y); return true;
+    case kRouteGemvMulti: *rc = launch_gemv_multi(ctx, p, d_a, lda, m, d_y); return true;
+    case kRouteSkinny: *rc = launch_nbits_skinny(ctx, p, d_a, lda, m, d_y, cw, nsl); return true;
+    default: return false;
+  }
+}
+
 // MatMulNBits with every scratch buffer carved from a caller's workspace
 // (ws, ws_bytes; 256-byte aligned): the GEMM's K-slice counters, row
 // exponents, prepared activations and K-slice partials, each followed by
 // kTailPad bytes of slack.  Allocates nothing.
 int launch_matmul_nbits_ws(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
                            int64_t m, float *d_y, void *ws, size_t ws_bytes) {
-  if (p->generic) return launch_nbits_generic(ctx, p, d_a, lda, m, d_y);  // no scratch
-  // the GEMVs use no scratch (the multi-row one falls back to the GEMM when A
-  // does not fit its LDS: that GEMM takes the workspace below)
-  if (m == 1 || (m <= 8 && gemv_multi_fits(ctx, p, m)))
-    return launch_gemv(ctx, p, d_a, lda, m, d_y);
-  GemmPlan pl;
   int rc;
+  // the workspace's M x K limit holds whichever kernel runs, except for M <= 8
+  // rows that fit a workgroup's LDS
+  if ((p->generic || m == 1 || (m <= 8 && gemv_multi_fits(ctx, p, m))) &&
+      launch_no_scratch(ctx, p, d_a, lda, m, d_y, &rc))
+    return rc;
+  GemmPlan pl;
   if ((rc = gemm_plan(ctx, p, m, pl))) return rc;
   auto up = [](size_t b) { return (b + kTailPad + 255) / 256 * 256; };
   const size_t o_cnt = 0;
@@ -1870,6 +1856,7 @@ int launch_matmul_nbits_ws(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, 
                 "MatMulNBits: this M x K needs " + std::to_string(need) +
                     " bytes of scratch, more than the " + std::to_string(ws_bytes) +
                     "-byte fixed workspace");
+  if (launch_no_scratch(ctx, p, d_a, lda, m, d_y, &rc)) return rc;
   char *b = (char *)ws;
   int *d_cnt = (int *)(b + o_cnt);
   const int nclear = pl.ksplit > 1 ? (int)pl.tiles : 0;
@@ -1882,9 +1869,9 @@ int launch_matmul_nbits_ws(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, 
 
 int launch_matmul_nbits(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
                         int64_t m, float *d_y) {
-  if (p->generic) return launch_nbits_generic(ctx, p, d_a, lda, m, d_y);
-  if (m <= 8) return launch_gemv(ctx, p, d_a, lda, m, d_y);
-  return launch_gemm(ctx, p, d_a, lda, m, d_y);
+  int rc;
+  if (launch_no_scratch(ctx, p, d_a, lda, m, d_y, &rc)) return rc;
+  return launch_nbits_gemm(ctx, p, d_a, lda, m, d_y);
 }
 
 }  // namespace mmnb

@@ -155,12 +155,15 @@ int mmnb_init(int device, mmnb_ctx **out) {
   if (e == hipSuccess) e = hipMemset((char *)ctx->d_pad + 2048, 0, 2048);
   if (e == hipSuccess) e = hipMalloc((void **)&ctx->d_gemm_cnt, kGemmMaxSplitTiles * sizeof(int));
   if (e == hipSuccess) e = hipMemset(ctx->d_gemm_cnt, 0, kGemmMaxSplitTiles * sizeof(int));
+  if (e == hipSuccess)
+    e = hipMalloc((void **)&ctx->d_sk_part, (size_t)kSkMaxGroups * kSkTile * sizeof(float));
   if (e == hipSuccess) e = hipDeviceSynchronize();
   if (e != hipSuccess) {
     if (ctx->d_pad) (void)hipFree(ctx->d_pad);
     if (ctx->d_gemm_cnt) (void)hipFree(ctx->d_gemm_cnt);
+    if (ctx->d_sk_part) (void)hipFree(ctx->d_sk_part);
     delete ctx;
-    return check_hip(e, "hipMalloc(pad page, GEMM counters)");
+    return check_hip(e, "hipMalloc(pad page, GEMM counters, few-row partials)");
   }
   // The fixed workspace serves only mmnb_matmul_nbits_dev_noalloc: when it
   // cannot be resolved the context still opens, and that entry point reports
@@ -187,6 +190,7 @@ int mmnb_shutdown(mmnb_ctx *ctx) {
       if (s.ptr) (void)hipFree(s.ptr);
     if (ctx->d_pad) (void)hipFree(ctx->d_pad);
     if (ctx->d_gemm_cnt) (void)hipFree(ctx->d_gemm_cnt);
+    if (ctx->d_sk_part) (void)hipFree(ctx->d_sk_part);
     for (auto &ev : ctx->events)
       if (ev) (void)hipEventDestroy(ev);
     for (auto &ev : ctx->tev) (void)hipEventDestroy(ev);
@@ -233,6 +237,7 @@ int mmnb::pack_nbits_core(mmnb_ctx *ctx, const uint8_t *b_q, const float *scales
   p->col_bytes = p->k64 / 2;
   auto cleanup = [&](int code) {
     if (p->d_w) (void)hipFree(p->d_w);
+    if (p->d_wt) (void)hipFree(p->d_wt);
     if (p->d_scales) (void)hipFree(p->d_scales);
     if (p->d_zp) (void)hipFree(p->d_zp);
     if (p->d_st) (void)hipFree(p->d_st);  // d_zt lies inside it
@@ -241,6 +246,8 @@ int mmnb::pack_nbits_core(mmnb_ctx *ctx, const uint8_t *b_q, const float *scales
   };
   const size_t wbytes = (size_t)(n * p->col_bytes);
   if ((rc = device_alloc(wbytes, (void **)&p->d_w))) return cleanup(rc);
+  const size_t wtbytes = (size_t)((n + 31) / 32 * 32 * p->col_bytes);
+  if ((rc = device_alloc(wtbytes, (void **)&p->d_wt))) return cleanup(rc);
   if ((rc = device_alloc((size_t)(n * nb) * 4, (void **)&p->d_scales))) return cleanup(rc);
   p->has_zp = zero_points != nullptr || zp_fill != 0x88;
   if ((rc = device_alloc((size_t)zp_need, (void **)&p->d_zp))) return cleanup(rc);
@@ -252,7 +259,7 @@ int mmnb::pack_nbits_core(mmnb_ctx *ctx, const uint8_t *b_q, const float *scales
                           ctx->stream)) != hipSuccess)
     return cleanup(check_hip(e, "hipMemcpyAsync(B)"));
   if ((rc = repack_nbits_weights(ctx, (const uint8_t *)d_raw, n, k, src_col, p->col_bytes,
-                                 p->d_w)))
+                                 p->d_w, p->d_wt)))
     return cleanup(rc);
   if ((e = hipMemcpyAsync(p->d_scales, scales, (size_t)(n * nb) * 4,
                           hipMemcpyHostToDevice, ctx->stream)) != hipSuccess)
@@ -268,7 +275,7 @@ int mmnb::pack_nbits_core(mmnb_ctx *ctx, const uint8_t *b_q, const float *scales
   if ((rc = build_gemm_sz(ctx, p))) return cleanup(rc);
   if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess)
     return cleanup(check_hip(e, "hipStreamSynchronize(pack)"));
-  p->bytes = (int64_t)wbytes + n * nb * 4 + zp_need + p->ldsz * nb * 8;
+  p->bytes = (int64_t)(wbytes + wtbytes) + n * nb * 4 + zp_need + p->ldsz * nb * 8;
   p->k_in = k;
   ctx->live_packs++;
   *out = p;
@@ -623,6 +630,7 @@ int mmnb_pack_free(mmnb_pack *p) {
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     if (p->d_w) (void)hipFree(p->d_w);
+    if (p->d_wt) (void)hipFree(p->d_wt);
     if (p->d_scales) (void)hipFree(p->d_scales);
     if (p->d_zp) (void)hipFree(p->d_zp);
     if (p->d_st) (void)hipFree(p->d_st);  // d_zt lies inside it

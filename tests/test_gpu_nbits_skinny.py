@@ -1,0 +1,69 @@
+"""The few-row MatMulNBits kernel where it can go wrong: every row layout at its
+edges (one, two and three split terms, several row groups), ragged K (a chunk
+cut short, an odd K, a block longer than K) and N, every block size class, K
+slices, and activations that are not 16-byte aligned.
+
+Bar as in test_gpu_mmnb.py: normwise 1e-5 against the oracle and
+gamma_{K+2} sum|a||W| against the 64-bit product; reruns give the same bits.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import refcpu
+from onnx_runtime_dart_amd import _lib, ops, synth
+from onnx_runtime_dart_amd._lib import check
+from tests.helpers import normwise_rel_err
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0 ** -24
+
+CASES = [
+    # m, k, n, block, zp
+    (2, 512, 33, 16, True),        # one chunk, one segment per k wave
+    (5, 1001, 70, 32, True),       # odd K
+    (8, 96, 1, 64, False),         # last row of the three-term layout, one column
+    (9, 1000, 3001, 32, True),     # first row of the two-term layout, K % 8 == 0
+    (16, 2048, 130, 128, True),    # four chunks
+    (17, 520, 64, 16, True),       # first row of the two-pass layout, 8 k in chunk 2
+    (32, 4096, 100, 32, True),     # K slices
+    (6, 5120, 65, 256, False),     # K slices of uneven length
+    (33, 1024, 65, 32, True),      # two row groups
+    (200, 640, 96, 64, True),      # seven row groups
+    (70, 4096, 64, 128, False),    # row groups with K slices
+    (4, 300, 40, 1024, True),      # a block longer than K
+    (3, 2500, 31, 16, False),
+]
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("m,k,n,block,zp", CASES)
+def test_few_rows(m, k, n, block, zp, offset):
+    ctx = _lib.default_context()
+    p = synth.mmnb_problem(m, k, n, block, zp, seed=m + k + n, outlier_frac=0.01)
+    pack = ops.pack_nbits(p.b_q, p.scales, p.zero_points, k=k, n=n, bits=4, block_size=block,
+                          ctx=ctx)
+    # offset 1: rows that start 4 bytes past a 16-byte boundary
+    host = np.zeros(m * k + offset, np.float32)
+    host[offset:] = p.a.ravel()
+    da, dy = ctx.to_device(host), ctx.alloc(m * n * 4)
+    try:
+        def run():
+            dy.upload(np.full(m * n, np.nan, np.float32))
+            check(ctx.lib.mmnb_matmul_nbits_dev(
+                ctx.handle, pack.handle, ctypes.c_void_p(da.ptr.value + 4 * offset), m, dy.ptr))
+            ctx.synchronize()
+            return dy.numpy(np.float32, (m, n))
+        y = run()
+        ref = refcpu.matmul_nbits(p.a, p.b_q, p.scales, p.zero_points, k, n, 4, block, threads=8)
+        assert normwise_rel_err(y, ref) <= 1e-5
+        y64, absdot = refcpu.matmul_nbits_f64(p.a, p.b_q, p.scales, p.zero_points, k, n, block)
+        gam = (k + 2) * U / (1 - (k + 2) * U)
+        assert np.all(np.abs(y - y64) <= gam * absdot + 1e-30)
+        np.testing.assert_array_equal(run(), y)
+    finally:
+        da.free()
+        dy.free()
+        pack.free()
