@@ -164,7 +164,9 @@ int nbits_prepare(const mmnb_nbits_desc *d, NbitsHost *out) {
                 "block_size >= 16");
   // ---- the virtual 4-bit weight
   const uint8_t *B = d->b_q;
-  const int64_t kp = nb * bs;
+  // bits = 8: each nibble plane padded to whole 64-k segments (blocks of scale
+  // 0), so a row's two nibbles sit at the same place of their segments
+  const int64_t kp = bits == 8 ? (nb * bs + 63) / 64 * 64 : nb * bs;
   const int64_t kv = bits == 8 ? 2 * kp : k;
   const int64_t nbv = (kv + bs - 1) / bs;
   const int64_t vblob = bs / 2;
@@ -191,12 +193,14 @@ int nbits_prepare(const mmnb_nbits_desc *d, NbitsHost *out) {
         put(c, kk, q8 >> 4);
         put(c, kp + kk, q8 & 15);
       }
-    vs.resize((size_t)(n * nbv));
+    vs.assign((size_t)(n * nbv), 0.0f);
     for (int64_t c = 0; c < n; c++)
       for (int64_t b = 0; b < nb; b++) {
         vs[(size_t)(c * nbv + b)] = 16.0f * s[(size_t)(c * nb + b)];
-        vs[(size_t)(c * nbv + nb + b)] = s[(size_t)(c * nb + b)];
+        vs[(size_t)(c * nbv + nbv / 2 + b)] = s[(size_t)(c * nb + b)];
       }
+    out->bytes8 = zf.empty();
+    out->z8.assign(zi.begin(), zi.end());
     out->corr.assign((size_t)nnb, 0.0);
     for (int64_t c = 0; c < n; c++)
       for (int64_t b = 0; b < nb; b++) {

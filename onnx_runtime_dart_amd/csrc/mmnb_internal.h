@@ -157,6 +157,11 @@ struct mmnb_pack {
   float *d_corr = nullptr;    // [corr_nb, n]
   int64_t corr_nb = 0;
   float *d_bias = nullptr;    // [n]
+  // bits = 8 with integer zero points (k_gemv8): the two halves of a column
+  // hold the bytes' high and low nibbles; d_z8 the zero points [n][corr_nb]
+  // (null: 128)
+  bool bytes8 = false;
+  uint8_t *d_z8 = nullptr;
   // --- MatMulInteger
   int64_t batch = 0;
   int64_t kpad = 0;          // k padded to a multiple of 64
@@ -311,6 +316,10 @@ int run_matmul_nbits(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_
                      int64_t m, float *d_y);
 
 // Kernel launchers (return MMNB_OK or an error code) -------------------------
+// The M = 1 GEMV with the bias of an extended pack added where it is stored
+// (packs without gather and correction).
+int launch_gemv_bias(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
+                     float *d_y);
 // MatMulNBits: y[m, n] = a[m, k] * W;  lda = row stride of a (elements).
 int launch_matmul_nbits(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a,
                         int64_t lda, int64_t m, float *d_y);

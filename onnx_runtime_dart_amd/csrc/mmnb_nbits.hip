@@ -155,16 +155,19 @@ int build_gemm_sz(mmnb_ctx *ctx, mmnb_pack *p) {
 constexpr int kGemvMaxWaves = 4;   // M = 1 GEMV
 constexpr int kDecMaxWaves = 4;    // decoder-step GEMV (K <= 4096)
 
-template <int R, int NBPC, bool HAS_ZP, bool FAST>
+// BIAS adds bias[n] where a column is stored (an argument of its own kernel:
+// the plain call carries neither the pointer nor the load).
+template <int R, int NBPC, bool HAS_ZP, bool FAST, bool BIAS>
 __global__ __launch_bounds__(64 * kGemvMaxWaves) void k_gemv_valu(
     const float *__restrict__ A, const uint8_t *__restrict__ W, int64_t col_bytes,
     const float *__restrict__ S, const uint8_t *__restrict__ Z, int nb, int bs_log2, int K,
-    int N, float *__restrict__ Y, int C, int iters) {
+    int N, float *__restrict__ Y, int C, int iters, const float *__restrict__ bias) {
   __shared__ float red[kGemvMaxWaves][2 * R];
   // every kernel argument (and the block size) in SGPRs before anything
   // else: left to itself the compiler fetched them in two dependent rounds
   // of scalar loads ahead of the first weight load
   kernarg_fence(A, W, col_bytes, S, Z, nb, bs_log2, K, N, Y, C, iters, blockDim.x);
+  if constexpr (BIAS) kernarg_fence(bias);
   const int nw = blockDim.x >> 6;
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   const int h = l >> 5, t = l & 31;
@@ -179,6 +182,8 @@ __global__ __launch_bounds__(64 * kGemvMaxWaves) void k_gemv_valu(
   float acc[R];
 #pragma unroll
   for (int r = 0; r < R; r++) acc[r] = 0.0f;
+  float bv = 0.0f;
+  if constexpr (BIAS) bv = bias[min(col0 + (int)threadIdx.x, N - 1)];
 
   for (int it = 0; it < iters; it++) {
     const int c = 32 * w + t + it * 32 * nw;
@@ -268,18 +273,18 @@ __global__ __launch_bounds__(64 * kGemvMaxWaves) void k_gemv_valu(
     float v = 0.0f;
     for (int ww = 0; ww < nw; ww++) v += red[ww][threadIdx.x];
     const int col = col0 + threadIdx.x;
-    if (col < N) Y[col] = v;
+    if (col < N) Y[col] = BIAS ? v + bv : v;
   }
 }
 
-template <int R>
+template <int R, bool BIAS>
 static int launch_gemv_r(mmnb_ctx *ctx, int nbpc, dim3 grid, dim3 block, const float *A,
                          const mmnb_pack *p, float *Y, int C, int iters, bool fast,
                          int bs_log2) {
   const int nb = (int)p->n_blocks, K = (int)p->k, N = (int)p->n;
 #define MMNB_GEMV_LAUNCH(Q, ZP, F)                                                           \
-  return launch(ctx, kKernGemv, k_gemv_valu<R, Q, ZP, F>, grid, block, 0, A, p->d_w,         \
-                p->col_bytes, p->d_scales, p->d_zp, nb, bs_log2, K, N, Y, C, iters)
+  return launch(ctx, kKernGemv, k_gemv_valu<R, Q, ZP, F, BIAS>, grid, block, 0, A, p->d_w,   \
+                p->col_bytes, p->d_scales, p->d_zp, nb, bs_log2, K, N, Y, C, iters, p->d_bias)
 #define MMNB_GEMV_LAUNCH_Q(ZP, F)             \
   {                                          \
     if (nbpc == 4) MMNB_GEMV_LAUNCH(4, ZP, F); \
@@ -950,6 +955,7 @@ static int launch_gemv_multi(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a
   }
 }
 
+template <bool BIAS>
 static int launch_gemv(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
                        float *d_y) {
   const int C = (int)(p->col_bytes / 16);  // chunks per column
@@ -977,10 +983,18 @@ static int launch_gemv(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int6
   const bool f = (lda % 4 == 0) && (((uintptr_t)d_a & 15) == 0) && (lda >= p->k64);
   const int bs_log2 = ilog2(p->block);
   const int nbpc = p->block >= 64 ? 1 : (p->block == 32 ? 2 : 4);
-  if (R == 8) return launch_gemv_r<8>(ctx, nbpc, grid, block, d_a, p, d_y, C, iters, f, bs_log2);
-  if (R == 4) return launch_gemv_r<4>(ctx, nbpc, grid, block, d_a, p, d_y, C, iters, f, bs_log2);
-  if (R == 2) return launch_gemv_r<2>(ctx, nbpc, grid, block, d_a, p, d_y, C, iters, f, bs_log2);
-  return launch_gemv_r<1>(ctx, nbpc, grid, block, d_a, p, d_y, C, iters, f, bs_log2);
+#define MMNB_GEMV_R(RR) \
+  return launch_gemv_r<RR, BIAS>(ctx, nbpc, grid, block, d_a, p, d_y, C, iters, f, bs_log2)
+  if (R == 8) MMNB_GEMV_R(8);
+  if (R == 4) MMNB_GEMV_R(4);
+  if (R == 2) MMNB_GEMV_R(2);
+  MMNB_GEMV_R(1);
+#undef MMNB_GEMV_R
+}
+
+int launch_gemv_bias(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
+                     float *d_y) {
+  return launch_gemv<true>(ctx, p, d_a, lda, d_y);
 }
 
 // ---------------------------------------------------------------------------
@@ -1824,7 +1838,7 @@ static bool launch_no_scratch(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_
   int cw, nsl;
   switch (nbits_route(ctx, p, m, &cw, &nsl)) {
     case kRouteGeneric: *rc = launch_nbits_generic(ctx, p, d_a, lda, m, d_y); return true;
-    case kRouteGemv: *rc = launch_gemv(ctx, p, d_a, lda, d_y); return true;
+    case kRouteGemv: *rc = launch_gemv<false>(ctx, p, d_a, lda, d_y); return true;
     case kRouteGemvMulti: *rc = launch_gemv_multi(ctx, p, d_a, lda, m, d_y); return true;
     case kRouteSkinny: *rc = launch_nbits_skinny(ctx, p, d_a, lda, m, d_y, cw, nsl); return true;
     default: return false;

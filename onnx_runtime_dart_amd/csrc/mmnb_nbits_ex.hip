@@ -6,7 +6,8 @@
 // 4-bit weight of Kv rows), plus an optional A gather before and one
 // correction pass after the product:
 //
-//   bits = 8:  q8 = 16 hi + lo, so (q8 - z) s = (hi - 8)(16 s) + (lo - 8) s
+//   bits = 8:  (one row with integer zero points: k_gemv8, directly)
+//              q8 = 16 hi + lo, so (q8 - z) s = (hi - 8)(16 s) + (lo - 8) s
 //              + (136 - z) s.  The virtual weight stacks the hi plane (scale
 //              16 s, exact) over the lo plane (scale s), both with zero
 //              point 8, over Kv = 2 * ceil(K/bs) * bs rows; A is gathered as
@@ -28,6 +29,7 @@
 #include <string>
 #include <vector>
 
+#include "mmnb_device.h"
 #include "mmnb_host.h"
 #include "mmnb_internal.h"
 
@@ -130,9 +132,175 @@ __global__ __launch_bounds__(256) void k_nbits_correct_rows(
   }
 }
 
+// ---------------------------------------------------------------------------
+// One row of 8-bit weights with integer zero points, in one launch: the GEMV of
+// k_gemv_valu on the virtual weight's two planes at once.  A lane reads the
+// high and the low nibbles of the same 32 k of a column (one 16-byte chunk
+// each), joins them into bytes and multiplies the exact q - z, so A is neither
+// gathered nor corrected for, and the bias is added where the column is stored.
+//
+// Bound by the weight stream once K * N fills the chip, by the launch below
+// that.  R columns per lane as in k_gemv_valu, each of two chunks: R = 2.
+// K = N = 4096, block 128, bias: 14.8 us (gather of A, GEMV of the virtual weight,
+// correction) -> 5.1 us back to back, 3.4 TB/s of weights and scales.
+// ---------------------------------------------------------------------------
+constexpr int kGemv8Waves = 4;
+
+template <int R, int NBPC, bool HAS_ZP, bool FAST>
+__global__ __launch_bounds__(64 * kGemv8Waves) void k_gemv8(
+    const float *__restrict__ A, const uint8_t *__restrict__ W, int64_t col_bytes,
+    const float *__restrict__ S, const uint8_t *__restrict__ Z, const float *__restrict__ bias,
+    int nb, int bs_log2, int K, int N, float *__restrict__ Y, int C, int iters, int nbv) {
+  __shared__ float red[kGemv8Waves][2 * R];
+  kernarg_fence(A, W, col_bytes, S, Z, bias, nb, bs_log2, K, N, Y, C, iters, nbv, blockDim.x);
+  const int nw = blockDim.x >> 6;
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int h = l >> 5, t = l & 31;
+  const int col0 = blockIdx.x * (2 * R);
+  int colr[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) colr[r] = min(col0 + 2 * r + h, N - 1);
+  // without a bias its pointer is the scales': read and not used
+  const float bv = bias[min(col0 + (int)threadIdx.x, N - 1)];
+  float acc[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) acc[r] = 0.0f;
+  for (int it = 0; it < iters; it++) {
+    const int c = 32 * w + t + it * 32 * nw;
+    const bool cv = c < C;
+    const int cc = cv ? c : 0;
+    const int s = cc >> 1, g = cc & 1;
+    float av[32];
+    const float *ar = A + s * kSegK + 8 * g;
+    if constexpr (FAST) {
+      load_chunk32_paired(ar, h, av);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const int k = s * kSegK + 8 * g + 16 * j + e;
+          const float x = A[k < K ? k : K - 1];
+          av[8 * j + e] = (cv && k < K) ? x : 0.0f;
+        }
+    }
+    float sraw[R][NBPC], zraw[R][NBPC];
+    bool inb[NBPC];
+#pragma unroll
+    for (int q = 0; q < NBPC; q++) {
+      const int kq = s * kSegK + 16 * (q * (4 / NBPC)) + (NBPC == 4 ? 8 * g : 0);
+      int blk = kq >> bs_log2;
+      inb[q] = cv && blk < nb;
+      blk = blk < nb ? blk : nb - 1;
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        sraw[r][q] = S[(int64_t)colr[r] * nbv + (nbv >> 1) + blk];
+        zraw[r][q] = HAS_ZP ? (float)Z[(int64_t)colr[r] * nb + blk] : 128.0f;
+      }
+    }
+    u4vec wh[R], wl[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const uint8_t *wc = W + (int64_t)colr[r] * col_bytes + (int64_t)cc * 16;
+      wh[r] = ld_weights16(wc);
+      wl[r] = ld_weights16(wc + (col_bytes >> 1));
+    }
+    // every load in flight before any arithmetic, column by column after it
+    // (as k_gemv_valu)
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+#pragma unroll
+      for (int q = 0; q < NBPC; q++) {
+        float d = 0.0f;
+#pragma unroll
+        for (int jj = 0; jj < 4 / NBPC; jj++) {
+          const int j = q * (4 / NBPC) + jj;
+          const uint32_t hi = wh[r][j], lo = wl[r][j];
+          uint32_t ev = ((hi << 4) & 0xF0F0F0F0u) | (lo & 0x0F0F0F0Fu);
+          uint32_t od = (hi & 0xF0F0F0F0u) | ((lo >> 4) & 0x0F0F0F0Fu);
+          float qv[8];
+          if constexpr (HAS_ZP) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              qv[2 * e] = (float)((ev >> (8 * e)) & 255u) - zraw[r][q];
+              qv[2 * e + 1] = (float)((od >> (8 * e)) & 255u) - zraw[r][q];
+            }
+          } else {
+            ev ^= 0x80808080u;
+            od ^= 0x80808080u;
+            qv[0] = sbyte_f32<0>(ev); qv[1] = sbyte_f32<0>(od);
+            qv[2] = sbyte_f32<1>(ev); qv[3] = sbyte_f32<1>(od);
+            qv[4] = sbyte_f32<2>(ev); qv[5] = sbyte_f32<2>(od);
+            qv[6] = sbyte_f32<3>(ev); qv[7] = sbyte_f32<3>(od);
+          }
+#pragma unroll
+          for (int e = 0; e < 8; e++) d = fmaf(av[8 * j + e], qv[e], d);
+        }
+        acc[r] = inb[q] ? fmaf(sraw[r][q], d, acc[r]) : acc[r];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const float v = half_wave_sum(acc[r]);
+    if (t == 0) red[w][2 * r + h] = v;
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < 2 * R) {
+    float v = 0.0f;
+    for (int ww = 0; ww < nw; ww++) v += red[ww][threadIdx.x];
+    const int col = col0 + threadIdx.x;
+    if (col < N) Y[col] = bias != S ? v + bv : v;
+  }
+}
+
+template <int R, int NBPC>
+static int launch_gemv8_r(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, bool fast,
+                          float *d_y) {
+  const int C = (int)(p->col_bytes / 32);  // chunks of a plane
+  int nw = (C + 31) / 32, iters = 1;
+  if (nw > kGemv8Waves) {
+    iters = (nw + kGemv8Waves - 1) / kGemv8Waves;
+    nw = (C + 32 * iters - 1) / (32 * iters);
+  }
+  const int64_t n = p->n;
+  const dim3 grid((unsigned)((n + 2 * R - 1) / (2 * R))), block((unsigned)(64 * nw));
+  int bs_log2 = 0;
+  while ((int64_t(1) << bs_log2) < p->block) bs_log2++;
+  const float *bias = p->d_bias ? p->d_bias : p->d_scales;
+#define MMNB_GEMV8(ZP, F)                                                                     \
+  return launch(ctx, kKernGemv, k_gemv8<R, NBPC, ZP, F>, grid, block, 0, d_a, p->d_w,         \
+                p->col_bytes, p->d_scales, p->d_z8, bias, (int)p->corr_nb, bs_log2,           \
+                (int)p->k_in, (int)n, d_y, C, iters, (int)p->n_blocks)
+  if (p->d_z8) {
+    if (fast) MMNB_GEMV8(true, true);
+    MMNB_GEMV8(true, false);
+  }
+  if (fast) MMNB_GEMV8(false, true);
+  MMNB_GEMV8(false, false);
+#undef MMNB_GEMV8
+}
+
+static int launch_gemv8(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
+                        float *d_y) {
+  // float4 loads of whole chunks where the row fills the plane (col_bytes rows
+  // of the virtual weight); past K the joined bytes are not the zero point, so
+  // there the kernel zeroes the activations
+  const bool fast = lda % 4 == 0 && ((uintptr_t)d_a & 15) == 0 && p->k_in == p->col_bytes;
+  if (p->block >= 64) return launch_gemv8_r<2, 1>(ctx, p, d_a, fast, d_y);
+  if (p->block == 32) return launch_gemv8_r<2, 2>(ctx, p, d_a, fast, d_y);
+  return launch_gemv8_r<2, 4>(ctx, p, d_a, fast, d_y);
+}
+
 int run_matmul_nbits(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
                      int64_t m, float *d_y) {
   if (!p->ext) return launch_matmul_nbits(ctx, p, d_a, lda, m, d_y);
+  // one row: the GEMVs that take 8-bit weights and the bias in one launch
+  if (m == 1 && p->bytes8) return launch_gemv8(ctx, p, d_a, lda, d_y);
+  if (m == 1 && !p->d_asrc && !p->d_corr && p->d_bias)
+    return launch_gemv_bias(ctx, p, d_a, lda, d_y);
   int rc;
   const float *a2 = d_a;
   int64_t lda2 = lda, ka = p->k_in;
@@ -214,6 +382,8 @@ int mmnb_pack_nbits_ex(mmnb_ctx *ctx, const mmnb_nbits_desc *d, mmnb_pack **out)
       p->corr_nb = h.n_blocks;
     }
     if (!urc && !h.bias.empty()) urc = upload(p, h.bias, &p->d_bias);
+    p->bytes8 = h.bytes8;
+    if (!urc && !h.z8.empty()) urc = upload(p, h.z8, &p->d_z8);
   }
   if (urc) {
     (void)mmnb_pack_free(p);  // takes the context lock itself

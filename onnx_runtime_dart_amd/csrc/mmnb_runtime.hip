@@ -640,6 +640,7 @@ int mmnb_pack_free(mmnb_pack *p) {
     if (p->d_asrc) (void)hipFree(p->d_asrc);
     if (p->d_corr) (void)hipFree(p->d_corr);
     if (p->d_bias) (void)hipFree(p->d_bias);
+    if (p->d_z8) (void)hipFree(p->d_z8);
     ctx->live_packs--;
   }
   delete p;
