@@ -345,8 +345,8 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Epilogue operands of one lane: A's zero point for each of its 8 rows, and
-// per column (2 of them) the pack's zero-point terms, the fp32 rescale's B
-// scale and the requantisation's multiplier and bias.  Loaded at the start of
+// per column (2 of them) the pack's zero-point terms and the fp32 rescale's B
+// scale.  Loaded at the start of
 // the kernel, unconditionally (clamped indices; arrays a call does not use are
 // read from the zero page `pad`), so they arrive during the K loop instead of
 // as a chain of dependent round trips after it (a load under a branch ends in
@@ -355,8 +355,6 @@ struct MmiEpiIn {
   int32_t z[2][4];
   int32_t e[2], cs[2];
   float bs[2];
-  double mch[2];
-  int32_t bias[2];
   float as;
 };
 
@@ -368,7 +366,7 @@ __device__ __forceinline__ void mmi_epi_load(MmiEpiIn &in, int64_t bz, int64_t M
                                              const int32_t *__restrict__ azp, int64_t azp_len,
                                              const MmiEpi &o, const void *pad) {
   const int r16 = lane & 15, q = lane >> 4;
-  const bool zload = azp_len > 0 && !o.azp_is_const;
+  const bool zload = azp_len > 0;
   const int32_t *zp = zload ? azp : (const int32_t *)pad;
 #pragma unroll
   for (int i = 0; i < TI; i++)
@@ -381,9 +379,6 @@ __device__ __forceinline__ void mmi_epi_load(MmiEpiIn &in, int64_t bz, int64_t M
   const bool fy = o.yf != nullptr;
   in.as = (fy ? o.a_scale : (const float *)pad)[0];
   const float *bsp = fy ? o.b_scale : (const float *)pad;
-  const bool rq2 = o.rq_mode == 2, hb = rq2 && o.rq_bias != nullptr;
-  const double *mp = rq2 ? o.rq_mult_ch : (const double *)pad;
-  const int32_t *bp = hb ? o.rq_bias : (const int32_t *)pad;
 #pragma unroll
   for (int j = 0; j < 2; j++) {
     int64_t col = n0 + j * 16 + r16;
@@ -391,24 +386,14 @@ __device__ __forceinline__ void mmi_epi_load(MmiEpiIn &in, int64_t bz, int64_t M
     in.e[j] = ecol[bz * o.ecol_bstride + col];
     in.cs[j] = colsum[bz * cs_bstride + col];
     in.bs[j] = bsp[(fy && o.b_scale_len != 1) ? col : 0];
-    const int64_t ch = o.trans ? bz * N + col : col;  // output channel (requant mode 2)
-    in.mch[j] = mp[rq2 ? ch : 0];
-    in.bias[j] = bp[hb ? ch : 0];
   }
 }
 
-// 8-bit requantisation of one exact accumulator v (QLinearMatMul /
-// QLinearConv): mode 1 rounds v * mult through binary32 as the reference's
-// float path does, otherwise (v + bias) * mult_ch in double; then round half
+// 8-bit requantisation of one exact accumulator v (QLinearMatMul): v * mult
+// rounded through binary32 as the reference's float path does, then round half
 // to even, add the output zero point and saturate.
-__device__ __forceinline__ uint32_t mmi_requant(uint32_t v, double mch, double bias,
-                                                const MmiEpi &o) {
-  double x;
-  if (o.rq_mode == 1) {
-    x = (double)(float)((double)(int32_t)v * (double)o.rq_mult);
-  } else {
-    x = ((double)(int32_t)v + bias) * mch;
-  }
+__device__ __forceinline__ uint32_t mmi_requant(uint32_t v, const MmiEpi &o) {
+  const double x = (double)(float)((double)(int32_t)v * (double)o.rq_mult);
   double t = rint(x) + (double)o.yzp;
   t = t < (double)o.lo ? (double)o.lo : (t > (double)o.hi ? (double)o.hi : t);
   return (uint32_t)(uint8_t)(int32_t)t;
@@ -438,7 +423,7 @@ __device__ __forceinline__ void mmi_epilogue(const int4v (&acc)[TI][2], int (&rs
     for (int r = 0; r < 4; r++) {
       rs[r] = __shfl(rsum[i], q * 4 + r, 64);  // lane holding that row's sum
       row[r] = m0 + i * 16 + q * 4 + r;
-      const int32_t z = o.azp_is_const ? o.azp_const : (azp_len > 0 ? in.z[i][r] : 0);
+      const int32_t z = azp_len > 0 ? in.z[i][r] : 0;
       cm[r] = (a_signed ? 0 : 128) - z;
     }
 #pragma unroll
@@ -448,17 +433,16 @@ __device__ __forceinline__ void mmi_epilogue(const int4v (&acc)[TI][2], int (&rs
       const uint32_t e = (uint32_t)in.e[j];
       const uint32_t cs = (uint32_t)in.cs[j];
       const float sj = in.as * in.bs[j];
-      const double mch = in.mch[j], bias = (double)in.bias[j];
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         if (row[r] >= M) continue;
         const uint32_t c = (uint32_t)cm[r];
         const uint32_t v = (uint32_t)acc[i][j][r] + e * (uint32_t)rs[r] + c * cs +
                            (uint32_t)K * c * e;
-        const int64_t oi = o.trans ? (bz * N + col) * M + row[r] : (bz * M + row[r]) * N + col;
+        const int64_t oi = (bz * M + row[r]) * N + col;
         if (o.y) o.y[oi] = (int32_t)v;
         if (o.yf) o.yf[oi] = (float)(int32_t)v * sj;
-        if (o.yq) o.yq[oi] = (uint8_t)mmi_requant(v, mch, bias, o);
+        if (o.yq) o.yq[oi] = (uint8_t)mmi_requant(v, o);
       }
     }
   }
@@ -493,14 +477,13 @@ __device__ __forceinline__ void mmi_epilogue_lds(const int4v (&acc)[TI][2], int 
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       rs[r] = __shfl(rsum[i], q * 4 + r, 64);
-      const int32_t z = o.azp_is_const ? o.azp_const : (azp_len > 0 ? ein.z[i][r] : 0);
+      const int32_t z = azp_len > 0 ? ein.z[i][r] : 0;
       cm[r] = (a_signed ? 0 : 128) - z;
     }
 #pragma unroll
     for (int j = 0; j < 2; j++) {
       const uint32_t e = (uint32_t)ein.e[j], csum = (uint32_t)ein.cs[j];
       const float sj = ein.as * ein.bs[j];
-      const double mch = ein.mch[j], bias = (double)ein.bias[j];
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const uint32_t c = (uint32_t)cm[r];
@@ -508,7 +491,7 @@ __device__ __forceinline__ void mmi_epilogue_lds(const int4v (&acc)[TI][2], int 
                            (uint32_t)K * c * e;
         const int at = (i * 16 + q * 4 + r) * 33 + j * 16 + r16;
         if (o.yq) {
-          ti[at] = mmi_requant(v, mch, bias, o);
+          ti[at] = mmi_requant(v, o);
         } else {
           ti[at] = v;
           tf[at] = (float)(int32_t)v * sj;
@@ -848,7 +831,7 @@ int launch_matmul_integer(mmnb_ctx *ctx, const mmnb_pack *p, const void *d_a, in
     const int64_t tiles64 = (int64_t)grid.x * grid.y * grid.z;
     const int tm = ctx->mmi_tm ? ctx->mmi_tm : (tiles64 < 3 * (int64_t)ctx->cu_count ? 32 : 64);
     // the LDS epilogue: row-major outputs, the 8-bit one only on its own
-    const bool le = !o.trans && (!o.yq || (!o.y && !o.yf));
+    const bool le = !o.yq || (!o.y && !o.yf);
     auto kern = le ? k_mmi_lds<true, 64, 64, 2> : k_mmi_lds<false, 64, 64, 2>;
     dim3 g = grid;
     if (tm == 32) {

@@ -63,7 +63,7 @@ struct mmnb_ctx {
   // Device staging/scratch buffers, grown on demand and kept for reuse:
   //  0: activations in (fp32 / uint8), 1: outputs, 2: prepared activations
   //  (fp16 hi/lo), 3: small reductions, 4: raw weights while packing,
-  //  5: small uploads (zero points), 6: convolution im2col rows, 7: block
+  //  5: small uploads (zero points), 6: unused, 7: block
   //  sums / the convolution's input zero point, 8: QLinearConv per-channel
   //  parameters, 9: gathered activations of an extended MatMulNBits pack,
   //  10: the prefill GEMM's K-slice partial tiles.
@@ -204,7 +204,7 @@ enum KernelId {
   kKernDecGemvRes = 13,  // decode MatMulNBits + residual (o, down)
   kKernDecGemvGlu = 14,  // decode MatMulNBits, RMSNorm + SwiGLU (gate/up)
   kKernDecGemvLm = 15,   // decode MatMulNBits, RMSNorm + argmax (lm_head)
-  kKernIm2col = 16,      // convolution input rows for the MatMulInteger kernels
+  kKernConv = 16,        // convolutions
   kKernNbitsEx = 17,     // extended MatMulNBits: A gather, block sums, correction
   kKernNbitsAny = 18,    // MatMulNBits of a block size the fast kernels do not take
   kKernCount = 19
@@ -355,13 +355,9 @@ int launch_dql(mmnb_ctx *ctx, const float *d_x, int64_t n, uint8_t *d_y,
 //   y:  int32 acc.
 //   yf: fl32(fl32(acc) * fl32(a_scale * b_scale[j])), a_scale read from the
 //       device (the dynamic-quantisation chain's Cast -> Mul -> Mul).
-//   yq: 8-bit requantisation, clamp(rint(x) + yzp, lo, hi) stored as a byte:
-//       rq_mode 1: x = fl32(acc * rq_mult) (QLinearMatMul's binary32 steps);
-//       rq_mode 2: x = (acc + rq_bias[c]) * rq_mult_ch[c] in double
-//                  (QLinearConv, c = output channel).
-// Output element (batch bz, row, col) goes to (bz*M + row)*N + col, or with
-// trans to (bz*N + col)*M + row (channel-major: a convolution's output with
-// rows = positions, columns = channels of group bz, channel = bz*N + col).
+//   yq: 8-bit requantisation, clamp(rint(x) + yzp, lo, hi) stored as a byte,
+//       x = fl32(acc * rq_mult) (QLinearMatMul's binary32 steps).
+// Output element (batch bz, row, col) goes to (bz*M + row)*N + col.
 // ecol_bstride: the pack's zero-point offsets per batch (0 = shared).
 struct MmiEpi {
   int32_t *y = nullptr;
@@ -370,16 +366,9 @@ struct MmiEpi {
   const float *b_scale = nullptr;
   int64_t b_scale_len = 0;
   uint8_t *yq = nullptr;
-  int rq_mode = 0;
   float rq_mult = 0.0f;
-  const double *rq_mult_ch = nullptr;
-  const int32_t *rq_bias = nullptr;
   int32_t yzp = 0, lo = 0, hi = 255;
-  int trans = 0;
   int64_t ecol_bstride = 0;
-  // A's zero point as a constant (azp_len must be 1; the pointer is unused)
-  int azp_is_const = 0;
-  int32_t azp_const = 0;
 };
 
 // MatMulInteger on the device.  d_azp: device int32 of length azp_len (0, 1

@@ -1,17 +1,18 @@
 // QLinearMatMul, ConvInteger and QLinearConv on the MatMulInteger kernels.
 //
 // QLinearMatMul (onnx_qlinear_ops.dart:83-106) is MatMulInteger with an
-// 8-bit requantising epilogue.  A convolution (:157-308) runs as one
-// MatMulInteger per image: an im2col pass writes A[g][p][kc] (p an output
+// 8-bit requantising epilogue.  A convolution (:157-308) is one launch
+// (k_conv) of the product A[p][kc] * w^T per image and group (p an output
 // position, kc = (c*kh + ky)*kw + kx, out-of-image taps set to the input zero
 // point so that (x - x_zp) = 0 there, which is the reference's skipping of
-// them), the weight w[m][c/g][kh][kw] is a MatMulInteger pack of B^T per
-// group (batch = group), and the epilogue stores channel-major
-// y[m][oy][ox] directly (MmiEpi::trans), requantising per output channel for
-// QLinearConv.
+// them): the weight w[m][c/g][kh][kw] is a MatMulInteger pack of B^T per
+// group (batch = group), and the epilogue stores channel-major y[m][oy][ox],
+// requantising per output channel for QLinearConv.
 #include <cmath>
 #include <cstdint>
+#include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "mmnb_internal.h"
@@ -20,43 +21,297 @@ using namespace mmnb;
 
 namespace mmnb {
 
-// One image: x [C][H][W] bytes -> out [groups][oh*ow][cg*kh*kw].  Grid
-// (items / 256, groups); 32-bit index arithmetic (the host checks that
-// groups * oh*ow * cg*kh*kw fits); the source index is clamped so every load
-// is in bounds.
-__global__ __launch_bounds__(256) void k_im2col(const uint8_t *__restrict__ x, int H, int W,
-                                                int cg, int kh, int kw, int ow, int sh, int sw,
-                                                int ph, int pw, int dh, int dw, uint32_t zp,
-                                                int items, int per, uint8_t *__restrict__ out) {
-  // the group's output [P][kcn] is contiguous: thread item i owns bytes
-  // per*i .. per*i + per - 1 of it (per = 4 when kcn % 4 == 0, one 32-bit
-  // store; else 1), all of whose source bytes are loaded before any store
-  const unsigned item = blockIdx.x * blockDim.x + threadIdx.x;
-  if (item >= (unsigned)items) return;
-  const int g = blockIdx.y;
-  const int kcn = cg * kh * kw, khw = kh * kw;
-  const int e0 = (int)item * per;
-  const int p = e0 / kcn, kc0 = e0 - p * kcn;
-  const int oy = p / ow, ox = p - oy * ow;
-  uint32_t v[4];
-  bool in[4];
-#pragma unroll
-  for (int u = 0; u < 4; u++) {
-    const int kc = kc0 + (u < per ? u : 0);
-    const int c = kc / khw, r = kc - c * khw;
-    const int ky = r / kw, kx = r - ky * kw;
-    const int iy = oy * sh - ph + ky * dh, ix = ox * sw - pw + kx * dw;
-    in[u] = iy >= 0 && iy < H && ix >= 0 && ix < W;
-    v[u] = x[((size_t)(g * cg + c) * H + (in[u] ? iy : 0)) * W + (in[u] ? ix : 0)];
-  }
-  uint8_t *o = out + (size_t)g * items * per + e0;
-  if (per == 4) {
-    uint32_t word = 0;
-#pragma unroll
-    for (int u = 0; u < 4; u++) word |= (in[u] ? v[u] : zp) << (8 * u);
-    *(uint32_t *)o = word;
+// ---------------------------------------------------------------------------
+// One convolution launch: PT output positions x 16 CW output channels of one
+// (image, group) per workgroup, as a matrix product whose A rows are gathered
+// from the image on the way into LDS.
+//
+// The products of an image layer are small (56 x 56 x 64 channels of 3 x 3: 0.05
+// us of the matrix cores); what such a call spends is launches, round trips and
+// the byte gather.  So there is one launch: A never goes to memory, and the
+// per-channel requantisation parameters ride in the kernel's arguments (INL, up
+// to kConvInline channels), which saves the upload and the wait for it.
+//
+// K (kc = (c*kh + ky)*kw + kx, the weight's order) moves in chunks of 32 KB of A.
+// Per chunk a table of every kc's source offset and window position is built
+// (two divisions per entry instead of per byte), then thread t gathers the bytes
+// of position t % PT -- neighbouring lanes read neighbouring image bytes -- with
+// all of its loads in flight, out-of-image taps taking the input zero point and
+// kc >= K zero.  16-byte piece c of row r lies at c ^ (r & 15), so the 16 rows
+// of an operand read spread over the banks.  The weights go straight to
+// registers, four 64-k steps ahead.
+//
+// 16 waves, all of which gather: CW of them (a power of two) take 16 channels
+// each, the other factor KW = 16 / CW splits the chunk's 64-k steps and meets in LDS
+// at the end (integer adds: exact in any order).  A workgroup covers the group's
+// channels up to 256, so that few bytes are gathered twice, and fewer where the
+// positions alone leave the chip idle (conv_run).
+//
+// Against an upload, an im2col launch and the MatMulInteger kernel (us per call, u8 x
+// i8, back to back): 64 channels of 56 x 56, 3 x 3 to 64 24.4 -> 6.8; 3 of 112 x 112
+// to 16, stride 2 21.0 -> 5.2; 256 of 14 x 14, 3 x 3 to 256 26.3 -> 13.3; 256 of 7 x
+// 7, 5 x 5 to 256 37.8 -> 27.4; 256 of 112 x 112, 5 x 5 to 256 233 -> 169.  (4 waves
+// and 64 channels per workgroup: 9.9 us on the first, 417 on the last.)
+// ---------------------------------------------------------------------------
+typedef int conv_i4 __attribute__((ext_vector_type(4)));
+typedef uint32_t conv_u4 __attribute__((ext_vector_type(4)));
+
+constexpr int kConvInline = 256;  // channels whose parameters fit the arguments
+struct ConvChan {
+  double mult[kConvInline];
+  int32_t bias[kConvInline];
+};
+struct ConvNoChan {};
+
+struct ConvArgs {
+  const uint8_t *x;       // [images][groups * cg][H][W]
+  const int8_t *bt;       // [groups][N][kpad]
+  const int32_t *colsum;  // [groups][N]
+  const int32_t *ecol;    // [N], or [groups][N] with ecol_bstride = N
+  int H, W, cg, kh, kw, ow, sh, sw, ph, pw, dh, dw;
+  int P, K, kpad, N, groups, ecol_bstride;
+  int cw;                 // channel waves of a workgroup: a power of two <= 16
+  uint32_t flip;          // 0x80808080: unsigned input
+  int32_t azp;            // input zero point
+  int32_t *y;             // int32 output, or
+  uint8_t *yq;            // requantised bytes
+  const double *mult;     // [groups * N] (without INL)
+  const int32_t *bias;    // [groups * N]
+  int32_t yzp, lo, hi;
+  int vec;                // P % 4 == 0 and an aligned output
+};
+
+constexpr int kConvThreads = 1024;
+constexpr int kConvLds = 32768;  // bytes of A per chunk; the sums' tile later
+
+// A table entry: source offset, and the window position (ky * dh, kx * dw) in 16
+// bits each (saturated: past every image that is not WIDE) or, WIDE, 32.
+struct ConvTap {
+  uint32_t off, pos;
+};
+struct ConvTapWide {
+  uint32_t off, dy, dx;
+};
+
+template <int PT, typename CHAN, bool WIDE = false>
+__global__ __launch_bounds__(kConvThreads) void k_conv(ConvArgs c, CHAN chan) {
+  constexpr int KC = kConvLds / PT;         // k per chunk
+  constexpr int TP = PT / 16;               // 16-position tiles
+  constexpr int WQ = kConvThreads / PT;     // words per position and gather pass
+  __shared__ conv_u4 sA[kConvLds / 16];
+  __shared__ std::conditional_t<WIDE, ConvTapWide, ConvTap> tab[KC];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int cw = wave & (c.cw - 1), kw = wave / c.cw, nkw = 16 / c.cw;
+  const int r16 = lane & 15, q = lane >> 4;
+  const int g = blockIdx.z % c.groups;
+  const int p0 = blockIdx.x * PT;
+
+  // this lane's output channel and its constants
+  const int n = (blockIdx.y * c.cw + cw) * 16 + r16;
+  const int col = n < c.N ? n : c.N - 1;
+  const uint32_t ce = (uint32_t)c.ecol[g * c.ecol_bstride + col];
+  const uint32_t cs = (uint32_t)c.colsum[(int64_t)g * c.N + col];
+  const int ch = g * c.N + col;
+  double cm;
+  int32_t cb;
+  if constexpr (std::is_same<CHAN, ConvChan>::value) {
+    cm = chan.mult[ch];
+    cb = chan.bias[ch];
   } else {
-    o[0] = (uint8_t)(in[0] ? v[0] : zp);
+    // (the int32 output has no parameters: both point at a zero page)
+    cm = c.mult[c.y ? 0 : ch];
+    cb = c.bias[c.y ? 0 : ch];
+  }
+  const int8_t *bp = c.bt + ((int64_t)g * c.N + col) * c.kpad + q * 16;
+
+  // this thread's position of the gather
+  const int row = tid % PT, wq = tid / PT;
+  const int pc = p0 + row < c.P ? p0 + row : c.P - 1;
+  const int oy = pc / c.ow, ox = pc - oy * c.ow;
+  const int iy0 = oy * c.sh - c.ph, ix0 = ox * c.sw - c.pw;
+  const unsigned base = (unsigned)iy0 * (unsigned)c.W + (unsigned)ix0;
+  const uint8_t *xg = c.x + (int64_t)blockIdx.z * c.cg * c.H * c.W;
+  const int khw = c.kh * c.kw;
+  const uint32_t zb = (uint32_t)c.azp & 255u, fb = c.flip & 255u;
+
+  conv_i4 acc[TP];
+  int rsum[TP];
+#pragma unroll
+  for (int t = 0; t < TP; t++) {
+    rsum[t] = 0;
+    acc[t] = (conv_i4){0, 0, 0, 0};
+  }
+
+  for (int k0 = 0; k0 < c.kpad; k0 += KC) {
+    const int kn = c.kpad - k0 < KC ? c.kpad - k0 : KC;  // a multiple of 64
+    const int nst = kn >> 6, words = kn >> 2;
+    // weights of this wave's steps s, s + nkw, ... (clamped to the chunk)
+    conv_i4 bw[4];
+    auto load_b = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+        bw[u] = *(const conv_i4 *)(bp + k0 + (s + u * nkw < nst ? s + u * nkw : nst - 1) * 64);
+    };
+    load_b(kw);
+    for (int i = tid; i < kn; i += kConvThreads) {
+      const int kk = k0 + i < c.K ? k0 + i : c.K - 1;
+      const int ci = kk / khw, r = kk - ci * khw;
+      const int ky = r / c.kw, kx = r - ky * c.kw;
+      const unsigned dy = (unsigned)ky * (unsigned)c.dh, dx = (unsigned)kx * (unsigned)c.dw;
+      const unsigned off = ((unsigned)ci * (unsigned)c.H + dy) * (unsigned)c.W + dx;
+      if constexpr (WIDE)
+        tab[i] = {off, dy, dx};
+      else
+        tab[i] = {off, (dy < 65535u ? dy : 65535u) << 16 | (dx < 65535u ? dx : 65535u)};
+    }
+    __syncthreads();  // the table, and every wave past the last chunk's products
+    // gather: words wq, wq + WQ, ... of the position's row (clamped: repeated)
+    auto gather = [&](auto count, int u0) __attribute__((always_inline)) {
+      constexpr int NP = decltype(count)::value;
+      uint32_t w[NP];
+#pragma unroll
+      for (int u = 0; u < NP; u++) {
+        const int word = wq + WQ * (u0 + u) < words ? wq + WQ * (u0 + u) : words - 1;
+        uint32_t v[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const auto t = tab[4 * word + e];
+          unsigned dy, dx;
+          if constexpr (WIDE) {
+            dy = t.dy;
+            dx = t.dx;
+          } else {
+            dy = t.pos >> 16;
+            dx = t.pos & 65535u;
+          }
+          const bool in = (unsigned)iy0 + dy < (unsigned)c.H && (unsigned)ix0 + dx < (unsigned)c.W;
+          const uint32_t b = xg[in ? base + t.off : 0u];
+          v[e] = k0 + 4 * word + e < c.K ? (in ? b : zb) : fb;
+        }
+        w[u] = v[0] | v[1] << 8 | v[2] << 16 | v[3] << 24;
+      }
+#pragma unroll
+      for (int u = 0; u < NP; u++) {
+        const int word = wq + WQ * (u0 + u) < words ? wq + WQ * (u0 + u) : words - 1;
+        ((uint32_t *)sA)[row * (KC / 4) + (((word >> 2) ^ (row & 15)) << 2) + (word & 3)] = w[u];
+      }
+    };
+    const int passes = (words + WQ - 1) / WQ;  // 1 .. 8
+    if (passes == 1)
+      gather(std::integral_constant<int, 1>(), 0);
+    else if (passes <= 3)
+      gather(std::integral_constant<int, 3>(), 0);
+    else if (passes <= 5)
+      gather(std::integral_constant<int, 5>(), 0);
+    else
+      gather(std::integral_constant<int, 8>(), 0);
+    __syncthreads();
+    for (int s = kw; s < nst; s += 4 * nkw) {
+      conv_i4 b[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) b[u] = bw[u];
+      if (s + 4 * nkw < nst) load_b(s + 4 * nkw);
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        if (s + u * nkw < nst) {
+#pragma unroll
+          for (int t = 0; t < TP; t++) {
+            const int ra = t * 16 + r16;
+            const conv_u4 x =
+                sA[ra * (KC / 16) + (((s + u * nkw) * 4 + q) ^ (ra & 15))] ^ c.flip;
+            const conv_i4 a = __builtin_bit_cast(conv_i4, x);
+#pragma unroll
+            for (int d = 0; d < 4; d++)
+              rsum[t] = __builtin_amdgcn_sdot4(a[d], 0x01010101, rsum[t], false);
+            acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b[u], acc[t], 0, 0, 0);
+          }
+        }
+      }
+    }
+  }
+
+  // acc += e * (row sum), per k wave; then the k waves' sums through LDS
+#pragma unroll
+  for (int t = 0; t < TP; t++) {
+    rsum[t] += __shfl_xor(rsum[t], 16, 64);
+    rsum[t] += __shfl_xor(rsum[t], 32, 64);
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      acc[t][r] = (int)((uint32_t)acc[t][r] + ce * (uint32_t)__shfl(rsum[t], q * 4 + r, 64));
+  }
+  if (nkw > 1) {
+    // [CW <= 8 channel waves][PT / 16][4][64] dwords fit the chunk's LDS
+    uint32_t *red = (uint32_t *)sA + cw * (TP * 256);
+    __syncthreads();
+    if (kw == 0) {
+#pragma unroll
+      for (int t = 0; t < TP; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) red[(t * 4 + r) * 64 + lane] = (uint32_t)acc[t][r];
+    }
+    __syncthreads();
+    if (kw > 0) {
+#pragma unroll
+      for (int t = 0; t < TP; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) atomicAdd(&red[(t * 4 + r) * 64 + lane], (uint32_t)acc[t][r]);
+    }
+    __syncthreads();
+    if (kw > 0) return;
+#pragma unroll
+    for (int t = 0; t < TP; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) acc[t][r] = (int)red[(t * 4 + r) * 64 + lane];
+  }
+
+  // exact zero-point corrections, in wrapping 32 bits, and the stores
+  if (n >= c.N) return;
+  const uint32_t azc = (uint32_t)((c.flip ? 128 : 0) - c.azp);
+  const uint32_t fix = azc * cs + (uint32_t)c.K * azc * ce;
+#pragma unroll
+  for (int t = 0; t < TP; t++) {
+    const int p = p0 + t * 16 + q * 4;
+    if (p >= c.P) continue;
+    uint32_t v[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) v[r] = (uint32_t)acc[t][r] + fix;
+    const int64_t at = ((int64_t)blockIdx.z * c.N + col) * c.P + p;
+    if (c.y) {
+      if (c.vec) {
+        *(conv_u4 *)(c.y + at) = (conv_u4){v[0], v[1], v[2], v[3]};
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          if (p + r < c.P) c.y[at + r] = (int32_t)v[r];
+      }
+    } else {
+      uint32_t o[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        // double, as the reference: (acc + bias) * mult, half to even, saturated
+        const double f = rint(((double)(int32_t)v[r] + (double)cb) * cm) + (double)c.yzp;
+        o[r] = (uint32_t)(uint8_t)(int32_t)fmin(fmax(f, (double)c.lo), (double)c.hi);
+      }
+      if (c.vec) {
+        *(uint32_t *)(c.yq + at) = o[0] | o[1] << 8 | o[2] << 16 | o[3] << 24;
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          if (p + r < c.P) c.yq[at + r] = (uint8_t)o[r];
+      }
+    }
+  }
+}
+
+// More channels than the arguments hold: 256 channels' parameters per launch,
+// written where k_conv reads them.
+__global__ __launch_bounds__(256) void k_conv_params(ConvChan chan, int n, double *mult,
+                                                     int32_t *bias) {
+  const int i = threadIdx.x;
+  if (i < n) {
+    mult[i] = chan.mult[i];
+    bias[i] = chan.bias[i];
   }
 }
 
@@ -107,42 +362,87 @@ int check_zp(int64_t v, int is_signed, const char *what) {
   return MMNB_OK;
 }
 
-// Device side of a convolution: per image, im2col then the MatMulInteger
-// kernel with a channel-major epilogue.  `o` carries the output pointers of
-// image 0; each image's output follows the previous one's m*oh*ow values.
-// Scratch: slot 6 = im2col.
+// Where a convolution's results go: int32 y, or bytes yq requantised with the
+// channels' parameters (in the arguments up to kConvInline channels, else in
+// scratch slot 8).
+struct ConvOut {
+  int32_t *y = nullptr;
+  uint8_t *yq = nullptr;
+  int32_t yzp = 0, lo = 0, hi = 255;
+  bool inl = false;
+  ConvChan chan;
+  const double *d_mult = nullptr;
+  const int32_t *d_bias = nullptr;
+};
+
+template <int PT, bool WIDE = false>
+int conv_launch(mmnb_ctx *ctx, const ConvArgs &c, const ConvOut &o, int64_t z) {
+  const dim3 grid((unsigned)((c.P + PT - 1) / PT), (unsigned)((c.N + 16 * c.cw - 1) / (16 * c.cw)),
+                  (unsigned)z);
+  const dim3 block(kConvThreads);
+  if (o.inl)
+    return launch(ctx, kKernConv, k_conv<PT, ConvChan, WIDE>, grid, block, 0, c, o.chan);
+  return launch(ctx, kKernConv, k_conv<PT, ConvNoChan, WIDE>, grid, block, 0, c, ConvNoChan{});
+}
+
+// Device side of a convolution: all images and groups in one launch (grid.z,
+// at most 65535 of them at a time).
 int conv_run(mmnb_ctx *ctx, const mmnb_pack *p, const uint8_t *d_x, int x_signed,
-             const ConvShape &s, int64_t x_zp, MmiEpi o) {
-  const int64_t P = s.oh * s.ow, kcn = p->k, g = p->conv_group, m = p->conv_m;
+             const ConvShape &s, int64_t x_zp, const ConvOut &o) {
+  const int64_t P = s.oh * s.ow, kcn = p->k, g = p->conv_group, n = p->n;
   if (s.n == 0 || P == 0) return MMNB_OK;
   if (kcn > 65535 * 256 || g > 65535 || g * P * kcn > INT32_MAX ||
       s.c * s.h * s.w > INT32_MAX)
     return fail(MMNB_ERR_UNSUPPORTED, "conv: image too large for one launch");
-  void *d_col = nullptr;
-  int rc;
-  if ((rc = scratch_get(ctx, 6, (size_t)(g * P * kcn) + 256, &d_col))) return rc;
-  o.azp_is_const = 1;
-  o.azp_const = (int32_t)x_zp;
-  const uint32_t zbyte = (uint32_t)(x_zp & 0xFF);
-  // 4 bytes per thread when the rows are whole dwords (the scratch buffer
-  // is 256-byte aligned, so then every dword is aligned)
-  const int per = kcn % 4 == 0 ? 4 : 1;
-  const int items = (int)(P * kcn / per);
-  const dim3 grid((unsigned)((items + 255) / 256), (unsigned)g);
-  for (int64_t b = 0; b < s.n; b++) {
-    const uint8_t *xb = d_x + b * s.c * s.h * s.w;
-    if ((rc = launch(ctx, kKernIm2col, k_im2col, grid, dim3(256), 0, xb, (int)s.h, (int)s.w,
-                     (int)p->conv_cg, (int)p->conv_kh, (int)p->conv_kw, (int)s.ow, s.sh, s.sw,
-                     s.ph, s.pw, s.dh, s.dw, zbyte, items, per, (uint8_t *)d_col)))
-      return rc;
-    MmiEpi ob = o;
-    ob.trans = 1;
-    const int64_t off = b * m * P;
-    if (o.y) ob.y = o.y + off;
-    if (o.yq) ob.yq = o.yq + off;
-    if ((rc = launch_matmul_integer(ctx, p, d_col, x_signed, g, P, (const int32_t *)ctx->d_pad,
-                                    1, ob)))
-      return rc;
+  const int64_t esz = o.y ? 4 : 1;
+  ConvArgs c{};
+  c.bt = p->d_bt;
+  c.colsum = p->d_colsum;
+  c.ecol = p->d_ecol;
+  c.H = (int)s.h; c.W = (int)s.w; c.cg = (int)p->conv_cg;
+  c.kh = (int)p->conv_kh; c.kw = (int)p->conv_kw; c.ow = (int)s.ow;
+  c.sh = s.sh; c.sw = s.sw; c.ph = s.ph; c.pw = s.pw; c.dh = s.dh; c.dw = s.dw;
+  c.P = (int)P; c.K = (int)kcn; c.kpad = (int)p->kpad; c.N = (int)n; c.groups = (int)g;
+  c.ecol_bstride = (int)p->ecol_bstride;
+  c.flip = x_signed ? 0u : 0x80808080u;
+  c.azp = (int32_t)x_zp;
+  c.mult = o.d_mult ? o.d_mult : (const double *)ctx->d_pad;
+  c.bias = o.d_bias ? o.d_bias : (const int32_t *)ctx->d_pad;
+  c.yzp = o.yzp; c.lo = o.lo; c.hi = o.hi;
+  // a window position saturated at 65535 lies past every image up to that size
+  // (with its padding)
+  const bool wide = s.h + s.ph > 65535 || s.w + s.pw > 65535;
+  const int64_t zmax = 65535 / g * g;  // whole images per launch
+  for (int64_t z0 = 0; z0 < s.n * g; z0 += zmax) {
+    const int64_t z = s.n * g - z0 < zmax ? s.n * g - z0 : zmax;
+    c.x = d_x + z0 * p->conv_cg * s.h * s.w;
+    c.y = o.y ? o.y + z0 * n * P : nullptr;
+    c.yq = o.y ? nullptr : o.yq + z0 * n * P;
+    const uintptr_t out = o.y ? (uintptr_t)c.y : (uintptr_t)c.yq;
+    c.vec = P % 4 == 0 && out % (4 * esz) == 0;
+    // the most positions per read of the weights that leave a workgroup on three
+    // quarters of the CUs; then, while half of them are idle, fewer channels per
+    // workgroup: the gather is repeated, but a workgroup reads less of the weights
+    // (256 channels of 14 x 14, 3 x 3 to 256: 13.3 us, with all 256 in one workgroup
+    // 25.8)
+    const int64_t cus = ctx->cu_count;
+    c.cw = 1;
+    while (c.cw < 16 && 16 * c.cw < n) c.cw *= 2;
+    auto groups = [&](int64_t pt) {
+      return (P + pt - 1) / pt * ((n + 16 * c.cw - 1) / (16 * c.cw)) * z;
+    };
+    const int64_t enough = 3 * cus / 4;
+    while (c.cw > 1 && groups(16) < cus / 2) c.cw /= 2;
+    int rc;
+    if (wide)
+      rc = conv_launch<16, true>(ctx, c, o, z);
+    else if (groups(64) >= enough)
+      rc = conv_launch<64>(ctx, c, o, z);
+    else if (groups(32) >= enough)
+      rc = conv_launch<32>(ctx, c, o, z);
+    else
+      rc = conv_launch<16>(ctx, c, o, z);
+    if (rc) return rc;
   }
   return MMNB_OK;
 }
@@ -197,7 +497,6 @@ int mmnb_qlinear_matmul_dev(mmnb_ctx *ctx, const mmnb_pack *pack, const void *d_
   if ((rc = set_device(ctx))) return rc;
   MmiEpi o;
   o.yq = (uint8_t *)d_y;
-  o.rq_mode = 1;
   o.rq_mult = mult;
   o.yzp = (int32_t)y_zero_point;
   o.lo = y_is_signed ? -128 : 0;
@@ -241,7 +540,6 @@ int mmnb_qlinear_matmul(mmnb_ctx *ctx, const mmnb_pack *pack, const void *a, int
                             ctx->stream));
   MmiEpi o;
   o.yq = (uint8_t *)d_y;
-  o.rq_mode = 1;
   o.rq_mult = mult;
   o.yzp = (int32_t)y_zero_point;
   o.lo = y_is_signed ? -128 : 0;
@@ -355,7 +653,7 @@ int mmnb_conv_integer_dev(mmnb_ctx *ctx, const mmnb_pack *w, const void *d_x, in
   if (!d_x || !d_y) return fail(MMNB_ERR_ARG, "ConvInteger: null buffer");
   CtxLock lk(ctx);
   if ((rc = set_device(ctx))) return rc;
-  MmiEpi o;
+  ConvOut o;
   o.y = d_y;
   return conv_run(ctx, w, (const uint8_t *)d_x, x_is_signed ? 1 : 0, s, x_zero_point, o);
 }
@@ -378,7 +676,7 @@ int mmnb_conv_integer(mmnb_ctx *ctx, const mmnb_pack *w, const void *x, int x_is
   if ((rc = scratch_get(ctx, 0, xb + 256, &d_x))) return rc;
   if ((rc = scratch_get(ctx, 1, yn * 4, &d_y))) return rc;
   if (xb) MMNB_HIP(hipMemcpyAsync(d_x, x, xb, hipMemcpyHostToDevice, ctx->stream));
-  MmiEpi o;
+  ConvOut o;
   o.y = (int32_t *)d_y;
   if ((rc = conv_run(ctx, w, (const uint8_t *)d_x, x_is_signed ? 1 : 0, s, x_zero_point, o)))
     return rc;
@@ -389,31 +687,44 @@ int mmnb_conv_integer(mmnb_ctx *ctx, const mmnb_pack *w, const void *x, int x_is
 
 // Per-channel requantisation parameters of QLinearConv, in double as the
 // reference computes them (onnx_qlinear_ops.dart:295-305): mult[c] =
-// x_scale * w_scale[c] / y_scale, bias[c] (int32, optional).  Written to
-// scratch slot 8 as [m doubles][m int32].
+// x_scale * w_scale[c] / y_scale, bias[c] (int32, optional).  Up to kConvInline
+// channels stay in o->chan; more go to scratch slot 8, [m doubles][m int32],
+// by way of kernel arguments too: no copy from host memory to wait for.
 static int qconv_params(mmnb_ctx *ctx, int64_t m, float x_scale, const float *w_scale,
-                        int64_t w_scale_len, float y_scale, const int32_t *bias,
-                        const double **d_mult, const int32_t **d_bias) {
+                        int64_t w_scale_len, float y_scale, const int32_t *bias, ConvOut *o) {
   if (!w_scale || (w_scale_len != 1 && w_scale_len != m))
     return fail(MMNB_ERR_ARG, "QLinearConv: w_scale must have 1 or M values");
   if (!std::isfinite(x_scale) || !std::isfinite(y_scale) || y_scale == 0.0f)
     return fail(MMNB_ERR_ARG, "QLinearConv: scales must be finite and y_scale non-zero");
-  std::vector<char> buf((size_t)m * 12);
-  double *mult = (double *)buf.data();
-  int32_t *bb = (int32_t *)(buf.data() + m * 8);
-  for (int64_t c = 0; c < m; c++) {
-    const double ws = (double)w_scale[w_scale_len == 1 ? 0 : c];
-    mult[c] = (double)x_scale * ws / (double)y_scale;
-    if (!std::isfinite(mult[c])) return fail(MMNB_ERR_ARG, "QLinearConv: non-finite scale");
-    bb[c] = bias ? bias[c] : 0;
+  auto mult = [&](int64_t c) {
+    return (double)x_scale * (double)w_scale[w_scale_len == 1 ? 0 : c] / (double)y_scale;
+  };
+  for (int64_t c = 0; c < m; c++)
+    if (!std::isfinite(mult(c))) return fail(MMNB_ERR_ARG, "QLinearConv: non-finite scale");
+  o->inl = m <= kConvInline;
+  double *d_mult = nullptr;
+  int32_t *d_bias = nullptr;
+  if (!o->inl) {
+    void *d = nullptr;
+    int rc = scratch_get(ctx, 8, (size_t)m * 12, &d);
+    if (rc) return rc;
+    d_mult = (double *)d;
+    d_bias = (int32_t *)((char *)d + m * 8);
+    o->d_mult = d_mult;
+    o->d_bias = d_bias;
   }
-  void *d = nullptr;
-  int rc = scratch_get(ctx, 8, buf.size(), &d);
-  if (rc) return rc;
-  MMNB_HIP(hipMemcpyAsync(d, buf.data(), buf.size(), hipMemcpyHostToDevice, ctx->stream));
-  MMNB_HIP(hipStreamSynchronize(ctx->stream));  // `buf` is about to go away
-  *d_mult = (const double *)d;
-  *d_bias = bias ? (const int32_t *)((char *)d + m * 8) : nullptr;
+  for (int64_t c0 = 0; c0 < m; c0 += kConvInline) {
+    const int cnt = (int)(m - c0 < kConvInline ? m - c0 : kConvInline);
+    std::memset(&o->chan, 0, sizeof(o->chan));
+    for (int i = 0; i < cnt; i++) {
+      o->chan.mult[i] = mult(c0 + i);
+      o->chan.bias[i] = bias ? bias[c0 + i] : 0;
+    }
+    if (o->inl) break;
+    int rc = launch(ctx, kKernConv, k_conv_params, dim3(1), dim3(kConvInline), 0, o->chan, cnt,
+                    d_mult + c0, d_bias + c0);
+    if (rc) return rc;
+  }
   return MMNB_OK;
 }
 
@@ -433,12 +744,10 @@ int mmnb_qlinear_conv_dev(mmnb_ctx *ctx, const mmnb_pack *w, const void *d_x, in
   if (!d_x || !d_y) return fail(MMNB_ERR_ARG, "QLinearConv: null buffer");
   CtxLock lk(ctx);
   if ((rc = set_device(ctx))) return rc;
-  MmiEpi o;
-  if ((rc = qconv_params(ctx, w->conv_m, x_scale, w_scale, w_scale_len, y_scale, bias,
-                         &o.rq_mult_ch, &o.rq_bias)))
+  ConvOut o;
+  if ((rc = qconv_params(ctx, w->conv_m, x_scale, w_scale, w_scale_len, y_scale, bias, &o)))
     return rc;
   o.yq = (uint8_t *)d_y;
-  o.rq_mode = 2;
   o.yzp = (int32_t)y_zero_point;
   o.lo = y_is_signed ? -128 : 0;
   o.hi = y_is_signed ? 127 : 255;
@@ -465,13 +774,11 @@ int mmnb_qlinear_conv(mmnb_ctx *ctx, const mmnb_pack *w, const void *x, int x_is
   void *d_x = nullptr, *d_y = nullptr;
   if ((rc = scratch_get(ctx, 0, xb + 256, &d_x))) return rc;
   if ((rc = scratch_get(ctx, 1, yn + 256, &d_y))) return rc;
-  MmiEpi o;
-  if ((rc = qconv_params(ctx, w->conv_m, x_scale, w_scale, w_scale_len, y_scale, bias,
-                         &o.rq_mult_ch, &o.rq_bias)))
+  ConvOut o;
+  if ((rc = qconv_params(ctx, w->conv_m, x_scale, w_scale, w_scale_len, y_scale, bias, &o)))
     return rc;
   if (xb) MMNB_HIP(hipMemcpyAsync(d_x, x, xb, hipMemcpyHostToDevice, ctx->stream));
   o.yq = (uint8_t *)d_y;
-  o.rq_mode = 2;
   o.yzp = (int32_t)y_zero_point;
   o.lo = y_is_signed ? -128 : 0;
   o.hi = y_is_signed ? 127 : 255;

@@ -1,0 +1,51 @@
+"""QLinearConv and ConvInteger at the edges of the convolution kernel's tiles, bit for bit
+against the oracle: position tiles (16 and 32), channel tiles (64 to 256), chunks of K,
+images of a launch, unaligned outputs, and more channels than travel in the arguments."""
+import numpy as np
+import pytest
+
+from oracle import qlinear as Q
+from onnx_runtime_dart_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,c,hw,m,ks,stride,group", [
+    (1, 1, 1, 1, 1, 1, 1),          # one product
+    (1, 3, 7, 16, 5, 2, 1),         # P = 16, ragged K
+    (2, 5, 17, 65, 3, 1, 1),        # P = 289: bytes stored one by one; a channel past a tile
+    (1, 256, 7, 40, 3, 1, 1),       # K = 2304: several chunks
+    (3, 57, 40, 130, 3, 1, 1),      # 32 positions, K = 513 (a chunk and one step), 4 channel tiles
+    (2, 16, 100, 72, 1, 1, 1),      # 32 positions, 2 channel tiles
+    (1, 8, 9, 300, 3, 1, 1),        # parameters by way of scratch
+    (2, 24, 11, 48, 3, 2, 24),      # depthwise
+])
+def test_conv_tiles(n, c, hw, m, ks, stride, group):
+    ctx = _lib.default_context()
+    rng = np.random.default_rng(n + 3 * c + 5 * hw + 7 * m)
+    x = rng.integers(0, 256, (n, c, hw, hw)).astype(np.uint8)
+    w = rng.integers(-128, 128, (m, c // group, ks, ks)).astype(np.int8)
+    xz, wz = np.uint8(rng.integers(0, 256)), rng.integers(-128, 128, m).astype(np.int8)
+    st, pads, dl = [stride] * 2, [ks // 2] * 4, [1, 1]
+    geo = dict(strides=st, pads=pads, dilations=dl, group=group)
+    y = ops.op_conv_integer(x, w, xz, wz, ctx=ctx, **geo)
+    np.testing.assert_array_equal(y, Q.conv_integer(x, w, xz, wz, st, pads, dl, group))
+    ws = rng.uniform(0.001, 0.01, m).astype(np.float32)
+    bias = rng.integers(-3000, 3000, m).astype(np.int32)
+    ys, yz = np.float32(0.05 * np.sqrt(c // group * ks * ks)), np.uint8(120)
+    y = ops.op_qlinear_conv(x, np.float32(0.02), xz, w, ws, wz, ys, yz, bias, lo=0, hi=255,
+                            ctx=ctx, **geo)
+    want = Q.qlinear_conv(x, np.float32(0.02), xz, w, ws, wz, ys, yz, bias, st, pads, dl, group,
+                          0, 255)
+    np.testing.assert_array_equal(y, want)
+
+
+def test_conv_of_an_image_beyond_16_bit_positions():
+    rng = np.random.default_rng(3)
+    x = rng.integers(0, 256, (1, 1, 70001, 2)).astype(np.uint8)
+    w = rng.integers(-128, 128, (4, 1, 3, 1)).astype(np.int8)
+    y = ops.op_conv_integer(x, w, np.uint8(9), np.int8(3), ctx=_lib.default_context(),
+                            strides=[1, 1], pads=[66000, 0, 66000, 0], dilations=[66000, 1])
+    want = Q.conv_integer(x, w, np.uint8(9), np.int8(3), [1, 1], [66000, 0, 66000, 0],
+                          [66000, 1])
+    np.testing.assert_array_equal(y, want)
