@@ -201,17 +201,29 @@ int nbits_prepare(const mmnb_nbits_desc *d, NbitsHost *out) {
       }
     out->bytes8 = zf.empty();
     out->z8.assign(zi.begin(), zi.end());
-    out->corr.assign((size_t)nnb, 0.0);
-    for (int64_t c = 0; c < n; c++)
-      for (int64_t b = 0; b < nb; b++) {
-        const double z = !zf.empty() ? (double)zf[(size_t)(c * nb + b)]
-                                     : !zi.empty() ? (double)zi[(size_t)(c * nb + b)] : 128.0;
-        out->corr[(size_t)(b * n + c)] = (136.0 - z) * (double)s[(size_t)(c * nb + b)];
+    out->planes = zi.empty() && zf.empty();
+    if (out->planes) {
+      // q8 - 128 = 16 (hi - 8) + lo
+      out->vz.assign((size_t)((n * nbv + 1) / 2), 0);
+      for (int64_t c = 0; c < n; c++)
+        for (int64_t b = 0; b < nbv / 2; b++) {
+          const int64_t i = c * nbv + b;
+          out->vz[(size_t)(i >> 1)] |= (uint8_t)(8 << ((i & 1) * 4));
+        }
+    } else {
+      out->corr.assign((size_t)nnb, 0.0);
+      for (int64_t c = 0; c < n; c++)
+        for (int64_t b = 0; b < nb; b++)
+        {
+          const int64_t i = c * nb + b;
+          const double z = !zf.empty() ? (double)zf[(size_t)i] : (double)zi[(size_t)i];
+          out->corr[(size_t)(b * n + c)] = (136.0 - z) * (double)s[(size_t)i];
+        }
+      out->asrc.resize((size_t)kv);
+      for (int64_t j = 0; j < kv; j++) {
+        const int64_t kk = j < kp ? j : j - kp;
+        out->asrc[(size_t)j] = kk < k ? (int32_t)kk : -1;
       }
-    out->asrc.resize((size_t)kv);
-    for (int64_t j = 0; j < kv; j++) {
-      const int64_t kk = j < kp ? j : j - kp;
-      out->asrc[(size_t)j] = kk < k ? (int32_t)kk : -1;
     }
   } else {
     if (perm.empty()) {

@@ -50,10 +50,12 @@ struct NbitsHost {
   std::vector<double> corr;       // [n_blocks][n], or empty
   std::vector<int32_t> asrc;      // [kv] column of A per virtual row (-1: 0)
   std::vector<float> bias;        // [n], or empty
-  // bits = 8 with integer zero points: the virtual weight's planes rebuild the
-  // bytes, whose zero points are z8 ([n][n_blocks]; empty: 128)
+  // bits = 8 with integer zero points z8 ([n][n_blocks]; empty: 128)
   bool bytes8 = false;
   std::vector<uint8_t> z8;
+  // ... all of them 128: the planes have zero points 8 and 0 (vz), and the kernels
+  // take them without gather and correction
+  bool planes = false;
 };
 
 // Validates d against its own lengths and builds the virtual weight.

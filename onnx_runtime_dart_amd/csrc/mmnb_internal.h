@@ -157,11 +157,20 @@ struct mmnb_pack {
   float *d_corr = nullptr;    // [corr_nb, n]
   int64_t corr_nb = 0;
   float *d_bias = nullptr;    // [n]
-  // bits = 8 with integer zero points (k_gemv8): the two halves of a column
-  // hold the bytes' high and low nibbles; d_z8 the zero points [n][corr_nb]
-  // (null: 128)
+  // bits = 8 with integer zero points: the two halves of a column hold the bytes'
+  // high and low nibbles (k / 2 rows each), nb8 blocks of each not padding; d_z8 the
+  // zero points [n][nb8] (null: 128)
   bool bytes8 = false;
+  int64_t nb8 = 0;
   uint8_t *d_z8 = nullptr;
+  // Whether the kernels take the operator's own A and bias (no gather, no correction
+  // pass).  Rows past k_wrap() are then A's from column 0 again, and A has k_read()
+  // columns.
+  bool direct() const { return !d_asrc && !d_corr; }
+  bool wraps() const { return bytes8 && direct(); }
+  int64_t k_wrap() const { return wraps() ? k / 2 : INT32_MAX; }
+  int64_t k_read() const { return wraps() ? k_in : k; }
+  const float *direct_bias() const { return direct() ? d_bias : nullptr; }
   // --- MatMulInteger
   int64_t batch = 0;
   int64_t kpad = 0;          // k padded to a multiple of 64

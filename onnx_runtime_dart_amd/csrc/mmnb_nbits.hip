@@ -1030,8 +1030,10 @@ int launch_gemv_bias(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_
 constexpr int kPrepWaves = 8;     // waves per row (one row per workgroup)
 constexpr int kPrepChunk = 4096;  // k per pass of a row's waves
 
+// WRAP: rows of the weight from kwrap on (a multiple of 64) read A from its start again.
+template <bool WRAP>
 __global__ __launch_bounds__(64 * kPrepWaves) void k_prep_a(
-    const float *__restrict__ A, int64_t lda, int64_t M, int64_t K, int64_t segsp,
+    const float *__restrict__ A, int64_t lda, int64_t M, int64_t K, int64_t kwrap, int64_t segsp,
     int *__restrict__ row_exp, uint4 *__restrict__ out, int *__restrict__ clear, int nclear,
     int nblocks) {
   // every argument in SGPRs up front (one round of scalar loads); the grid
@@ -1051,6 +1053,7 @@ __global__ __launch_bounds__(64 * kPrepWaves) void k_prep_a(
   const int64_t kp = segsp * kSegK;  // padded K
   const bool vec = ((lda & 3) == 0) && ((((uintptr_t)A) & 15) == 0);
   auto load8 = [&](int64_t k0, float *v) {
+    if constexpr (WRAP) k0 = k0 < kwrap ? k0 : k0 - kwrap;
     const float *ar = A + row * lda + k0;
     if (row < M && vec && k0 + 8 <= K) {
       const float4 x0 = *(const float4 *)ar;
@@ -1110,11 +1113,12 @@ __global__ __launch_bounds__(64 * kPrepWaves) void k_prep_a(
   }
 }
 
-static int launch_prep_a(mmnb_ctx *ctx, const float *d_a, int64_t lda, int64_t m, int64_t k,
-                         int64_t mpad, int64_t segsp, int *d_exp, uint4 *d_ap, int *clear,
+static int launch_prep_a(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
+                         int64_t m, int64_t mpad, int64_t segsp, int *d_exp, uint4 *d_ap, int *clear,
                          int nclear) {
-  return launch(ctx, kKernPrep, k_prep_a, dim3((unsigned)mpad), dim3(64 * kPrepWaves), 0, d_a,
-                lda, m, k, segsp, d_exp, d_ap, clear, nclear, (int)mpad);
+  auto kern = p->wraps() ? k_prep_a<true> : k_prep_a<false>;
+  return launch(ctx, kKernPrep, kern, dim3((unsigned)mpad), dim3(64 * kPrepWaves), 0, d_a, lda,
+                m, p->k_read(), p->k_wrap(), segsp, d_exp, d_ap, clear, nclear, (int)mpad);
 }
 
 // ---------------------------------------------------------------------------
@@ -1152,13 +1156,15 @@ constexpr int kGemmBN = 128;  // four 32-column blocks
 constexpr int kGemmGroup = 2; // row bands per tile group (L2 reuse of A)
 
 
-template <int NBPS, int NST, int GROUPS, int CB>
+// BIAS: the columns' bias added where they are stored (in a kernel of its own: as an
+// argument of all, M = 512, 4096^2 went from 48.1 to 50.1 us).
+template <int NBPS, int NST, int GROUPS, int CB, bool BIAS>
 __global__ __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_mfma(
     const uint4 *__restrict__ Ap, const int *__restrict__ row_exp, int segs, int segsp,
     const uint8_t *__restrict__ W, int64_t col_bytes, const float *__restrict__ ST,
     const uint32_t *__restrict__ ZT, int ldsz, int nb, int bs_log2, int M, int N, int grid_x,
-    int grid_y, float *__restrict__ Y, int ksplit, float *__restrict__ part,
-    int *__restrict__ tile_cnt) {
+    int grid_y, float *__restrict__ Y, const float *__restrict__ bias, int ksplit,
+    float *__restrict__ part, int *__restrict__ tile_cnt) {
   constexpr int kBN = kGemmBN * CB;                    // columns per workgroup tile
   constexpr int kSz = kBN * NBPS;                       // scale (and zero-point) dwords per stage
   constexpr int kStageU4 = 1024 + 256 * CB + kSz / 2;   // uint4 per stage: A, W, scales + zp
@@ -1255,6 +1261,10 @@ __global__ __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(2,
     col[cb] = colok[cb] ? ccol : N - 1;
     my_c[cb] = (wave * CB + cb) * 32 + cl;
   }
+  // their bias, loaded now as the exponents above
+  float bv[CB];
+#pragma unroll
+  for (int cb = 0; cb < CB; cb++) bv[cb] = BIAS ? bias[col[cb]] : 0.0f;
 
   auto issue = [&](int seg, int buf) {
     const int sa_ = min(seg, segsp - 1);
@@ -1657,7 +1667,8 @@ __global__ __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(2,
         const int tr = rb * 32 + (r >> 2) * 8 + g * 4 + (r & 3);  // row in the tile
         const int row = rb0 * 32 + tr;
         const int ex = __shfl(rexp, tr, 64);
-        if (colok[cb] && row < M) Y[(size_t)row * N + col[cb]] = ldexpf(acc[rb][cb][r], -ex);
+        const float v = ldexpf(acc[rb][cb][r], -ex);
+        if (colok[cb] && row < M) Y[(size_t)row * N + col[cb]] = BIAS ? v + bv[cb] : v;
       }
     }
   }
@@ -1736,7 +1747,8 @@ static int gemm_run(mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, const GemmPlan
   const dim3 grid((unsigned)(gx * gy * ksplit));
 #define MMNB_GEMM_LAUNCH(Q, NS, GR, CB)                                                      \
   {                                                                                          \
-    auto kern = k_gemm_mfma<Q, NS, GR, CB>;                                                  \
+    auto kern = p->direct_bias() ? k_gemm_mfma<Q, NS, GR, CB, true>                          \
+                                 : k_gemm_mfma<Q, NS, GR, CB, false>;                        \
     if (shmem > 65536) {                                                                     \
       hipError_t e_ = hipFuncSetAttribute(                                                   \
           (const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);       \
@@ -1745,7 +1757,7 @@ static int gemm_run(mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, const GemmPlan
     return launch(ctx, kKernGemm, kern, grid, dim3(256 * GR), shmem, (const uint4 *)d_ap,   \
                   (const int *)d_exp, (int)segs, (int)segsp, p->d_w, p->col_bytes,          \
                   p->d_st, p->d_zt, (int)p->ldsz, (int)p->n_blocks, bs_log2, (int)m,        \
-                  (int)p->n, gx, gy, d_y, ksplit, (float *)d_part, d_cnt);                  \
+                  (int)p->n, gx, gy, d_y, p->direct_bias(), ksplit, (float *)d_part, d_cnt); \
   }
 #define MMNB_GEMM_NB(NS, GR, CB)                     \
   {                                                  \
@@ -1784,7 +1796,7 @@ int launch_nbits_gemm(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64
   if ((rc = scratch_get(ctx, 2, pl.ap_bytes, &d_ap))) return rc;
   if ((rc = scratch_get(ctx, 3, (size_t)pl.mpad * 4, &d_exp))) return rc;
   if ((rc = gemm_ctx_part(ctx, pl, &d_part))) return rc;
-  if ((rc = launch_prep_a(ctx, d_a, lda, m, p->k, pl.mpad, pl.segsp, (int *)d_exp,
+  if ((rc = launch_prep_a(ctx, p, d_a, lda, m, pl.mpad, pl.segsp, (int *)d_exp,
                            (uint4 *)d_ap, nullptr, 0)))
     return rc;
   return gemm_run(ctx, p, m, pl, d_ap, d_exp, d_y, d_part, ctx->d_gemm_cnt);
@@ -1822,7 +1834,7 @@ static NbitsRoute nbits_route(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m
   if (p->generic) return kRouteGeneric;
   if (m == 1) return kRouteGemv;
   if (ctx->gemm_cb || ctx->gemm_ksplit || ctx->gemm_stages != 2) return kRouteGemm;
-  if (gemv_multi_takes(ctx, p, m)) return kRouteGemvMulti;
+  if (!p->ext && gemv_multi_takes(ctx, p, m)) return kRouteGemvMulti;
   return nbits_skinny_plan(ctx, p, m, cw, nsl) ? kRouteSkinny : kRouteGemm;
 }
 
@@ -1874,7 +1886,7 @@ int launch_matmul_nbits_ws(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, 
   char *b = (char *)ws;
   int *d_cnt = (int *)(b + o_cnt);
   const int nclear = pl.ksplit > 1 ? (int)pl.tiles : 0;
-  if ((rc = launch_prep_a(ctx, d_a, lda, m, p->k, pl.mpad, pl.segsp, (int *)(b + o_exp),
+  if ((rc = launch_prep_a(ctx, p, d_a, lda, m, pl.mpad, pl.segsp, (int *)(b + o_exp),
                            (uint4 *)(b + o_ap), d_cnt, nclear)))
     return rc;
   return gemm_run(ctx, p, m, pl, b + o_ap, b + o_exp, d_y,

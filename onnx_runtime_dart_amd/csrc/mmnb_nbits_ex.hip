@@ -6,18 +6,23 @@
 // 4-bit weight of Kv rows), plus an optional A gather before and one
 // correction pass after the product:
 //
-//   bits = 8:  (one row with integer zero points: k_gemv8, directly)
-//              q8 = 16 hi + lo, so (q8 - z) s = (hi - 8)(16 s) + (lo - 8) s
-//              + (136 - z) s.  The virtual weight stacks the hi plane (scale
-//              16 s, exact) over the lo plane (scale s), both with zero
-//              point 8, over Kv = 2 * ceil(K/bs) * bs rows; A is gathered as
-//              [A | A]; the last term is the correction below.
+//   bits = 8:  q8 = 16 hi + lo.  The virtual weight stacks the hi plane (scale
+//              16 s, exact) over the lo plane (scale s), over Kv = 2 * kp rows (kp:
+//              K padded to whole blocks and 64-k segments).  Without zero points
+//              (q8 - 128) s = (hi - 8)(16 s) + lo s: the planes have zero points 8
+//              and 0, the kernels read A again from row kp on, and no correction is
+//              left.  Otherwise both planes have zero point 8, A is gathered as
+//              [A | A], and (136 - z) s is the correction below (zero points z / 16
+//              and z % 16 in the planes need none, but the larger terms left the GEMM
+//              5% further from the 64-bit product).  One row with integer zero points
+//              takes k_gemv8, on the joined bytes.
 //   float zp:  (q - z) s = q s - z s: the kernels run with zero point 0 and
 //              the correction adds -z s per block.
 //   g_idx:     the rows are sorted by group (stable), so every group is one
 //              block of the virtual weight; A is gathered in the same order.
 //              Each group must hold exactly block_size rows.
-//   bias:      added in the correction pass.
+//   bias:      added where the kernels store a result, or in the correction pass
+//              where there is one.
 //
 // Correction: y[m, n] += bias[n] + sum_b c[b][n] * asum[m][b], with asum the
 // block sums of the (gathered) A over the first corr_nb blocks.  c is built
@@ -272,7 +277,7 @@ static int launch_gemv8_r(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, b
   const float *bias = p->d_bias ? p->d_bias : p->d_scales;
 #define MMNB_GEMV8(ZP, F)                                                                     \
   return launch(ctx, kKernGemv, k_gemv8<R, NBPC, ZP, F>, grid, block, 0, d_a, p->d_w,         \
-                p->col_bytes, p->d_scales, p->d_z8, bias, (int)p->corr_nb, bs_log2,           \
+                p->col_bytes, p->d_scales, p->d_z8, bias, (int)p->nb8, bs_log2,               \
                 (int)p->k_in, (int)n, d_y, C, iters, (int)p->n_blocks)
   if (p->d_z8) {
     if (fast) MMNB_GEMV8(true, true);
@@ -297,10 +302,14 @@ static int launch_gemv8(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int
 int run_matmul_nbits(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
                      int64_t m, float *d_y) {
   if (!p->ext) return launch_matmul_nbits(ctx, p, d_a, lda, m, d_y);
-  // one row: the GEMVs that take 8-bit weights and the bias in one launch
   if (m == 1 && p->bytes8) return launch_gemv8(ctx, p, d_a, lda, d_y);
-  if (m == 1 && !p->d_asrc && !p->d_corr && p->d_bias)
-    return launch_gemv_bias(ctx, p, d_a, lda, d_y);
+  // without gather and correction the kernels take A and the bias themselves (us a
+  // call with the passes and without, block 128: 8 bits, bias, M = 8, 4096^2 34.2 and
+  // 12.0; M = 24 39.2 and 18.4; M = 512 120 and 78; M = 24, 1024^2 21.2 and 8.9; 4
+  // bits, bias, M = 8, (1000, 3001) 8.8 and 4.8)
+  if (p->direct())
+    return m > 1 ? launch_matmul_nbits(ctx, p, d_a, lda, m, d_y)
+                 : launch_gemv_bias(ctx, p, d_a, lda, d_y);
   int rc;
   const float *a2 = d_a;
   int64_t lda2 = lda, ka = p->k_in;
@@ -367,14 +376,14 @@ int mmnb_pack_nbits_ex(mmnb_ctx *ctx, const mmnb_nbits_desc *d, mmnb_pack **out)
     if ((rc = set_device(ctx))) return rc;
     // the reference's own form takes any even block size (pack_nbits_any);
     // the extensions run on power-of-two blocks (nbits_prepare checks)
-    const bool plain = h.asrc.empty() && h.corr.empty() && h.bias.empty();
+    const bool plain = h.asrc.empty() && h.corr.empty() && h.bias.empty() && !h.planes;
     const uint8_t *vz = h.vz.empty() ? nullptr : h.vz.data();
     rc = plain ? pack_nbits_any(ctx, h.vb.data(), h.vs.data(), vz, h.zfill, h.kv, h.n, h.block, &p)
                : pack_nbits_core(ctx, h.vb.data(), h.vs.data(), vz, h.zfill, h.kv, h.n, h.block,
                                  &p);
     if (rc) return rc;
     p->k_in = h.k;
-    p->ext = !h.asrc.empty() || !h.corr.empty() || !h.bias.empty();
+    p->ext = !plain;
     if (!h.asrc.empty()) urc = upload(p, h.asrc, &p->d_asrc);
     if (!urc && !h.corr.empty()) {
       std::vector<float> c32(h.corr.begin(), h.corr.end());
@@ -383,6 +392,7 @@ int mmnb_pack_nbits_ex(mmnb_ctx *ctx, const mmnb_nbits_desc *d, mmnb_pack **out)
     }
     if (!urc && !h.bias.empty()) urc = upload(p, h.bias, &p->d_bias);
     p->bytes8 = h.bytes8;
+    p->nb8 = h.n_blocks;
     if (!urc && !h.z8.empty()) urc = upload(p, h.z8, &p->d_z8);
   }
   if (urc) {

@@ -119,9 +119,9 @@ struct SkRows {
 template <int V, int CW, int KW, int NBPS>
 __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
     const float *__restrict__ Aall, int64_t lda, const uint8_t *__restrict__ Wt,
-    const float *__restrict__ ST, int ldsz, int nb, int bs_log2, int segs, int K, int Mall, int N,
-    float *__restrict__ Yall, int nchunks, int cps, int nsl, int gy, int vec, float *__restrict__ part,
-    int *__restrict__ tile_cnt) {
+    const float *__restrict__ ST, int ldsz, int nb, int bs_log2, int segs, int K, int kwrap,
+    int Mall, int N, float *__restrict__ Yall, const float *__restrict__ bias, int nchunks, int cps,
+    int nsl, int gy, int vec, float *__restrict__ part, int *__restrict__ tile_cnt) {
   using R = SkRows<V>;
   static_assert(CW * KW == 8, "eight waves");
   constexpr int kWS = kSkSegs / KW;   // segments of a chunk per k wave
@@ -129,8 +129,8 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
   constexpr int kJB = 4 / NBPS;       // 16-k steps per quantisation block
   extern __shared__ u4vec sk_smem[];  // operand units, then (reused) the k waves' tiles
   __shared__ int sex[R::kMax];        // piece exponents of the staged chunk
-  kernarg_fence(Aall, lda, Wt, ST, ldsz, nb, bs_log2, segs, K, Mall, N, Yall, nchunks, cps, nsl,
-                gy, vec, part, tile_cnt);
+  kernarg_fence(Aall, lda, Wt, ST, ldsz, nb, bs_log2, segs, K, kwrap, Mall, N, Yall, bias, nchunks,
+                cps, nsl, gy, vec, part, tile_cnt);
   const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63, cl = lane & 31, g = lane >> 5;
   const int cw = wid % CW, kw = wid / CW;
@@ -173,8 +173,11 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
     }
   };
   float av[R::kPer][8];
+  // the column of A under row k of the weight (8-bit weights: two planes of kwrap
+  // rows, a multiple of 64, over the same A)
+  auto col_of = [&](int k) __attribute__((always_inline)) { return k < kwrap ? k : k - kwrap; };
   auto load_a = [&](int c) __attribute__((always_inline)) {
-    const int kc = c * kSkChunk, k0 = kc + 8 * lane;
+    const int kc = c * kSkChunk, k0 = col_of(kc + 8 * lane);
     if (vec && (kc + kSkChunk <= K || (K & 7) == 0)) {  // uniform
       // a lane past a row's end reads its last 8 values and drops them
       const uint32_t off = 4u * (uint32_t)min(k0, K - 8);
@@ -203,7 +206,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
   // it all fall on the same banks.
   auto stage = [&](int c) __attribute__((always_inline)) {
     const int u = lane >> 1, gg = lane & 1;
-    const int left = K - (c * kSkChunk + 8 * lane);  // values of the lane inside K
+    const int left = K - col_of(c * kSkChunk + 8 * lane);  // values of the lane inside K
     if (c * kSkChunk + kSkChunk > K) {                // uniform
 #pragma unroll
       for (int i = 0; i < R::kPer; i++)
@@ -362,7 +365,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
     const float v = (float)sum;
     if (nsl == 1) {
       const int cc = n0 + e % kBN;
-      if (cc < N) Y[(int64_t)(e / kBN) * N + cc] = v;
+      if (cc < N) Y[(int64_t)(e / kBN) * N + cc] = bias ? v + bias[cc] : v;
     } else {
       st_act<true>(pt + slice * (R::kMax * kBN) + e, v);
     }
@@ -391,7 +394,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
     for (int q = 1; q < kSkMaxSlices; q++) sum += q < nsl ? (double)t[q] : 0.0;
     const float v = (float)sum;
     const int cc = n0 + e % kBN;
-    if (cc < N) Y[(int64_t)(e / kBN) * N + cc] = v;
+    if (cc < N) Y[(int64_t)(e / kBN) * N + cc] = bias ? v + bias[cc] : v;
   }
   if (threadIdx.x == 0)
     __hip_atomic_store(&tile_cnt[tile], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -423,8 +426,9 @@ static int launch_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, in
     return launch(ctx, kKernGemv, kern, dim3((unsigned)nsl, (unsigned)tiles, (unsigned)((m + R::kMax - 1) / R::kMax)), dim3(kSkThreads),      \
                   shmem, d_a, lda, (const uint8_t *)p->d_wt,                     \
                   (const float *)p->d_st, (int)p->ldsz, (int)p->n_blocks, bs_log2,            \
-                  (int)(p->k64 / kSegK), (int)p->k, (int)m, (int)n, d_y, nchunks, cps, nsl, tiles, vec,   \
-                  ctx->d_sk_part, ctx->d_gemm_cnt);                                           \
+                  (int)(p->k64 / kSegK), (int)p->k_read(), (int)p->k_wrap(), (int)m, (int)n,  \
+                  d_y, p->direct_bias(), nchunks, cps, nsl, tiles, vec, ctx->d_sk_part,       \
+                  ctx->d_gemm_cnt);                                                           \
   }
   if (p->block >= 64) MMNB_SKINNY(1);
   if (p->block == 32) MMNB_SKINNY(2);

@@ -1,6 +1,6 @@
-"""GPU parity of the one-launch GEMVs of extended packs (one row): 8-bit weights with
-integer zero points (k_gemv8) and 4-bit weights with a bias, at the edges of their
-chunks, waves and column groups; and the padded nibble planes with more rows.
+"""GPU parity of extended packs that need no correction pass: 8-bit weights with integer
+zero points (k_gemv8 for one row, else the planes through the few-row kernel and the
+GEMM) and 4-bit weights with a bias, at the edges of chunks, planes and column groups.
 
 Bar: |y - y64| <= gamma_{K + n_blocks + 4} * sum|a| |q - zp| scale (+ |bias|) for one
 row, whose kernels form q - zp exactly (no hi/lo split and no correction); the bound of
@@ -40,7 +40,16 @@ def _problem(m, k, n, bits, bs, zp, bias, seed):
     (1, 1000, 4096, 8, 128, True, True),   # a partial block
     (3, 96, 70, 8, 32, True, True),        # padded planes through the few-row kernel
     (100, 96, 70, 8, 32, True, False),     # ... and through the GEMM
-    (1, 1000, 301, 4, 32, True, True),     # 4-bit weights with a bias
+    (2, 36, 33, 8, 16, True, True),        # rows that are not whole 8-k runs
+    (8, 1000, 130, 8, 128, True, True),    # the second plane inside a 512-k piece
+    (16, 4096, 96, 8, 32, False, True),    # K slices
+    (20, 700, 65, 8, 64, True, False),
+    (600, 1000, 520, 8, 128, True, True),  # the GEMM, tiles with and without K groups
+    (70, 4160, 300, 8, 64, False, True),   # ... its K slices
+    (5, 1000, 301, 4, 32, True, True),     # 4-bit weights with a bias, several rows
+    (24, 4096, 100, 4, 128, False, True),
+    (130, 2048, 300, 4, 64, True, True),
+    (1, 1000, 301, 4, 32, True, True),     # ... and one
     (1, 4160, 3, 4, 128, False, True),
 ])
 def test_one_row_gemvs(m, k, n, bits, bs, zp, bias):
