@@ -121,7 +121,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
     const float *__restrict__ Aall, int64_t lda, const uint8_t *__restrict__ Wt,
     const float *__restrict__ ST, int ldsz, int nb, int bs_log2, int segs, int K, int kwrap,
     int Mall, int N, float *__restrict__ Yall, const float *__restrict__ bias, int nchunks, int cps,
-    int nsl, int gy, int vec, float *__restrict__ part, int *__restrict__ tile_cnt) {
+    int nsl, int gy, float *__restrict__ part, int *__restrict__ tile_cnt) {
   using R = SkRows<V>;
   static_assert(CW * KW == 8, "eight waves");
   constexpr int kWS = kSkSegs / KW;   // segments of a chunk per k wave
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
   extern __shared__ u4vec sk_smem[];  // operand units, then (reused) the k waves' tiles
   __shared__ int sex[R::kMax];        // piece exponents of the staged chunk
   kernarg_fence(Aall, lda, Wt, ST, ldsz, nb, bs_log2, segs, K, kwrap, Mall, N, Yall, bias, nchunks,
-                cps, nsl, gy, vec, part, tile_cnt);
+                cps, nsl, gy, part, tile_cnt);
   const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63, cl = lane & 31, g = lane >> 5;
   const int cw = wid % CW, kw = wid / CW;
@@ -178,16 +178,22 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
   auto col_of = [&](int k) __attribute__((always_inline)) { return k < kwrap ? k : k - kwrap; };
   auto load_a = [&](int c) __attribute__((always_inline)) {
     const int kc = c * kSkChunk, k0 = col_of(kc + 8 * lane);
-    if (vec && (kc + kSkChunk <= K || (K & 7) == 0)) {  // uniform
-      // a lane past a row's end reads its last 8 values and drops them
-      const uint32_t off = 4u * (uint32_t)min(k0, K - 8);
+    // (buffer loads of four dwords need no more than dword alignment: rows of any
+    // length and start.  Value by value where K % 8 or a row's alignment forbade the
+    // aligned form, M = 54, (1999, 4083) took 36.3 us, M = 3, (859, 2142) 6.7; now
+    // 15.2 and 4.7.)
+    if (K >= 4) {  // uniform
+      // four values that end past the row's end are read from its last four, and
+      // moved to their places in stage(), which also drops those past the end
+      const uint32_t off0 = 4u * (uint32_t)min(k0, K - 4);
+      const uint32_t off1 = 4u * (uint32_t)min(k0 + 4, K - 4);
 #pragma unroll
       for (int i = 0; i < R::kPer; i++) {
         const __amdgpu_buffer_rsrc_t rs = buf_rsrc(A + (int64_t)min(wid + 8 * i, M - 1) * lda);
         const f4vec x0 =
-            __builtin_bit_cast(f4vec, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+            __builtin_bit_cast(f4vec, __builtin_amdgcn_raw_buffer_load_b128(rs, off0, 0, 0));
         const f4vec x1 =
-            __builtin_bit_cast(f4vec, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 16, 0));
+            __builtin_bit_cast(f4vec, __builtin_amdgcn_raw_buffer_load_b128(rs, off1, 0, 0));
         av[i][0] = x0.x; av[i][1] = x0.y; av[i][2] = x0.z; av[i][3] = x0.w;
         av[i][4] = x1.x; av[i][5] = x1.y; av[i][6] = x1.z; av[i][7] = x1.w;
       }
@@ -209,9 +215,20 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
     const int left = K - col_of(c * kSkChunk + 8 * lane);  // values of the lane inside K
     if (c * kSkChunk + kSkChunk > K) {                // uniform
 #pragma unroll
-      for (int i = 0; i < R::kPer; i++)
+      for (int i = 0; i < R::kPer; i++) {
+        if (K >= 4 && (K & 3)) {  // uniform: else no four values straddle the end
+#pragma unroll
+          for (int q = 0; q < 8; q += 4) {  // values q .. q + 3 were read 4 - n further on
+            const int n = left - q;
+            const float x0 = av[i][q], x1 = av[i][q + 1], x2 = av[i][q + 2], x3 = av[i][q + 3];
+            av[i][q] = n == 1 ? x3 : n == 2 ? x2 : n == 3 ? x1 : x0;
+            av[i][q + 1] = n == 2 ? x3 : n == 3 ? x2 : x1;
+            av[i][q + 2] = n == 3 ? x3 : x2;
+          }
+        }
 #pragma unroll
         for (int e = 0; e < 8; e++) av[i][e] = e < left ? av[i][e] : 0.0f;
+      }
     }
 #pragma unroll
     for (int i = 0; i < R::kPer; i++) {
@@ -412,7 +429,6 @@ static int launch_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, in
   nsl = (nchunks + cps - 1) / cps;
   const size_t red = (size_t)KW * R::kMax * 32 * CW * 4;
   const size_t shmem = std::max<size_t>((size_t)R::kUnits * 1024, red);
-  const int vec = ((lda % 4 == 0) && (((uintptr_t)d_a & 15) == 0)) ? 1 : 0;
   int bs_log2 = 0;
   while ((int64_t(1) << (bs_log2 + 1)) <= p->block) bs_log2++;
 #define MMNB_SKINNY(Q)                                                                        \
@@ -427,7 +443,7 @@ static int launch_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, in
                   shmem, d_a, lda, (const uint8_t *)p->d_wt,                     \
                   (const float *)p->d_st, (int)p->ldsz, (int)p->n_blocks, bs_log2,            \
                   (int)(p->k64 / kSegK), (int)p->k_read(), (int)p->k_wrap(), (int)m, (int)n,  \
-                  d_y, p->direct_bias(), nchunks, cps, nsl, tiles, vec, ctx->d_sk_part,       \
+                  d_y, p->direct_bias(), nchunks, cps, nsl, tiles, ctx->d_sk_part,            \
                   ctx->d_gemm_cnt);                                                           \
   }
   if (p->block >= 64) MMNB_SKINNY(1);

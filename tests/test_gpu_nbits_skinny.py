@@ -35,6 +35,11 @@ CASES = [
     (70, 4096, 64, 128, False),    # row groups with K slices
     (4, 300, 40, 1024, True),      # a block longer than K
     (3, 2500, 31, 16, False),
+    (3, 859, 33, 128, False),      # rows of no alignment: K % 4 = 3, 2, 1
+    (20, 1514, 65, 32, True),
+    (54, 2001, 64, 128, False),
+    (2, 5, 7, 16, True),
+    (4, 3, 5, 16, False),          # fewer than four values
 ]
 
 
