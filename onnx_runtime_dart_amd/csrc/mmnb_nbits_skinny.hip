@@ -21,10 +21,13 @@
 //
 // Row layout V of the 32-row operand tile.  With few rows the tile's free
 // rows hold the other terms of the split, so one MFMA multiplies all of them:
-//   0: M <= 8,  three terms at rows 8p + m: 33 bits, i.e. the activations
-//      exactly as fp32 held them (elements below 2^-15 of the piece's maximum
-//      to 2^-39 of it): 7.3e-8 .. 9e-8 off the 64-bit product where the fp32
-//      FMA kernel is 1.0e-7 .. 1.3e-7 (K = 1024 .. 4096, 2-norm);
+//   0: M <= 8,  three terms at rows 8p + m, each times a power of two of its
+//      own (kSkGain1, kSkGain2): the activations exactly as fp32 holds them,
+//      down to 2^-39 of the piece's largest.  What the terms miss of smaller
+//      ones is multiplied at the end, in passes with a power of two of their
+//      own until nothing is left (9 at most, over the whole range of fp32):
+//      7.3e-8 .. 9e-8 off the 64-bit product where the fp32 FMA kernel is
+//      1.0e-7 .. 1.3e-7 (K = 1024 .. 4096, 2-norm);
 //   1: M <= 16, two terms at rows 16p + m;
 //   2: M <= 32, two MFMAs (hi, lo) per step.
 // Two terms are what the prefill GEMM uses (they leave 2^-22); with a power of
@@ -48,6 +51,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "mmnb_device.h"
 #include "mmnb_internal.h"
@@ -103,7 +107,12 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
                          (uint32_t)__builtin_amdgcn_readlane((int)v, 16));
   const uint32_t b = max((uint32_t)__builtin_amdgcn_readlane((int)v, 32),
                          (uint32_t)__builtin_amdgcn_readlane((int)v, 48));
-  return max(a, b);
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)max(a, b));
+}
+// The power of two that takes a finite magnitude's bits to [2^13, 2^14) (subnormal
+// ones, and 0, as far as the smallest normal one), in scalar integers.
+__device__ __forceinline__ int sk_exponent(uint32_t bits) {
+  return 140 - (int)max(bits >> 23, 1u);
 }
 
 template <int V>
@@ -115,6 +124,14 @@ struct SkRows {
   static constexpr int kPer = kMax / 8;                  // row pieces per wave
   static constexpr int kUnits = 32 * kMfma;        // 1 KB operand units per chunk
 };
+
+// Layout 0: log2 of the second and third term's powers of two.  A scaled
+// activation x is below 2^14, so the first fp16 term misses at most 4 of it and
+// the second, of that times 2^13, 8: every term stays below 2^16.  The third has
+// a resolution of 2^-48, the ulp of the binary32 numbers from 2^-25 on: from there
+// up the three terms add up to x.
+constexpr int kSkGain1 = 13, kSkGain2 = 24;
+constexpr int kSkWindow = -25;
 
 template <int V, int CW, int KW, int NBPS>
 __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
@@ -129,6 +146,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
   constexpr int kJB = 4 / NBPS;       // 16-k steps per quantisation block
   extern __shared__ u4vec sk_smem[];  // operand units, then (reused) the k waves' tiles
   __shared__ int sex[R::kMax];        // piece exponents of the staged chunk
+  __shared__ __align__(16) int srest[8];  // waves whose terms miss something (layout 0)
   kernarg_fence(Aall, lda, Wt, ST, ldsz, nb, bs_log2, segs, K, kwrap, Mall, N, Yall, bias, nchunks,
                 cps, nsl, gy, part, tile_cnt);
   const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -210,8 +228,8 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
   // 16-k step u = l >> 1 (unit u of a part).  A unit's 32 rows are stored at
   // row ^ u: the 64 lanes of a piece write one row of 32 units, which without
   // it all fall on the same banks.
-  auto stage = [&](int c) __attribute__((always_inline)) {
-    const int u = lane >> 1, gg = lane & 1;
+  // (Values that end past the row's end to their places, those past it dropped.)
+  auto trim = [&](int c) __attribute__((always_inline)) {
     const int left = K - col_of(c * kSkChunk + 8 * lane);  // values of the lane inside K
     if (c * kSkChunk + kSkChunk > K) {                // uniform
 #pragma unroll
@@ -230,6 +248,10 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
         for (int e = 0; e < 8; e++) av[i][e] = e < left ? av[i][e] : 0.0f;
       }
     }
+  };
+  // STORE: to LDS.  REST: av becomes what the terms miss (layout 0).
+  auto stage = [&](auto STORE, auto REST) __attribute__((always_inline)) {
+    const int u = lane >> 1, gg = lane & 1;
 #pragma unroll
     for (int i = 0; i < R::kPer; i++) {
       const int row = wid + 8 * i;  // wave-uniform
@@ -249,23 +271,48 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
           mu = max(mu, __builtin_bit_cast(uint32_t, finite_abs(av[i][e])));
         mu = wave_max_u32(mu);
       }
-      const int ex = prep_a_exponent(__builtin_bit_cast(float, mu));
+      const int ex = sk_exponent(mu);
       half2_t t[R::kParts][4];  // pairs (e, e + 4): the operand's k order
+      constexpr int kUp[3] = {0, V == 0 ? kSkGain1 : 0, V == 0 ? kSkGain2 - kSkGain1 : 0};
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         f2vec x = {ldexpf(av[i][e], ex), ldexpf(av[i][e + 4], ex)};
         t[0][e] = __builtin_convertvector(x, half2_t);
 #pragma unroll
         for (int p = 1; p < R::kParts; p++) {
-          x.x = fmaf((float)t[p - 1][e].x, -1.0f, x.x);
-          x.y = fmaf((float)t[p - 1][e].y, -1.0f, x.y);
+          const float up = 1 << kUp[p];
+          x.x = fmaf((float)t[p - 1][e].x, -up, x.x * up);
+          x.y = fmaf((float)t[p - 1][e].y, -up, x.y * up);
           if (!fin) {  // the first term alone, so that the sums follow IEEE
             x.x = x.x == x.x ? x.x : 0.0f;
             x.y = x.y == x.y ? x.y : 0.0f;
           }
           t[p][e] = __builtin_convertvector(x, half2_t);
         }
+        if constexpr (REST) {
+          // (below 2^-50 all terms are 0, and x may be subnormal and rounded; a row
+          // with an infinity or NaN is one or the other in every column)
+          const float tiny = ldexpf(1.0f, -50 - ex);
+          x.x -= (float)t[2][e].x;
+          x.y -= (float)t[2][e].y;
+          av[i][e] = fabsf(av[i][e]) < tiny ? av[i][e] : ldexpf(x.x, -kSkGain2 - ex);
+          av[i][e + 4] = fabsf(av[i][e + 4]) < tiny ? av[i][e + 4] : ldexpf(x.y, -kSkGain2 - ex);
+          av[i][e] = fin ? av[i][e] : 0.0f;
+          av[i][e + 4] = fin ? av[i][e + 4] : 0.0f;
+        }
       }
+      if constexpr (V == 0 && !REST) {
+        // whether the terms miss anything: a value other than 0 below the window
+        // (as integers without sign and less 1, in which 0 is the largest)
+        uint32_t mn = 0xFFFFFFFFu;
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+          mn = min(mn, (__builtin_bit_cast(uint32_t, av[i][e]) << 1) - 1u);
+        const uint32_t lim = __builtin_bit_cast(uint32_t, ldexpf(1.0f, kSkWindow - ex)) << 1;
+        if (__builtin_amdgcn_ballot_w64(mn < max(lim, 1u) - 1u) != 0 && lane == 0)
+          srest[wid] = row < M;
+      }
+      if (!STORE) continue;
       if (row < M) {  // wave-uniform
         if (lane == 0) sex[row] = ex;
 #pragma unroll
@@ -291,15 +338,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
   // segments multiplied together: independent accumulators, so that a step's
   // MFMA does not wait for the one before it
   constexpr int kG = kWS < 2 ? 1 : 2;
-  auto chunk = [&](const int c, const Weights &wc, Weights &wn) __attribute__((always_inline)) {
-    stage(c);
-    // the next chunk's loads go out before this one is multiplied, the
-    // activations first: the next stage() waits for them alone
-    if (c + 1 < c1) {  // uniform
-      load_a(c + 1);
-      load_w(wn, c + 1);
-    }
-    sk_lds_barrier();
+  auto multiply = [&](const int c, const Weights &wc) __attribute__((always_inline)) {
     float acc[16];
 #pragma unroll
     for (int r = 0; r < 16; r++) acc[r] = 0.0f;
@@ -347,18 +386,62 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
     for (int i = 0; i < R::kOut; i++) {
       const int row = (i >> 2) * 8 + g * 4 + (i & 3);
       float v = acc[i];
-      if constexpr (V == 0) v = (acc[8 + i] + acc[4 + i]) + acc[i];
+      if constexpr (V == 0) v = fmaf(fmaf(acc[8 + i], 0x1p-11f, acc[4 + i]), 0x1p-13f, acc[i]);
       if constexpr (V == 1) v = acc[8 + i] + acc[i];
       tot[i] += ldexpf(v, -sex[row]);
     }
-    sk_lds_barrier();  // every wave is done with the staged chunk
   };
-  Weights w0, w1;
+  const std::true_type yes;
+  const std::false_type no;
+  if (V == 0 && lane == 0) srest[wid] = 0;
+  Weights w0;
   load_a(c0);
   load_w(w0, c0);
-  for (int c = c0; c < c1; c += 2) {
-    chunk(c, w0, w1);
-    if (c + 1 < c1) chunk(c + 1, w1, w0);
+  for (int c = c0; c < c1; c++) {
+    trim(c);
+    stage(yes, no);
+    // the next chunk's loads go out before this one is multiplied, the
+    // activations first: the next stage() waits for them alone.  (The weights are
+    // moved, not alternated between two copies of the loop's code: M = 8, (4096,
+    // 14336) 16.4 -> 14.6 us, (1024, 1024) 4.75 -> 4.6.)
+    const Weights wc = w0;
+    if (c + 1 < c1) {  // uniform
+      load_a(c + 1);
+      load_w(w0, c + 1);
+    }
+    sk_lds_barrier();
+    multiply(c, wc);
+    sk_lds_barrier();  // every wave is done with the staged chunk
+  }
+  if constexpr (V == 0) {
+    auto any_rest = [&]() __attribute__((always_inline)) {
+      int r = 0;
+#pragma unroll
+      for (int q = 0; q < 8; q++) r |= srest[q];
+      return __builtin_amdgcn_readfirstlane(r) != 0;  // of the workgroup
+    };
+    if (__builtin_expect(any_rest(), 0)) {
+      for (int c = c0; c < c1; c++) {
+        load_a(c);
+        trim(c);
+        stage(no, yes);
+        while (true) {
+          int nz = 0;
+#pragma unroll
+          for (int e = 0; e < 8; e++) nz |= av[0][e] != 0.0f;
+          nz = __any(nz) && wid < M;
+          sk_lds_barrier();  // every wave has read srest
+          if (lane == 0) srest[wid] = nz;
+          sk_lds_barrier();
+          if (!any_rest()) break;
+          stage(yes, yes);  // (zeros in the rows with nothing left)
+          load_w(w0, c);
+          sk_lds_barrier();
+          multiply(c, w0);
+          sk_lds_barrier();
+        }
+      }
+    }
   }
 
   // ---- the k waves' tiles -> LDS [kw][row][kBN], summed by all threads

@@ -72,3 +72,40 @@ def test_few_rows(m, k, n, block, zp, offset):
         da.free()
         dy.free()
         pack.free()
+
+
+def _spread(p, rng, ratios):
+    """Rows whose magnitudes differ by powers of `ratios` inside 512 k, the large ones over
+    weights that equal their zero point, so that no large product hides a lost small one."""
+    n, nb, half = p.b_q.shape
+    zi = np.arange(n * nb)
+    z = np.full(n * nb, 8, np.uint8) if p.zero_points is None else \
+        (p.zero_points[zi >> 1] >> (4 * (zi & 1))) & 15
+    z = z.astype(np.uint8).reshape(n, nb)
+    for r, ratio in enumerate(ratios):
+        for k in rng.choice(p.k, max(1, p.k // 300), replace=False):
+            p.a[:, k] = 0.0
+            p.a[r, k] = ratio
+            b, i, sh = k // p.block, k % p.block // 2, 4 * (k & 1)
+            p.b_q[:, b, i] = (p.b_q[:, b, i] & (0xF0 >> sh)) | (z[:, b] << sh)
+
+
+@pytest.mark.parametrize("m,k,n,block,zp,ratios", [
+    (5, 512, 40, 32, True, (1e6, 1e8, 1e12, 1e20, 1e38)),     # one piece, every row another
+    (8, 4096, 70, 128, False, (1e9, 1.0, 1e38)),              # K slices; rows without
+    (2, 1999, 33, 64, True, (1e15,)),                         # a cut chunk, K % 4 = 3
+    (6, 1000, 3001, 32, False, (1e11, 1e13, 1e10)),           # 32-column workgroups
+    (3, 20, 9, 16, True, (1e12, 1e30)),
+    (8, 6000, 9000, 16, False, (1e13, 1e25)),                 # several chunks without slices
+])
+def test_magnitudes_of_any_range_in_a_row(m, k, n, block, zp, ratios):
+    ctx = _lib.default_context()
+    p = synth.mmnb_problem(m, k, n, block, zp, seed=5 * m + k)
+    rng = np.random.default_rng(k)
+    p.a[m - 1, 1::2] *= np.float32(2.0) ** rng.integers(-140, 30, p.a[m - 1, 1::2].shape)
+    _spread(p, rng, ratios)
+    y = ops.op_matmul_nbits(p.a, p.b_q, p.scales, p.zero_points, k=k, n=n, bits=4,
+                            block_size=block, ctx=ctx)
+    y64, absdot = refcpu.matmul_nbits_f64(p.a, p.b_q, p.scales, p.zero_points, k, n, block)
+    gam = (k + 2) * U / (1 - (k + 2) * U)
+    assert np.all(np.abs(y - y64) <= gam * absdot + 1e-30)
