@@ -150,6 +150,7 @@ __global__ __launch_bounds__(256) void k_nbits_correct_rows(
 // correction) -> 5.1 us back to back, 3.4 TB/s of weights and scales.
 // ---------------------------------------------------------------------------
 constexpr int kGemv8Waves = 4;
+typedef float gemv8_f4 __attribute__((ext_vector_type(4), aligned(4)));
 
 template <int R, int NBPC, bool HAS_ZP, bool FAST>
 __global__ __launch_bounds__(64 * kGemv8Waves) void k_gemv8(
@@ -180,14 +181,23 @@ __global__ __launch_bounds__(64 * kGemv8Waves) void k_gemv8(
     if constexpr (FAST) {
       load_chunk32_paired(ar, h, av);
     } else {
+      // rows that do not fill the plane or start off 16 bytes: four values at a time
+      // (dword-aligned loads); those that end past the row are its last four, moved to
+      // their places below.  (Value by value, 32 loads a lane, block 128: K = 1000, N =
+      // 14336 15.1 us and the former gather, GEMV and correction 10.6; now 5.9.  K =
+      // 4000, N = 14336 56.4 and 22.5; now 15.2.  K = 1000, N = 4096 5.8 and 8.6; 3.8.)
 #pragma unroll
-      for (int j = 0; j < 4; j++)
+      for (int i = 0; i < 8; i++) {
+        const int k = s * kSegK + 8 * g + 16 * (i >> 1) + 4 * (i & 1);
+        if (K >= 4) {  // uniform
+          const gemv8_f4 x = *(const gemv8_f4 *)(A + min(k, K - 4));
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-          const int k = s * kSegK + 8 * g + 16 * j + e;
-          const float x = A[k < K ? k : K - 1];
-          av[8 * j + e] = (cv && k < K) ? x : 0.0f;
+          for (int e = 0; e < 4; e++) av[4 * i + e] = x[e];
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; e++) av[4 * i + e] = A[max(K - 4 + e, 0)];
         }
+      }
     }
     float sraw[R][NBPC], zraw[R][NBPC];
     bool inb[NBPC];
@@ -213,6 +223,20 @@ __global__ __launch_bounds__(64 * kGemv8Waves) void k_gemv8(
     // every load in flight before any arithmetic, column by column after it
     // (as k_gemv_valu)
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!FAST) {
+#pragma unroll
+      for (int i = 0; i < 32; i += 4) {
+        // n values inside the row, read 4 - n further on where n < 4
+        const int n = cv ? K - (s * kSegK + 8 * g + 16 * (i >> 3) + (i & 4)) : 0;
+        const float x0 = av[i], x1 = av[i + 1], x2 = av[i + 2], x3 = av[i + 3];
+        const float y0 = n == 1 ? x3 : n == 2 ? x2 : n == 3 ? x1 : x0;
+        const float y1 = n == 2 ? x3 : n == 3 ? x2 : x1, y2 = n == 3 ? x3 : x2;
+        av[i] = n > 0 ? y0 : 0.0f;
+        av[i + 1] = n > 1 ? y1 : 0.0f;
+        av[i + 2] = n > 2 ? y2 : 0.0f;
+        av[i + 3] = n > 3 ? x3 : 0.0f;
+      }
+    }
 #pragma unroll
     for (int r = 0; r < R; r++) {
 #pragma unroll

@@ -32,6 +32,10 @@ def _problem(m, k, n, bits, bs, zp, bias, seed):
 
 @pytest.mark.parametrize("m,k,n,bits,bs,zp,bias", [
     (1, 16, 1, 8, 16, True, False),        # one block, one column
+    (1, 3, 5, 8, 16, True, True),          # fewer than four values
+    (1, 2907, 130, 8, 64, False, True),    # K % 4 = 3, 2, 1
+    (1, 1014, 66, 8, 32, True, False),
+    (1, 4165, 9, 8, 128, True, True),
     (1, 100, 5, 8, 16, False, True),       # ragged K, blocks of 16 (padded planes)
     (1, 96, 130, 8, 32, True, True),       # an odd number of blocks
     (1, 2048, 67, 8, 32, False, False),
