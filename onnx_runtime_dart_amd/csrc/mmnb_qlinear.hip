@@ -35,9 +35,8 @@ namespace mmnb {
 // K (kc = (c*kh + ky)*kw + kx, the weight's order) moves in chunks of 32 KB of A.
 // Per chunk a table of every kc's source offset and window position is built
 // (two divisions per entry instead of per byte), then thread t gathers the bytes
-// of position t % PT -- neighbouring lanes read neighbouring image bytes -- with
-// all of its loads in flight, out-of-image taps taking the input zero point and
-// kc >= K zero.  16-byte piece c of row r lies at c ^ (r & 15), so the 16 rows
+// of position t % PT -- neighbouring lanes read neighbouring image bytes -- with 16
+// loads in flight, out-of-image taps taking the input zero point.  16-byte piece c of row r lies at c ^ (r & 15), so the 16 rows
 // of an operand read spread over the banks.  The weights go straight to
 // registers, four 64-k steps ahead.
 //
@@ -47,11 +46,11 @@ namespace mmnb {
 // channels up to 256, so that few bytes are gathered twice, and fewer where the
 // positions alone leave the chip idle (conv_run).
 //
-// Against an upload, an im2col launch and the MatMulInteger kernel (us per call, u8 x
-// i8, back to back): 64 channels of 56 x 56, 3 x 3 to 64 24.4 -> 6.8; 3 of 112 x 112
-// to 16, stride 2 21.0 -> 5.2; 256 of 14 x 14, 3 x 3 to 256 26.3 -> 13.3; 256 of 7 x
-// 7, 5 x 5 to 256 37.8 -> 27.4; 256 of 112 x 112, 5 x 5 to 256 233 -> 169.  (4 waves
-// and 64 channels per workgroup: 9.9 us on the first, 417 on the last.)
+// Against an im2col launch and the MatMulInteger kernel (ConvInteger, us per call, u8
+// x i8, back to back; QLinearConv took 13 us more there for the parameters): 64
+// channels of 56 x 56, 3 x 3 to 64 11.6 -> 6.3; 256 of 14 x 14 to 256 12.9 -> 10.8; 512
+// of 7 x 7 to 512 18.7 -> 16.3; 512 of 28 x 28 to 512 29.0 -> 27.2; 256 of 112 x 112 to
+// 256 104 -> 34.9; 512 of 112 x 112 to 512 243 -> 126.
 // ---------------------------------------------------------------------------
 typedef int conv_i4 __attribute__((ext_vector_type(4)));
 typedef uint32_t conv_u4 __attribute__((ext_vector_type(4)));
@@ -70,6 +69,7 @@ struct ConvArgs {
   const int32_t *ecol;    // [N], or [groups][N] with ecol_bstride = N
   int H, W, cg, kh, kw, ow, sh, sw, ph, pw, dh, dw;
   int P, K, kpad, N, groups, ecol_bstride;
+  uint32_t mkhw, mkw;     // floor(2^32 / d) + 1 of kh * kw and kw
   int cw;                 // channel waves of a workgroup: a power of two <= 16
   uint32_t flip;          // 0x80808080: unsigned input
   int32_t azp;            // input zero point
@@ -85,10 +85,11 @@ constexpr int kConvThreads = 1024;
 constexpr int kConvLds = 32768;  // bytes of A per chunk; the sums' tile later
 
 // A table entry: source offset, and the window position (ky * dh, kx * dw) in 16
-// bits each (saturated: past every image that is not WIDE) or, WIDE, 32.
+// bits each or, WIDE (images whose padded coordinates need more), 32.
 struct ConvTap {
   uint32_t off, pos;
 };
+typedef unsigned short conv_h2 __attribute__((ext_vector_type(2)));  // (x, y)
 struct ConvTapWide {
   uint32_t off, dy, dx;
 };
@@ -99,7 +100,7 @@ __global__ __launch_bounds__(kConvThreads) void k_conv(ConvArgs c, CHAN chan) {
   constexpr int TP = PT / 16;               // 16-position tiles
   constexpr int WQ = kConvThreads / PT;     // words per position and gather pass
   __shared__ conv_u4 sA[kConvLds / 16];
-  __shared__ std::conditional_t<WIDE, ConvTapWide, ConvTap> tab[KC];
+  __shared__ __align__(16) std::conditional_t<WIDE, ConvTapWide, ConvTap> tab[KC];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int cw = wave & (c.cw - 1), kw = wave / c.cw, nkw = 16 / c.cw;
@@ -133,7 +134,9 @@ __global__ __launch_bounds__(kConvThreads) void k_conv(ConvArgs c, CHAN chan) {
   const unsigned base = (unsigned)iy0 * (unsigned)c.W + (unsigned)ix0;
   const uint8_t *xg = c.x + (int64_t)blockIdx.z * c.cg * c.H * c.W;
   const int khw = c.kh * c.kw;
-  const uint32_t zb = (uint32_t)c.azp & 255u, fb = c.flip & 255u;
+  const uint32_t zb = (uint32_t)c.azp & 255u;
+  const conv_h2 pos0 = {(unsigned short)ix0, (unsigned short)iy0};
+  const conv_h2 last = {(unsigned short)(c.W - 1), (unsigned short)(c.H - 1)};
 
   conv_i4 acc[TP];
   int rsum[TP];
@@ -156,56 +159,73 @@ __global__ __launch_bounds__(kConvThreads) void k_conv(ConvArgs c, CHAN chan) {
     load_b(kw);
     for (int i = tid; i < kn; i += kConvThreads) {
       const int kk = k0 + i < c.K ? k0 + i : c.K - 1;
-      const int ci = kk / khw, r = kk - ci * khw;
-      const int ky = r / c.kw, kx = r - ky * c.kw;
+      // (kk < 2^16, so the multiplications give the quotients)
+      const int ci = khw == 1 ? kk : (int)__umulhi((uint32_t)kk, c.mkhw), r = kk - ci * khw;
+      const int ky = c.kw == 1 ? r : (int)__umulhi((uint32_t)r, c.mkw), kx = r - ky * c.kw;
       const unsigned dy = (unsigned)ky * (unsigned)c.dh, dx = (unsigned)kx * (unsigned)c.dw;
       const unsigned off = ((unsigned)ci * (unsigned)c.H + dy) * (unsigned)c.W + dx;
       if constexpr (WIDE)
         tab[i] = {off, dy, dx};
       else
-        tab[i] = {off, (dy < 65535u ? dy : 65535u) << 16 | (dx < 65535u ? dx : 65535u)};
+        tab[i] = {off, dy << 16 | (dx & 65535u)};
     }
     __syncthreads();  // the table, and every wave past the last chunk's products
-    // gather: words wq, wq + WQ, ... of the position's row (clamped: repeated)
+    // gather: words wq, wq + WQ, ... of the position's row (clamped: repeated).  No
+    // conditional around a load or in its use that the compiler could turn into a
+    // branch: as conditional expressions every byte was a basic block of its own
+    // and waited for its table entry alone (512 channels of 7 x 7, 3 x 3: 21.6 us
+    // instead of 16.3; of 112 x 112 264 instead of 126)
     auto gather = [&](auto count, int u0) __attribute__((always_inline)) {
       constexpr int NP = decltype(count)::value;
-      uint32_t w[NP];
+      uint32_t v[NP][4];
+      bool in[NP][4];
 #pragma unroll
       for (int u = 0; u < NP; u++) {
-        const int word = wq + WQ * (u0 + u) < words ? wq + WQ * (u0 + u) : words - 1;
-        uint32_t v[4];
+        const int word = min(wq + WQ * (u0 + u), words - 1);
+        ConvTap t4[4];
+        if constexpr (!WIDE) {
+          const conv_u4 *tp = (const conv_u4 *)&tab[4 * word];
+          const conv_u4 lo = tp[0], hi = tp[1];
+          t4[0] = {lo.x, lo.y}, t4[1] = {lo.z, lo.w}, t4[2] = {hi.x, hi.y}, t4[3] = {hi.z, hi.w};
+        }
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          const auto t = tab[4 * word + e];
-          unsigned dy, dx;
+          std::conditional_t<WIDE, ConvTapWide, ConvTap> t;
+          if constexpr (WIDE) t = tab[4 * word + e];
+          else t = t4[e];
           if constexpr (WIDE) {
-            dy = t.dy;
-            dx = t.dx;
+            in[u][e] = ((unsigned)iy0 + t.dy < (unsigned)c.H) & ((unsigned)ix0 + t.dx < (unsigned)c.W);
           } else {
-            dy = t.pos >> 16;
-            dx = t.pos & 65535u;
+            const conv_h2 at = pos0 + __builtin_bit_cast(conv_h2, t.pos);
+            in[u][e] = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(at, last)) ==
+                       __builtin_bit_cast(uint32_t, at);
           }
-          const bool in = (unsigned)iy0 + dy < (unsigned)c.H && (unsigned)ix0 + dx < (unsigned)c.W;
-          const uint32_t b = xg[in ? base + t.off : 0u];
-          v[e] = k0 + 4 * word + e < c.K ? (in ? b : zb) : fb;
+          v[u][e] = xg[(base + t.off) & (0u - (uint32_t)in[u][e])];
         }
-        w[u] = v[0] | v[1] << 8 | v[2] << 16 | v[3] << 24;
       }
 #pragma unroll
       for (int u = 0; u < NP; u++) {
-        const int word = wq + WQ * (u0 + u) < words ? wq + WQ * (u0 + u) : words - 1;
-        ((uint32_t *)sA)[row * (KC / 4) + (((word >> 2) ^ (row & 15)) << 2) + (word & 3)] = w[u];
+        const int word = min(wq + WQ * (u0 + u), words - 1);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const uint32_t m = 0u - (uint32_t)in[u][e];
+          v[u][e] = (v[u][e] & m) | (zb & ~m);
+        }
+        ((uint32_t *)sA)[row * (KC / 4) + (((word >> 2) ^ (row & 15)) << 2) + (word & 3)] =
+            v[u][0] | v[u][1] << 8 | v[u][2] << 16 | v[u][3] << 24;
       }
     };
     const int passes = (words + WQ - 1) / WQ;  // 1 .. 8
-    if (passes == 1)
+    if (passes == 1) {
       gather(std::integral_constant<int, 1>(), 0);
-    else if (passes <= 3)
-      gather(std::integral_constant<int, 3>(), 0);
-    else if (passes <= 5)
-      gather(std::integral_constant<int, 5>(), 0);
-    else
-      gather(std::integral_constant<int, 8>(), 0);
+    } else if (passes == 2) {
+      gather(std::integral_constant<int, 2>(), 0);
+    } else if (passes <= 4) {
+      gather(std::integral_constant<int, 4>(), 0);
+    } else {
+      gather(std::integral_constant<int, 4>(), 0);
+      gather(std::integral_constant<int, 4>(), 4);
+    }
     __syncthreads();
     for (int s = kw; s < nst; s += 4 * nkw) {
       conv_i4 b[4];
@@ -215,6 +235,16 @@ __global__ __launch_bounds__(kConvThreads) void k_conv(ConvArgs c, CHAN chan) {
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         if (s + u * nkw < nst) {
+          // row sums over k < K only (the weights past K are 0, A's bytes there are not)
+          int ones[4] = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+          const int k1 = k0 + (s + u * nkw) * 64;
+          if (k1 + 64 > c.K) {  // uniform
+#pragma unroll
+            for (int d = 0; d < 4; d++) {
+              const int left = min(max(c.K - k1 - 16 * q - 4 * d, 0), 4);
+              ones[d] = (int)(0x01010101ull >> (8 * (4 - left)));
+            }
+          }
 #pragma unroll
           for (int t = 0; t < TP; t++) {
             const int ra = t * 16 + r16;
@@ -223,7 +253,7 @@ __global__ __launch_bounds__(kConvThreads) void k_conv(ConvArgs c, CHAN chan) {
             const conv_i4 a = __builtin_bit_cast(conv_i4, x);
 #pragma unroll
             for (int d = 0; d < 4; d++)
-              rsum[t] = __builtin_amdgcn_sdot4(a[d], 0x01010101, rsum[t], false);
+              rsum[t] = __builtin_amdgcn_sdot4(a[d], ones[d], rsum[t], false);
             acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b[u], acc[t], 0, 0, 0);
           }
         }
@@ -409,9 +439,14 @@ int conv_run(mmnb_ctx *ctx, const mmnb_pack *p, const uint8_t *d_x, int x_signed
   c.mult = o.d_mult ? o.d_mult : (const double *)ctx->d_pad;
   c.bias = o.d_bias ? o.d_bias : (const int32_t *)ctx->d_pad;
   c.yzp = o.yzp; c.lo = o.lo; c.hi = o.hi;
-  // a window position saturated at 65535 lies past every image up to that size
-  // (with its padding)
-  const bool wide = s.h + s.ph > 65535 || s.w + s.pw > 65535;
+  auto magic = [](int64_t d) { return (uint32_t)((int64_t(1) << 32) / d + 1); };
+  c.mkhw = magic(p->conv_kh * p->conv_kw);
+  c.mkw = magic(p->conv_kw);
+  // 16-bit window positions: every input coordinate of a tap, from -pad to the
+  // last window's end, is told apart from those inside the image modulo 2^16
+  const int64_t ymax = (s.oh - 1) * s.sh - s.ph + (p->conv_kh - 1) * s.dh;
+  const int64_t xmax = (s.ow - 1) * s.sw - s.pw + (p->conv_kw - 1) * s.dw;
+  const bool wide = s.h + s.ph > 65536 || s.w + s.pw > 65536 || ymax > 65535 || xmax > 65535;
   const int64_t zmax = 65535 / g * g;  // whole images per launch
   for (int64_t z0 = 0; z0 < s.n * g; z0 += zmax) {
     const int64_t z = s.n * g - z0 < zmax ? s.n * g - z0 : zmax;

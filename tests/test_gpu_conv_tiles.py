@@ -49,3 +49,18 @@ def test_conv_of_an_image_beyond_16_bit_positions():
     want = Q.conv_integer(x, w, np.uint8(9), np.int8(3), [1, 1], [66000, 0, 66000, 0],
                           [66000, 1])
     np.testing.assert_array_equal(y, want)
+
+
+@pytest.mark.parametrize("pad", [36, 37])
+@pytest.mark.parametrize("side", [0, 1])
+def test_conv_at_the_limit_of_16_bit_positions(pad, side):
+    # taps from -pad to 65499 + pad: told apart modulo 2^16 up to a pad of 36
+    rng = np.random.default_rng(pad)
+    shape, kern, pads = [1, 1, 3, 3], [2, 1, 1, 1], [0] * 4
+    shape[2 + side], kern[2 + side], pads[side], pads[2 + side] = 65500, 3, pad, pad
+    x = rng.integers(0, 256, shape).astype(np.uint8)
+    w = rng.integers(-128, 128, kern).astype(np.int8)
+    y = ops.op_conv_integer(x, w, np.uint8(9), np.int8(3), ctx=_lib.default_context(),
+                            strides=[1, 1], pads=pads, dilations=[1, 1])
+    want = Q.conv_integer(x, w, np.uint8(9), np.int8(3), [1, 1], pads, [1, 1])
+    np.testing.assert_array_equal(y, want)
