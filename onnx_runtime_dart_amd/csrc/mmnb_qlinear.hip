@@ -94,13 +94,58 @@ struct ConvTapWide {
   uint32_t off, dy, dx;
 };
 
-template <int PT, typename CHAN, bool WIDE = false>
+// double, as the reference: (acc + bias) * mult, half to even, saturated
+__device__ __forceinline__ uint32_t conv_requant(uint32_t v, double mult, int32_t bias,
+                                                 const ConvArgs &c) {
+  const double f = rint(((double)(int32_t)v + (double)bias) * mult) + (double)c.yzp;
+  return (uint32_t)(uint8_t)(int32_t)fmin(fmax(f, (double)c.lo), (double)c.hi);
+}
+
+template <bool WIDE>
+using ConvTapOf = std::conditional_t<WIDE, ConvTapWide, ConvTap>;
+
+// An output position: its window's first input coordinates (y, x) and offset.
+struct ConvPos {
+  int iy0, ix0;
+  unsigned base;
+  __device__ ConvPos(const ConvArgs &c, int p) {
+    const int oy = p / c.ow, ox = p - oy * c.ow;
+    iy0 = oy * c.sh - c.ph;
+    ix0 = ox * c.sw - c.pw;
+    base = (unsigned)iy0 * (unsigned)c.W + (unsigned)ix0;
+  }
+  // whether the tap lies inside the image
+  template <typename TAP>
+  __device__ bool inside(const ConvArgs &c, const TAP &t) const {
+    if constexpr (std::is_same<TAP, ConvTapWide>::value) {
+      return ((unsigned)iy0 + t.dy < (unsigned)c.H) & ((unsigned)ix0 + t.dx < (unsigned)c.W);
+    } else {
+      const conv_h2 pos0 = {(unsigned short)ix0, (unsigned short)iy0};
+      const conv_h2 last = {(unsigned short)(c.W - 1), (unsigned short)(c.H - 1)};
+      const conv_h2 at = pos0 + __builtin_bit_cast(conv_h2, t.pos);
+      return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(at, last)) ==
+             __builtin_bit_cast(uint32_t, at);
+    }
+  }
+};
+template <bool WIDE>
+__host__ __device__ __forceinline__ ConvTapOf<WIDE> conv_tap(const ConvArgs &c, unsigned ci,
+                                                             unsigned ky, unsigned kx) {
+  const unsigned dy = ky * (unsigned)c.dh, dx = kx * (unsigned)c.dw;
+  const unsigned off = (ci * (unsigned)c.H + dy) * (unsigned)c.W + dx;
+  if constexpr (WIDE)
+    return {off, dy, dx};
+  else
+    return {off, dy << 16 | (dx & 65535u)};
+}
+
+template <int PT, typename CHAN, bool WIDE>
 __global__ __launch_bounds__(kConvThreads) void k_conv(ConvArgs c, CHAN chan) {
   constexpr int KC = kConvLds / PT;         // k per chunk
   constexpr int TP = PT / 16;               // 16-position tiles
   constexpr int WQ = kConvThreads / PT;     // words per position and gather pass
   __shared__ conv_u4 sA[kConvLds / 16];
-  __shared__ __align__(16) std::conditional_t<WIDE, ConvTapWide, ConvTap> tab[KC];
+  __shared__ __align__(16) ConvTapOf<WIDE> tab[KC];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int cw = wave & (c.cw - 1), kw = wave / c.cw, nkw = 16 / c.cw;
@@ -129,14 +174,10 @@ __global__ __launch_bounds__(kConvThreads) void k_conv(ConvArgs c, CHAN chan) {
   // this thread's position of the gather
   const int row = tid % PT, wq = tid / PT;
   const int pc = p0 + row < c.P ? p0 + row : c.P - 1;
-  const int oy = pc / c.ow, ox = pc - oy * c.ow;
-  const int iy0 = oy * c.sh - c.ph, ix0 = ox * c.sw - c.pw;
-  const unsigned base = (unsigned)iy0 * (unsigned)c.W + (unsigned)ix0;
+  const ConvPos at(c, pc);
   const uint8_t *xg = c.x + (int64_t)blockIdx.z * c.cg * c.H * c.W;
   const int khw = c.kh * c.kw;
   const uint32_t zb = (uint32_t)c.azp & 255u;
-  const conv_h2 pos0 = {(unsigned short)ix0, (unsigned short)iy0};
-  const conv_h2 last = {(unsigned short)(c.W - 1), (unsigned short)(c.H - 1)};
 
   conv_i4 acc[TP];
   int rsum[TP];
@@ -162,12 +203,7 @@ __global__ __launch_bounds__(kConvThreads) void k_conv(ConvArgs c, CHAN chan) {
       // (kk < 2^16, so the multiplications give the quotients)
       const int ci = khw == 1 ? kk : (int)__umulhi((uint32_t)kk, c.mkhw), r = kk - ci * khw;
       const int ky = c.kw == 1 ? r : (int)__umulhi((uint32_t)r, c.mkw), kx = r - ky * c.kw;
-      const unsigned dy = (unsigned)ky * (unsigned)c.dh, dx = (unsigned)kx * (unsigned)c.dw;
-      const unsigned off = ((unsigned)ci * (unsigned)c.H + dy) * (unsigned)c.W + dx;
-      if constexpr (WIDE)
-        tab[i] = {off, dy, dx};
-      else
-        tab[i] = {off, dy << 16 | (dx & 65535u)};
+      tab[i] = conv_tap<WIDE>(c, (unsigned)ci, (unsigned)ky, (unsigned)kx);
     }
     __syncthreads();  // the table, and every wave past the last chunk's products
     // gather: words wq, wq + WQ, ... of the position's row (clamped: repeated).  No
@@ -182,25 +218,19 @@ __global__ __launch_bounds__(kConvThreads) void k_conv(ConvArgs c, CHAN chan) {
 #pragma unroll
       for (int u = 0; u < NP; u++) {
         const int word = min(wq + WQ * (u0 + u), words - 1);
-        ConvTap t4[4];
-        if constexpr (!WIDE) {
+        ConvTapOf<WIDE> t4[4];
+        if constexpr (WIDE) {
+#pragma unroll
+          for (int e = 0; e < 4; e++) t4[e] = tab[4 * word + e];
+        } else {
           const conv_u4 *tp = (const conv_u4 *)&tab[4 * word];
           const conv_u4 lo = tp[0], hi = tp[1];
           t4[0] = {lo.x, lo.y}, t4[1] = {lo.z, lo.w}, t4[2] = {hi.x, hi.y}, t4[3] = {hi.z, hi.w};
         }
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          std::conditional_t<WIDE, ConvTapWide, ConvTap> t;
-          if constexpr (WIDE) t = tab[4 * word + e];
-          else t = t4[e];
-          if constexpr (WIDE) {
-            in[u][e] = ((unsigned)iy0 + t.dy < (unsigned)c.H) & ((unsigned)ix0 + t.dx < (unsigned)c.W);
-          } else {
-            const conv_h2 at = pos0 + __builtin_bit_cast(conv_h2, t.pos);
-            in[u][e] = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(at, last)) ==
-                       __builtin_bit_cast(uint32_t, at);
-          }
-          v[u][e] = xg[(base + t.off) & (0u - (uint32_t)in[u][e])];
+          in[u][e] = at.inside(c, t4[e]);
+          v[u][e] = xg[(at.base + t4[e].off) & (0u - (uint32_t)in[u][e])];
         }
       }
 #pragma unroll
@@ -306,29 +336,118 @@ __global__ __launch_bounds__(kConvThreads) void k_conv(ConvArgs c, CHAN chan) {
     uint32_t v[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) v[r] = (uint32_t)acc[t][r] + fix;
-    const int64_t at = ((int64_t)blockIdx.z * c.N + col) * c.P + p;
+    const int64_t o0 = ((int64_t)blockIdx.z * c.N + col) * c.P + p;
     if (c.y) {
       if (c.vec) {
-        *(conv_u4 *)(c.y + at) = (conv_u4){v[0], v[1], v[2], v[3]};
+        *(conv_u4 *)(c.y + o0) = (conv_u4){v[0], v[1], v[2], v[3]};
       } else {
 #pragma unroll
         for (int r = 0; r < 4; r++)
-          if (p + r < c.P) c.y[at + r] = (int32_t)v[r];
+          if (p + r < c.P) c.y[o0 + r] = (int32_t)v[r];
       }
     } else {
       uint32_t o[4];
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        // double, as the reference: (acc + bias) * mult, half to even, saturated
-        const double f = rint(((double)(int32_t)v[r] + (double)cb) * cm) + (double)c.yzp;
-        o[r] = (uint32_t)(uint8_t)(int32_t)fmin(fmax(f, (double)c.lo), (double)c.hi);
+        o[r] = conv_requant(v[r], cm, cb, c);
       }
       if (c.vec) {
-        *(uint32_t *)(c.yq + at) = o[0] | o[1] << 8 | o[2] << 16 | o[3] << 24;
+        *(uint32_t *)(c.yq + o0) = o[0] | o[1] << 8 | o[2] << 16 | o[3] << 24;
       } else {
 #pragma unroll
         for (int r = 0; r < 4; r++)
-          if (p + r < c.P) c.yq[at + r] = (uint8_t)o[r];
+          if (p + r < c.P) c.yq[o0 + r] = (uint8_t)o[r];
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Few taps (K <= 4 NW) and few output channels per group, depthwise above all: a
+// lane per output position.  It gathers its K bytes into NW registers and
+// multiplies them by each channel's weights, four at a time (v_dot4); taps (a table
+// in the arguments) and weights are the same for all lanes, so both are scalars.
+// No LDS and no barrier, and a wave goes over several blocks of 64 positions.
+//
+// k_conv pads such a product to 64 taps, 16 channels and 16 waves, and what it then
+// takes is the launch of its waves (300 000 for 384 channels of 56 x 56).  Bound
+// here by the gather's instructions, about 8 a byte; few positions, by the launch.
+//
+// ConvInteger, us per call by im2col and MatMulInteger launches, k_conv and here: 384
+// channels of 56 x 56, 3 x 3 depthwise 103, 342 and 9.2; four images of 960 of 28 x
+// 28, 5 x 5 depthwise 470, 941 and 33.7; 1 of 512 x 512, 3 x 3 to 8 27.7, 75.5 and
+// 6.0; 16 of 160000 samples, 3 taps, to 16 35.7, 139 and 15.8.
+// ---------------------------------------------------------------------------
+typedef __attribute__((address_space(4))) int conv_const_int;
+
+template <int NW, bool WIDE>
+struct ConvTaps {
+  ConvTapOf<WIDE> t[4 * NW];
+};
+
+template <int NW, bool WIDE, typename CHAN>
+__global__ __launch_bounds__(256) void k_conv_taps(ConvArgs c, ConvTaps<NW, WIDE> taps, CHAN chan,
+                                                   int nper) {
+  const int g = blockIdx.z % c.groups;
+  const int n0 = blockIdx.y * nper, n1 = min(n0 + nper, c.N);
+  const uint8_t *xg = c.x + (int64_t)blockIdx.z * c.cg * c.H * c.W;
+  const int8_t *bt = c.bt + (int64_t)g * c.N * c.kpad;
+  const uint32_t zb = (uint32_t)c.azp & 255u;
+  const uint32_t azc = (uint32_t)((c.flip ? 128 : 0) - c.azp);
+  for (unsigned p = blockIdx.x * blockDim.x + threadIdx.x; p < (unsigned)c.P;
+       p += gridDim.x * blockDim.x) {
+    const ConvPos at(c, (int)p);
+    int a[NW];
+    int rs = 0;  // sum over k < K
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      uint32_t v[4];
+      bool in[4];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const ConvTapOf<WIDE> t = taps.t[4 * w + e];
+        in[e] = at.inside(c, t);
+        v[e] = xg[(at.base + t.off) & (0u - (uint32_t)in[e])];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const uint32_t m = 0u - (uint32_t)in[e];
+        v[e] = (v[e] & m) | (zb & ~m);
+      }
+      a[w] = (int)((v[0] | v[1] << 8 | v[2] << 16 | v[3] << 24) ^ c.flip);
+      const int left = min(max(c.K - 4 * w, 0), 4);
+      rs = __builtin_amdgcn_sdot4(a[w], (int)(0x01010101ull >> (8 * (4 - left))), rs, false);
+    }
+    const int64_t o0 = ((int64_t)blockIdx.z * c.N + n0) * c.P + p;
+    // (scalar loads: left to itself the compiler reads them per lane, for the stores
+    // between them could alias)
+#pragma unroll NW > 8 ? 2 : 4
+    for (int n = n0; n < n1; n++) {
+      const conv_const_int *wp = (const conv_const_int *)(uintptr_t)(bt + (int64_t)n * c.kpad);
+      int acc = 0;
+#pragma unroll
+      for (int w = 0; w < NW; w++) acc = __builtin_amdgcn_sdot4(a[w], wp[w], acc, false);
+      const uint32_t ce =
+          (uint32_t)((const conv_const_int *)(uintptr_t)c.ecol)[g * c.ecol_bstride + n];
+      const uint32_t cs =
+          (uint32_t)((const conv_const_int *)(uintptr_t)c.colsum)[(int64_t)g * c.N + n];
+      // exact zero-point corrections, in wrapping 32 bits
+      const uint32_t v = (uint32_t)acc + ce * (uint32_t)rs + azc * cs + (uint32_t)c.K * azc * ce;
+      const int64_t o = o0 + (int64_t)(n - n0) * c.P;
+      if (c.y) {
+        c.y[o] = (int32_t)v;
+      } else {
+        const int ch = g * c.N + n;
+        double cm;
+        int32_t cb;
+        if constexpr (std::is_same<CHAN, ConvChan>::value) {
+          cm = chan.mult[ch];
+          cb = chan.bias[ch];
+        } else {
+          cm = c.mult[ch];
+          cb = c.bias[ch];
+        }
+        c.yq[o] = (uint8_t)conv_requant(v, cm, cb, c);
       }
     }
   }
@@ -405,7 +524,7 @@ struct ConvOut {
   const int32_t *d_bias = nullptr;
 };
 
-template <int PT, bool WIDE = false>
+template <int PT, bool WIDE>
 int conv_launch(mmnb_ctx *ctx, const ConvArgs &c, const ConvOut &o, int64_t z) {
   const dim3 grid((unsigned)((c.P + PT - 1) / PT), (unsigned)((c.N + 16 * c.cw - 1) / (16 * c.cw)),
                   (unsigned)z);
@@ -413,6 +532,67 @@ int conv_launch(mmnb_ctx *ctx, const ConvArgs &c, const ConvOut &o, int64_t z) {
   if (o.inl)
     return launch(ctx, kKernConv, k_conv<PT, ConvChan, WIDE>, grid, block, 0, c, o.chan);
   return launch(ctx, kKernConv, k_conv<PT, ConvNoChan, WIDE>, grid, block, 0, c, ConvNoChan{});
+}
+
+template <int NW, bool WIDE>
+int conv_taps_launch(mmnb_ctx *ctx, const ConvArgs &c, const ConvOut &o, int64_t z) {
+  const int64_t waves = (c.P + 63) / 64;  // of one (image, group)
+  // a wave per SIMD at least, with fewer channels each and the bytes gathered again;
+  // more than 8 per SIMD go over several blocks of positions
+  int nper = c.N;
+  while (nper > 4 && waves * z * ((c.N + nper - 1) / nper) < 4 * (int64_t)ctx->cu_count)
+    nper = (nper + 1) / 2;
+  const int64_t gy = (c.N + nper - 1) / nper;
+  const int64_t nw = waves < 4 ? waves : 4;
+  int64_t gx = (waves + nw - 1) / nw;
+  const int64_t most = 32 * (int64_t)ctx->cu_count / (nw * gy * z);
+  if (gx > most) gx = most > 1 ? most : 1;
+  ConvTaps<NW, WIDE> taps;
+  for (int i = 0; i < 4 * NW; i++) {
+    // (past the last tap: the last one again, times weights of 0)
+    const int k = i < c.K ? i : c.K - 1, r = k % (c.kh * c.kw);
+    taps.t[i] = conv_tap<WIDE>(c, (unsigned)(k / (c.kh * c.kw)), (unsigned)(r / c.kw),
+                               (unsigned)(r % c.kw));
+  }
+  const dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)z), block((unsigned)(64 * nw));
+  if (o.inl)
+    return launch(ctx, kKernConv, k_conv_taps<NW, WIDE, ConvChan>, grid, block, 0, c, taps,
+                  o.chan, nper);
+  return launch(ctx, kKernConv, k_conv_taps<NW, WIDE, ConvNoChan>, grid, block, 0, c, taps,
+                ConvNoChan{}, nper);
+}
+
+template <bool WIDE>
+int conv_dispatch(mmnb_ctx *ctx, ConvArgs &c, const ConvOut &o, int64_t z) {
+  const int64_t cus = ctx->cu_count, blocks = ((int64_t)c.P + 63) / 64 * z;
+  // Few taps: k_conv_taps for as many channels per group as it is the faster one (us
+  // here and in k_conv, ConvInteger; from two rounds of k_conv's workgroups on their
+  // launch counts):
+  //   K <= 12: 128 channels, 112 x 112 6.6 and 7.5; 256 channels 10.2 and 8.4;
+  //   K <= 28: 64 channels, 112 x 112 6.0 and 6.6, 128 channels 7.9 and 7.5, but 224 x
+  //     224 18.9 and 25.1, 256 channels 43.6 and 26.0;
+  //   K <= 64: 32 channels, 112 x 112 8.6 and 6.2, but 64 channels, 224 x 224 15.9 and
+  //     22.4, 128 channels as bytes 26.8 and 23.8.
+  const bool many = blocks > 2 * cus;
+  if (c.N <= (c.K <= 12 ? 128 : c.K <= 28 ? (many ? 128 : 64) : c.K <= 64 && many ? 64 : 0))
+    return c.K <= 12   ? conv_taps_launch<3, WIDE>(ctx, c, o, z)
+           : c.K <= 28 ? conv_taps_launch<7, WIDE>(ctx, c, o, z)
+                       : conv_taps_launch<16, WIDE>(ctx, c, o, z);
+  // the most positions per read of the weights that leave a workgroup on three
+  // quarters of the CUs; then, while half of them are idle, fewer channels per
+  // workgroup: the gather is repeated, but a workgroup reads less of the weights
+  // (256 channels of 14 x 14, 3 x 3 to 256: 13.3 us, with all 256 in one workgroup
+  // 25.8)
+  c.cw = 1;
+  while (c.cw < 16 && 16 * c.cw < c.N) c.cw *= 2;
+  auto groups = [&](int64_t pt) {
+    return ((int64_t)c.P + pt - 1) / pt * ((c.N + 16 * c.cw - 1) / (16 * c.cw)) * z;
+  };
+  const int64_t enough = 3 * cus / 4;
+  while (c.cw > 1 && groups(16) < cus / 2) c.cw /= 2;
+  if (groups(64) >= enough) return conv_launch<64, WIDE>(ctx, c, o, z);
+  if (groups(32) >= enough) return conv_launch<32, WIDE>(ctx, c, o, z);
+  return conv_launch<16, WIDE>(ctx, c, o, z);
 }
 
 // Device side of a convolution: all images and groups in one launch (grid.z,
@@ -455,28 +635,7 @@ int conv_run(mmnb_ctx *ctx, const mmnb_pack *p, const uint8_t *d_x, int x_signed
     c.yq = o.y ? nullptr : o.yq + z0 * n * P;
     const uintptr_t out = o.y ? (uintptr_t)c.y : (uintptr_t)c.yq;
     c.vec = P % 4 == 0 && out % (4 * esz) == 0;
-    // the most positions per read of the weights that leave a workgroup on three
-    // quarters of the CUs; then, while half of them are idle, fewer channels per
-    // workgroup: the gather is repeated, but a workgroup reads less of the weights
-    // (256 channels of 14 x 14, 3 x 3 to 256: 13.3 us, with all 256 in one workgroup
-    // 25.8)
-    const int64_t cus = ctx->cu_count;
-    c.cw = 1;
-    while (c.cw < 16 && 16 * c.cw < n) c.cw *= 2;
-    auto groups = [&](int64_t pt) {
-      return (P + pt - 1) / pt * ((n + 16 * c.cw - 1) / (16 * c.cw)) * z;
-    };
-    const int64_t enough = 3 * cus / 4;
-    while (c.cw > 1 && groups(16) < cus / 2) c.cw /= 2;
-    int rc;
-    if (wide)
-      rc = conv_launch<16, true>(ctx, c, o, z);
-    else if (groups(64) >= enough)
-      rc = conv_launch<64>(ctx, c, o, z);
-    else if (groups(32) >= enough)
-      rc = conv_launch<32>(ctx, c, o, z);
-    else
-      rc = conv_launch<16>(ctx, c, o, z);
+    const int rc = wide ? conv_dispatch<true>(ctx, c, o, z) : conv_dispatch<false>(ctx, c, o, z);
     if (rc) return rc;
   }
   return MMNB_OK;

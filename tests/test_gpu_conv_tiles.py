@@ -19,6 +19,13 @@ pytestmark = pytest.mark.gpu
     (2, 16, 100, 72, 1, 1, 1),      # 32 positions, 2 channel tiles
     (1, 8, 9, 300, 3, 1, 1),        # parameters by way of scratch
     (2, 24, 11, 48, 3, 2, 24),      # depthwise
+    (2, 130, 20, 260, 3, 1, 130),   # ... with parameters by way of scratch
+    (1, 12, 13, 128, 1, 1, 1),      # a lane per position: K = 12, 13, 28, channels split
+    (1, 13, 9, 3, 1, 1, 1),
+    (3, 28, 10, 64, 1, 1, 1),
+    (1, 29, 190, 9, 1, 1, 1),       # ... K = 29 and 64 with many positions
+    (1, 64, 182, 3, 1, 1, 1),
+    (1, 1, 740, 2, 1, 1, 1),        # ... several blocks of positions per wave
 ])
 def test_conv_tiles(n, c, hw, m, ks, stride, group):
     ctx = _lib.default_context()
@@ -63,4 +70,14 @@ def test_conv_at_the_limit_of_16_bit_positions(pad, side):
     y = ops.op_conv_integer(x, w, np.uint8(9), np.int8(3), ctx=_lib.default_context(),
                             strides=[1, 1], pads=pads, dilations=[1, 1])
     want = Q.conv_integer(x, w, np.uint8(9), np.int8(3), [1, 1], pads, [1, 1])
+    np.testing.assert_array_equal(y, want)
+
+
+def test_wide_image_of_many_taps():
+    rng = np.random.default_rng(5)
+    x = rng.integers(0, 256, (1, 65, 1, 70001)).astype(np.uint8)
+    w = rng.integers(-128, 128, (4, 65, 1, 3)).astype(np.int8)
+    y = ops.op_conv_integer(x, w, np.uint8(9), np.int8(3), ctx=_lib.default_context(),
+                            strides=[1, 1], pads=[0, 1, 0, 1], dilations=[1, 1])
+    want = Q.conv_integer(x, w, np.uint8(9), np.int8(3), [1, 1], [0, 1, 0, 1], [1, 1])
     np.testing.assert_array_equal(y, want)
