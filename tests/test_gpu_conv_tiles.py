@@ -18,6 +18,7 @@ pytestmark = pytest.mark.gpu
     (3, 57, 40, 130, 3, 1, 1),      # 32 positions, K = 513 (a chunk and one step), 4 channel tiles
     (2, 16, 100, 72, 1, 1, 1),      # 32 positions, 2 channel tiles
     (1, 8, 9, 300, 3, 1, 1),        # parameters by way of scratch
+    (1, 40, 5, 1100, 2, 1, 1),      # ... copied there
     (2, 24, 11, 48, 3, 2, 24),      # depthwise
     (2, 130, 20, 260, 3, 1, 130),   # ... with parameters by way of scratch
     (1, 12, 13, 128, 1, 1, 1),      # a lane per position: K = 12, 13, 28, channels split
