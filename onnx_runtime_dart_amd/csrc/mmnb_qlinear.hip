@@ -15,6 +15,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "mmnb_conv_plan.h"
 #include "mmnb_internal.h"
 
 using namespace mmnb;
@@ -69,6 +70,7 @@ struct ConvArgs {
   const int32_t *ecol;    // [N], or [groups][N] with ecol_bstride = N
   int H, W, cg, kh, kw, ow, sh, sw, ph, pw, dh, dw;
   int P, K, kpad, N, groups, ecol_bstride;
+  int p0;                 // first position of the launch (k_conv)
   uint32_t mkhw, mkw;     // floor(2^32 / d) + 1 of kh * kw and kw
   int cw;                 // channel waves of a workgroup: a power of two <= 16
   uint32_t flip;          // 0x80808080: unsigned input
@@ -80,9 +82,6 @@ struct ConvArgs {
   int32_t yzp, lo, hi;
   int vec;                // P % 4 == 0 and an aligned output
 };
-
-constexpr int kConvThreads = 1024;
-constexpr int kConvLds = 32768;  // bytes of A per chunk; the sums' tile later
 
 // A table entry: source offset, and the window position (ky * dh, kx * dw) in 16
 // bits each or, WIDE (images whose padded coordinates need more), 32.
@@ -144,14 +143,14 @@ __global__ __launch_bounds__(kConvThreads) void k_conv(ConvArgs c, CHAN chan) {
   constexpr int KC = kConvLds / PT;         // k per chunk
   constexpr int TP = PT / 16;               // 16-position tiles
   constexpr int WQ = kConvThreads / PT;     // words per position and gather pass
-  __shared__ conv_u4 sA[kConvLds / 16];
+  __shared__ conv_u4 sA[kConvLds / 16];  // the chunk; at the end the sums' tile
   __shared__ __align__(16) ConvTapOf<WIDE> tab[KC];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int cw = wave & (c.cw - 1), kw = wave / c.cw, nkw = 16 / c.cw;
   const int r16 = lane & 15, q = lane >> 4;
   const int g = blockIdx.z % c.groups;
-  const int p0 = blockIdx.x * PT;
+  const int p0 = c.p0 + (int)blockIdx.x * PT, left = c.P - p0;
 
   // this lane's output channel and its constants
   const int n = (blockIdx.y * c.cw + cw) * 16 + r16;
@@ -173,7 +172,7 @@ __global__ __launch_bounds__(kConvThreads) void k_conv(ConvArgs c, CHAN chan) {
 
   // this thread's position of the gather
   const int row = tid % PT, wq = tid / PT;
-  const int pc = p0 + row < c.P ? p0 + row : c.P - 1;
+  const int pc = row < left ? p0 + row : c.P - 1;
   const ConvPos at(c, pc);
   const uint8_t *xg = c.x + (int64_t)blockIdx.z * c.cg * c.H * c.W;
   const int khw = c.kh * c.kw;
@@ -271,8 +270,8 @@ __global__ __launch_bounds__(kConvThreads) void k_conv(ConvArgs c, CHAN chan) {
           if (k1 + 64 > c.K) {  // uniform
 #pragma unroll
             for (int d = 0; d < 4; d++) {
-              const int left = min(max(c.K - k1 - 16 * q - 4 * d, 0), 4);
-              ones[d] = (int)(0x01010101ull >> (8 * (4 - left)));
+              const int in4 = min(max(c.K - k1 - 16 * q - 4 * d, 0), 4);
+              ones[d] = (int)(0x01010101ull >> (8 * (4 - in4)));
             }
           }
 #pragma unroll
@@ -331,19 +330,19 @@ __global__ __launch_bounds__(kConvThreads) void k_conv(ConvArgs c, CHAN chan) {
   const uint32_t fix = azc * cs + (uint32_t)c.K * azc * ce;
 #pragma unroll
   for (int t = 0; t < TP; t++) {
-    const int p = p0 + t * 16 + q * 4;
-    if (p >= c.P) continue;
+    const int pt = t * 16 + q * 4;  // of the workgroup's positions
+    if (pt >= left) continue;
     uint32_t v[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) v[r] = (uint32_t)acc[t][r] + fix;
-    const int64_t o0 = ((int64_t)blockIdx.z * c.N + col) * c.P + p;
+    const int64_t o0 = ((int64_t)blockIdx.z * c.N + col) * c.P + p0 + pt;
     if (c.y) {
       if (c.vec) {
         *(conv_u4 *)(c.y + o0) = (conv_u4){v[0], v[1], v[2], v[3]};
       } else {
 #pragma unroll
         for (int r = 0; r < 4; r++)
-          if (p + r < c.P) c.y[o0 + r] = (int32_t)v[r];
+          if (pt + r < left) c.y[o0 + r] = (int32_t)v[r];
       }
     } else {
       uint32_t o[4];
@@ -356,7 +355,7 @@ __global__ __launch_bounds__(kConvThreads) void k_conv(ConvArgs c, CHAN chan) {
       } else {
 #pragma unroll
         for (int r = 0; r < 4; r++)
-          if (p + r < c.P) c.yq[o0 + r] = (uint8_t)o[r];
+          if (pt + r < left) c.yq[o0 + r] = (uint8_t)o[r];
       }
     }
   }
@@ -525,28 +524,24 @@ struct ConvOut {
 };
 
 template <int PT, bool WIDE>
-int conv_launch(mmnb_ctx *ctx, const ConvArgs &c, const ConvOut &o, int64_t z) {
-  const dim3 grid((unsigned)((c.P + PT - 1) / PT), (unsigned)((c.N + 16 * c.cw - 1) / (16 * c.cw)),
-                  (unsigned)z);
-  const dim3 block(kConvThreads);
-  if (o.inl)
-    return launch(ctx, kKernConv, k_conv<PT, ConvChan, WIDE>, grid, block, 0, c, o.chan);
-  return launch(ctx, kKernConv, k_conv<PT, ConvNoChan, WIDE>, grid, block, 0, c, ConvNoChan{});
+int conv_launch(mmnb_ctx *ctx, ConvArgs &c, const ConvOut &o, int64_t z, const ConvPlan &pl) {
+  for (int64_t p0 = 0; p0 < c.P; p0 += pl.step) {
+    c.p0 = (int)p0;
+    const int64_t np = c.P - p0 < pl.step ? c.P - p0 : pl.step;
+    const dim3 grid((unsigned)((np + PT - 1) / PT), (unsigned)pl.gy, (unsigned)z);
+    const dim3 block((unsigned)pl.threads);
+    const int rc =
+        o.inl ? launch(ctx, kKernConv, k_conv<PT, ConvChan, WIDE>, grid, block, 0, c, o.chan)
+              : launch(ctx, kKernConv, k_conv<PT, ConvNoChan, WIDE>, grid, block, 0, c,
+                       ConvNoChan{});
+    if (rc) return rc;
+  }
+  return MMNB_OK;
 }
 
 template <int NW, bool WIDE>
-int conv_taps_launch(mmnb_ctx *ctx, const ConvArgs &c, const ConvOut &o, int64_t z) {
-  const int64_t waves = (c.P + 63) / 64;  // of one (image, group)
-  // a wave per SIMD at least, with fewer channels each and the bytes gathered again;
-  // more than 8 per SIMD go over several blocks of positions
-  int nper = c.N;
-  while (nper > 4 && waves * z * ((c.N + nper - 1) / nper) < 4 * (int64_t)ctx->cu_count)
-    nper = (nper + 1) / 2;
-  const int64_t gy = (c.N + nper - 1) / nper;
-  const int64_t nw = waves < 4 ? waves : 4;
-  int64_t gx = (waves + nw - 1) / nw;
-  const int64_t most = 32 * (int64_t)ctx->cu_count / (nw * gy * z);
-  if (gx > most) gx = most > 1 ? most : 1;
+int conv_taps_launch(mmnb_ctx *ctx, const ConvArgs &c, const ConvOut &o, int64_t z,
+                     const ConvPlan &pl) {
   ConvTaps<NW, WIDE> taps;
   for (int i = 0; i < 4 * NW; i++) {
     // (past the last tap: the last one again, times weights of 0)
@@ -554,45 +549,25 @@ int conv_taps_launch(mmnb_ctx *ctx, const ConvArgs &c, const ConvOut &o, int64_t
     taps.t[i] = conv_tap<WIDE>(c, (unsigned)(k / (c.kh * c.kw)), (unsigned)(r / c.kw),
                                (unsigned)(r % c.kw));
   }
-  const dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)z), block((unsigned)(64 * nw));
+  const dim3 grid((unsigned)pl.gx, (unsigned)pl.gy, (unsigned)z), block((unsigned)pl.threads);
   if (o.inl)
     return launch(ctx, kKernConv, k_conv_taps<NW, WIDE, ConvChan>, grid, block, 0, c, taps,
-                  o.chan, nper);
+                  o.chan, (int)pl.nper);
   return launch(ctx, kKernConv, k_conv_taps<NW, WIDE, ConvNoChan>, grid, block, 0, c, taps,
-                ConvNoChan{}, nper);
+                ConvNoChan{}, (int)pl.nper);
 }
 
 template <bool WIDE>
 int conv_dispatch(mmnb_ctx *ctx, ConvArgs &c, const ConvOut &o, int64_t z) {
-  const int64_t cus = ctx->cu_count, blocks = ((int64_t)c.P + 63) / 64 * z;
-  // Few taps: k_conv_taps for as many channels per group as it is the faster one (us
-  // here and in k_conv, ConvInteger; from two rounds of k_conv's workgroups on their
-  // launch counts):
-  //   K <= 12: 128 channels, 112 x 112 6.6 and 7.5; 256 channels 10.2 and 8.4;
-  //   K <= 28: 64 channels, 112 x 112 6.0 and 6.6, 128 channels 7.9 and 7.5, but 224 x
-  //     224 18.9 and 25.1, 256 channels 43.6 and 26.0;
-  //   K <= 64: 32 channels, 112 x 112 8.6 and 6.2, but 64 channels, 224 x 224 15.9 and
-  //     22.4, 128 channels as bytes 26.8 and 23.8.
-  const bool many = blocks > 2 * cus;
-  if (c.N <= (c.K <= 12 ? 128 : c.K <= 28 ? (many ? 128 : 64) : c.K <= 64 && many ? 64 : 0))
-    return c.K <= 12   ? conv_taps_launch<3, WIDE>(ctx, c, o, z)
-           : c.K <= 28 ? conv_taps_launch<7, WIDE>(ctx, c, o, z)
-                       : conv_taps_launch<16, WIDE>(ctx, c, o, z);
-  // the most positions per read of the weights that leave a workgroup on three
-  // quarters of the CUs; then, while half of them are idle, fewer channels per
-  // workgroup: the gather is repeated, but a workgroup reads less of the weights
-  // (256 channels of 14 x 14, 3 x 3 to 256: 13.3 us, with all 256 in one workgroup
-  // 25.8)
-  c.cw = 1;
-  while (c.cw < 16 && 16 * c.cw < c.N) c.cw *= 2;
-  auto groups = [&](int64_t pt) {
-    return ((int64_t)c.P + pt - 1) / pt * ((c.N + 16 * c.cw - 1) / (16 * c.cw)) * z;
-  };
-  const int64_t enough = 3 * cus / 4;
-  while (c.cw > 1 && groups(16) < cus / 2) c.cw /= 2;
-  if (groups(64) >= enough) return conv_launch<64, WIDE>(ctx, c, o, z);
-  if (groups(32) >= enough) return conv_launch<32, WIDE>(ctx, c, o, z);
-  return conv_launch<16, WIDE>(ctx, c, o, z);
+  const ConvPlan pl = conv_plan(c.P, c.K, c.N, z, ctx->cu_count);
+  if (pl.taps)
+    return pl.nw == 3   ? conv_taps_launch<3, WIDE>(ctx, c, o, z, pl)
+           : pl.nw == 7 ? conv_taps_launch<7, WIDE>(ctx, c, o, z, pl)
+                        : conv_taps_launch<16, WIDE>(ctx, c, o, z, pl);
+  c.cw = pl.cw;
+  return pl.pt == 64   ? conv_launch<64, WIDE>(ctx, c, o, z, pl)
+         : pl.pt == 32 ? conv_launch<32, WIDE>(ctx, c, o, z, pl)
+                       : conv_launch<16, WIDE>(ctx, c, o, z, pl);
 }
 
 // Device side of a convolution: all images and groups in one launch (grid.z,

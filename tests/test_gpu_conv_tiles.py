@@ -1,11 +1,13 @@
-"""QLinearConv and ConvInteger at the edges of the convolution kernel's tiles, bit for bit
-against the oracle: position tiles (16 and 32), channel tiles (64 to 256), chunks of K,
-images of a launch, unaligned outputs, and more channels than travel in the arguments."""
+"""QLinearConv and ConvInteger at the edges of the convolution kernels' tiles, bit for bit
+against the oracle: position tiles (16, 32 and 64), channel tiles, chunks of K, images of a
+launch, unaligned outputs, more channels than travel in the arguments, and the kernel of a
+lane per position.  test_conv_plans asserts the tiles that its sizes stand for."""
 import numpy as np
 import pytest
 
 from oracle import qlinear as Q
 from onnx_runtime_dart_amd import _lib, ops
+from tests.conv_plan import plan
 
 pytestmark = pytest.mark.gpu
 
@@ -15,8 +17,8 @@ pytestmark = pytest.mark.gpu
     (1, 3, 7, 16, 5, 2, 1),         # P = 16, ragged K
     (2, 5, 17, 65, 3, 1, 1),        # P = 289: bytes stored one by one; a channel past a tile
     (1, 256, 7, 40, 3, 1, 1),       # K = 2304: several chunks
-    (3, 57, 40, 130, 3, 1, 1),      # 32 positions, K = 513 (a chunk and one step), 4 channel tiles
-    (2, 16, 100, 72, 1, 1, 1),      # 32 positions, 2 channel tiles
+    (3, 57, 40, 130, 3, 1, 1),      # all channels in one workgroup, ragged K of one chunk
+    (2, 16, 100, 72, 1, 1, 1),      # K = 16, 72 channels
     (1, 8, 9, 300, 3, 1, 1),        # parameters by way of scratch
     (1, 40, 5, 1100, 2, 1, 1),      # ... copied there
     (2, 24, 11, 48, 3, 2, 24),      # depthwise
@@ -29,6 +31,27 @@ pytestmark = pytest.mark.gpu
     (1, 1, 740, 2, 1, 1, 1),        # ... several blocks of positions per wave
 ])
 def test_conv_tiles(n, c, hw, m, ks, stride, group):
+    check(n, c, hw, m, ks, stride, group)
+
+
+@pytest.mark.parametrize("n,c,hw,m,ks,pt,cw,chunks,tiles", [
+    (1, 120, 90, 20, 3, 32, 2, 2, 1),
+    (1, 130, 91, 9, 3, 32, 1, 2, 1),     # an odd number of positions
+    (1, 15, 81, 33, 9, 32, 4, 2, 1),
+    (1, 257, 87, 100, 2, 32, 8, 2, 1),   # K = 1028
+    (1, 60, 130, 20, 3, 64, 2, 2, 1),
+    (1, 65, 113, 300, 3, 64, 16, 2, 2),  # no LDS reduction, two channel tiles
+    (5, 230, 20, 270, 3, 16, 16, 2, 2),
+])
+def test_conv_plans(n, c, hw, m, ks, pt, cw, chunks, tiles):
+    o, k = hw + 2 * (ks // 2) - ks + 1, c * ks * ks
+    p = plan(o * o, k, m, n, _lib.default_context().info()["compute_units"])
+    assert (p["taps"], p["pt"], p["cw"], p["gy"]) == (0, pt, cw, tiles)
+    assert -(-(-(-k // 64) * 64) // (32768 // pt)) == chunks
+    check(n, c, hw, m, ks, 1, 1)
+
+
+def check(n, c, hw, m, ks, stride, group):
     ctx = _lib.default_context()
     rng = np.random.default_rng(n + 3 * c + 5 * hw + 7 * m)
     x = rng.integers(0, 256, (n, c, hw, hw)).astype(np.uint8)
