@@ -313,8 +313,14 @@ bool nbits_block_native(int64_t bs);
 // counters of the context): whether a call should take it, with its column
 // waves cw and K slices nsl, and the launch.
 bool nbits_skinny_plan(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, int *cw, int *nsl);
+// wrap: rows of the weight from k / 2 on read A from column 0 again (8-bit planes).
 int launch_nbits_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
-                        int64_t m, float *d_y, int cw, int nsl);
+                        int64_t m, float *d_y, int cw, int nsl, bool wrap);
+// The planes of 8-bit weights times A read twice, without bias and correction, where
+// the few-row kernel takes the call: launches and returns true with the status in
+// *rc, or returns false.
+bool launch_nbits_planes(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
+                         int64_t m, float *d_y, int *rc);
 // MatMulNBits on a generic pack (no scratch; the reference's order and bits).
 int launch_nbits_generic(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
                          int64_t m, float *d_y);

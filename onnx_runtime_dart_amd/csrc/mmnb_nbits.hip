@@ -636,7 +636,7 @@ int launch_dec_gemv_attn(mmnb_ctx *ctx, const mmnb_pack *p, const DecAttnPartial
 }
 
 // ---------------------------------------------------------------------------
-// Decode-shape GEMV for 2 <= M <= 4 and small weights (gemv_multi_takes),
+// Decode-shape GEMV for 2 <= M <= 5 and small weights (gemv_multi_takes),
 // activations staged in LDS.
 //
 // Holding a chunk's 32 activations per row in registers (the M = 1 kernel)
@@ -698,12 +698,12 @@ template <int M, int R, int NBPC, bool HAS_ZP>
 __global__ __launch_bounds__(512) void k_gemv_lds(
     const float *__restrict__ A, int64_t lda, const uint8_t *__restrict__ W,
     int64_t col_bytes, const float *__restrict__ S, const uint8_t *__restrict__ Z, int nb,
-    int bs_log2, int K, int N, float *__restrict__ Y, int C, int kw, int iters, int groups,
-    int vec) {
+    int bs_log2, int K, int N, float *__restrict__ Y, const float *__restrict__ bias, int C,
+    int kw, int iters, int groups, int vec) {
   extern __shared__ float4 sact[];
   __shared__ float red[8][M][2 * R];
-  kernarg_fence(A, lda, W, col_bytes, S, Z, nb, bs_log2, K, N, Y, C, kw, iters, groups, vec,
-                blockDim.x, gridDim.x);
+  kernarg_fence(A, lda, W, col_bytes, S, Z, nb, bs_log2, K, N, Y, bias, C, kw, iters, groups,
+                vec, blockDim.x, gridDim.x);
   const int cs = 32 * kw * iters;  // staged chunk slots
   const int P = cs + 1;            // slot pitch (float4)
   const int nthr = blockDim.x;
@@ -838,7 +838,7 @@ __global__ __launch_bounds__(512) void k_gemv_lds(
       float v = 0.0f;
       for (int ww = 0; ww < kw; ww++) v += red[sg * kw + ww][m][cl];
       const int col = gi * (2 * R) + cl;
-      if (gi < groups && col < N) Y[(int64_t)m * N + col] = v;
+      if (gi < groups && col < N) Y[(int64_t)m * N + col] = bias ? v + bias[col] : v;
     }
     __syncthreads();
   }
@@ -859,7 +859,8 @@ static int launch_gemv_lds_mr(mmnb_ctx *ctx, int nbpc, dim3 grid, dim3 block, si
       if (e_ != hipSuccess) return check_hip(e_, "hipFuncSetAttribute");                     \
     }                                                                                        \
     return launch(ctx, kKernGemv, kern, grid, block, shmem, A, lda, p->d_w, p->col_bytes,   \
-                  p->d_scales, p->d_zp, nb, bs_log2, K, N, Y, C, kw, iters, groups, vec);   \
+                  p->d_scales, p->d_zp, nb, bs_log2, K, N, Y, p->direct_bias(), C, kw,      \
+                  iters, groups, vec);                                                       \
   }
   if (p->has_zp) {
     if (nbpc == 4) MMNB_GEMV_LDS_LAUNCH(4, true);
@@ -909,18 +910,40 @@ static bool gemv_multi_fits(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m) 
   return gemv_multi_lds(p, m, nullptr, nullptr) + 8 * 8 * 8 * 4 <= (size_t)ctx->lds_max;
 }
 
-// Whether a call of 2 <= M <= 4 rows takes the multi-row GEMV: its rows fit
-// LDS and the weight is small but K longer than two chunks of the matrix-core kernel
-// (us there and here: M = 2, (2048, 4096) 6.7 and 5.1, (4096, 4096) 8.5 and
-// 7.5; M = 4, (2048, 2048) 5.8 and 5.5; but M = 3, (1024, 4096) 4.5 and 4.6,
-// (3072, 8192) 9.5 and 11.4; M = 4, 4096^2 8.5 and 9.7).
+// Whether a call of 2 <= M <= 5 rows takes the multi-row GEMV instead of the few-row
+// matrix-core kernel (us there and here, block 128 if not said otherwise).  It wins
+// on small weights with K longer than two chunks of that kernel (M = 2, (2048, 4096) 6.7
+// and 5.1; M = 4, (2048, 2048) 5.8 and 5.5; M = 5, (2048, 4096) 6.8 and 6.3; but M = 3,
+// (3072, 8192) 9.5 and 11.4), and loses with every row more.  Larger weights:
+//   two rows, where K is a multiple of 4096, so that its waves' chunks come out even:
+//     K = 4096, N = 6144 10.2 and 7.7; K = 8192, N = 4096 10.7 and 9.1, N = 12288 22.9
+//     and 18.5, but N = 16384 23.2 and 23.1 (K = 5120, N = 5120 10.0 and 11.7); beyond,
+//     K = 16384, N = 4096 15.9 and 15.0, N = 8192 26.7 and 28.8 and, where the few-row
+//     kernel has one slice on up to three quarters of the CUs, N = 10240 43.7 and 41.9;
+//     other K where its workgroups are just one round, K = 5120, N = 4096 9.6 and 8.4,
+//     K = 11008 13.5 and 12.5, but in block 32 14.7 and 14.5;
+//   three and four rows, K = 4096, N = 8192 11.5 and 9.5, 11.6 and 11.0 (block 32 12.4
+//     and 11.0; N = 4096, four rows 9.0 and 8.6).
+// K = 1024: M = 2, N = 2048 4.2 and 4.0, block 16 4.8 and 4.3; M = 3, block 16 4.8 and
+// 4.5.
 static bool gemv_multi_takes(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m) {
-  return m >= 2 && m <= 4 && p->k64 > 1024 &&
-         p->n * p->col_bytes <= (int64_t)(m <= 3 ? 8 : 4) << 20 &&
-         gemv_multi_fits(ctx, p, m);
+  if (m < 2 || m > 5 || p->k64 < 1024 || !gemv_multi_fits(ctx, p, m)) return false;
+  const int64_t bytes = p->n * p->col_bytes, k = p->k64;
+  const int64_t mb = (bytes + (1 << 20) - 1) >> 20;
+  if (k <= 1024) return mb <= 2 && (m == 2 || (m == 3 && p->block == 16));
+  if (m == 5) return k <= 2048 && mb <= 4;
+  if (mb <= (m <= 3 ? 8 : 4)) return true;
+  if (m == 2 && k <= 11264 && p->n > 3072 && p->n <= 4096 && (p->block >= 64 || k <= 5120))
+    return true;
+  if (k % 4096 != 0) return false;
+  if (m >= 3) return k == 4096 && mb <= (m == 3 || p->block >= 64 ? 16 : 8);
+  const int64_t wgs = (p->n + 63) / 64;  // the few-row kernel's, in one slice
+  return k <= 8192 ? mb <= 48
+                   : (mb <= 32 && p->block >= 64) ||
+                         (2 * wgs > ctx->cu_count && 4 * wgs <= 3 * ctx->cu_count);
 }
 
-// 2 <= M <= 4 (gemv_multi_takes).
+// 2 <= M <= 5 (gemv_multi_takes).
 static int launch_gemv_multi(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a,
                              int64_t lda, int64_t m, float *d_y) {
   const int C = (int)(p->col_bytes / 16);
@@ -949,6 +972,7 @@ static int launch_gemv_multi(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a
     MMNB_CASE(2)
     MMNB_CASE(3)
     MMNB_CASE(4)
+    MMNB_CASE(5)
 #undef MMNB_CASE
     default:
       return fail(MMNB_ERR_ARG, "GEMV: M out of range");
@@ -1834,7 +1858,7 @@ static NbitsRoute nbits_route(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m
   if (p->generic) return kRouteGeneric;
   if (m == 1) return kRouteGemv;
   if (ctx->gemm_cb || ctx->gemm_ksplit || ctx->gemm_stages != 2) return kRouteGemm;
-  if (!p->ext && gemv_multi_takes(ctx, p, m)) return kRouteGemvMulti;
+  if (!p->wraps() && gemv_multi_takes(ctx, p, m)) return kRouteGemvMulti;
   return nbits_skinny_plan(ctx, p, m, cw, nsl) ? kRouteSkinny : kRouteGemm;
 }
 
@@ -1852,9 +1876,19 @@ static bool launch_no_scratch(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_
     case kRouteGeneric: *rc = launch_nbits_generic(ctx, p, d_a, lda, m, d_y); return true;
     case kRouteGemv: *rc = launch_gemv<false>(ctx, p, d_a, lda, d_y); return true;
     case kRouteGemvMulti: *rc = launch_gemv_multi(ctx, p, d_a, lda, m, d_y); return true;
-    case kRouteSkinny: *rc = launch_nbits_skinny(ctx, p, d_a, lda, m, d_y, cw, nsl); return true;
+    case kRouteSkinny:
+      *rc = launch_nbits_skinny(ctx, p, d_a, lda, m, d_y, cw, nsl, p->wraps());
+      return true;
     default: return false;
   }
+}
+
+bool launch_nbits_planes(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
+                         int64_t m, float *d_y, int *rc) {
+  int cw, nsl;
+  if (nbits_route(ctx, p, m, &cw, &nsl) != kRouteSkinny) return false;
+  *rc = launch_nbits_skinny(ctx, p, d_a, lda, m, d_y, cw, nsl, true);
+  return true;
 }
 
 // MatMulNBits with every scratch buffer carved from a caller's workspace

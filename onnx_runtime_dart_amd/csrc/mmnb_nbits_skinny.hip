@@ -502,7 +502,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
 
 template <int V, int CW, int KW>
 static int launch_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
-                         int64_t m, float *d_y, int nsl) {
+                         int64_t m, float *d_y, int nsl, bool wrap) {
   using R = SkRows<V>;
   const int64_t n = p->n;
   const int tiles = (int)((n + 32 * CW - 1) / (32 * CW));
@@ -510,22 +510,18 @@ static int launch_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, in
   // whole chunks per slice, no slice empty
   const int cps = (nchunks + nsl - 1) / nsl;
   nsl = (nchunks + cps - 1) / cps;
+  const int k = (int)(wrap ? p->k_in : p->k), kwrap = (int)(wrap ? p->k / 2 : INT32_MAX);
   const size_t red = (size_t)KW * R::kMax * 32 * CW * 4;
-  const size_t shmem = std::max<size_t>((size_t)R::kUnits * 1024, red);
+  const size_t shmem = std::max<size_t>((size_t)R::kUnits * 1024, red);  // 64 KB at most
   int bs_log2 = 0;
   while ((int64_t(1) << (bs_log2 + 1)) <= p->block) bs_log2++;
 #define MMNB_SKINNY(Q)                                                                        \
   {                                                                                           \
     auto kern = k_nbits_skinny<V, CW, KW, Q>;                                                 \
-    if (shmem > 65536) {                                                                      \
-      hipError_t e_ = hipFuncSetAttribute(                                                    \
-          (const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);        \
-      if (e_ != hipSuccess) return check_hip(e_, "hipFuncSetAttribute");                      \
-    }                                                                                         \
     return launch(ctx, kKernGemv, kern, dim3((unsigned)nsl, (unsigned)tiles, (unsigned)((m + R::kMax - 1) / R::kMax)), dim3(kSkThreads),      \
                   shmem, d_a, lda, (const uint8_t *)p->d_wt,                     \
                   (const float *)p->d_st, (int)p->ldsz, (int)p->n_blocks, bs_log2,            \
-                  (int)(p->k64 / kSegK), (int)p->k_read(), (int)p->k_wrap(), (int)m, (int)n,  \
+                  (int)(p->k64 / kSegK), k, kwrap, (int)m, (int)n,                             \
                   d_y, p->direct_bias(), nchunks, cps, nsl, tiles, ctx->d_sk_part,            \
                   ctx->d_gemm_cnt);                                                           \
   }
@@ -541,20 +537,24 @@ static int launch_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, in
 //     (1024, 4096): 5.4 against 7.3; M = 256, (1024, 2048), 512 and 256
 //     workgroups: 14.0 against 9.2);
 //   - three or four chunks: 64 columns with a slice per chunk when all of it
-//     is one round of the CUs (M = 2, (2048, 2048): 5.6 against 6.6), else as
-//     above;
+//     stays below one round of the CUs (M = 2, (2048, 2048): 5.6 against 6.6; M = 5,
+//     (1999, 4083), 256 workgroups: 7.8 against 7.2), else as above;
 //   - longer K: 64 columns and the slices that fill the CUs (M = 24, 4096^2:
 //     12.6 with 4 slices, 17.5 with 2, 19.3 with 8; 128-column workgroups 21
 //     and more, their registers spill).
-// Up to 16 rows it always beats the other kernels that take the call (M = 12,
-// (4096, 28672): 37.5 against 39.5); up to 32 rows while one round of the CUs
-// holds the columns (M = 20, N = 14336 26.7 against 29.2, but M = 17, N =
-// 28672 49.6 against 40.0); with more rows, i.e. several row groups, for at
-// most 4 chunks of one round (M = 64, 4096^2: 20.8 against 22.3; 28 with the 8
-// chunks of one slice) or one chunk of two (M = 2048, 512^2: 12.5 against
-// 20.8; four rounds, M = 100, (512, 14336): 19.6 against 13.2).  Blocks of 16
-// fill the registers of the two-pass layout: two chunks at most (M = 24,
-// 4096^2: 18.2 against 22.8; M = 64, four chunks: 30.2 against 23.6).
+// It takes all calls of up to 16 rows that the multi-row GEMV does not (M = 12, (4096,
+// 28672): 37.5 against the GEMM's 39.5; M = 16, (28672, 8192) 63 against 64).  Up to
+// 32 rows while one round of the CUs holds the columns (M = 20, N = 14336 26.7 against
+// 29.2, but M = 17, N = 28672 49.6 against 40.0) and a workgroup has at most 8 chunks
+// (M = 32, (4096, 14336) 26.2 against 25.4, (5120, 13824), 10 chunks, 32.0 against 28.8,
+// (16384, 16384), 32 chunks, 100 against 73) or, of four slices and more, whose columns
+// the GEMM's tiles leave CUs idle for, 14 ((28672, 4096) 48.7 against 48.0).  With more
+// rows, i.e. several row groups, for at most 4 chunks of one round (M = 64, 4096^2: 20.8
+// against 22.3; 28 with the 8 chunks of one slice) or one chunk, more than half filled,
+// of two (M = 2048, 512^2: 12.5 against 20.8; M = 256, N = 4096, K = 384 10.8 against
+// 11.3, K = 256 10.8 against 10.0; four rounds, M = 100, (512, 14336): 19.6 against
+// 13.2).  Blocks of 16 fill the registers of the two-pass layout: two chunks at most (M
+// = 24, 4096^2: 18.2 against 22.8; M = 64, four chunks: 30.2 against 23.6).
 bool nbits_skinny_plan(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, int *cw, int *nsl) {
   // 31-bit column offsets, 32-bit unit offsets, grid.y
   if (p->generic || m < 2 || p->n > ((int64_t)1 << 21) || p->k64 > ((int64_t)1 << 26))
@@ -562,26 +562,26 @@ bool nbits_skinny_plan(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, int *
   const int64_t cus = ctx->cu_count, chunks = (p->k + kSkChunk - 1) / kSkChunk;
   const int64_t rows = (m + kSkRows - 1) / kSkRows;
   const int64_t g1 = (p->n + 31) / 32 * rows, g2 = (p->n + 63) / 64 * rows;
-  *cw = chunks <= 4 && g1 <= cus && (chunks <= 2 || g2 * chunks > cus) ? 1 : 2;
+  *cw = chunks <= 4 && g1 <= cus && (chunks <= 2 || g2 * chunks >= cus) ? 1 : 2;
   *nsl = *cw == 1 || g2 > cus
              ? 1
              : (int)std::min<int64_t>({cus / g2, chunks, (int64_t)kSkMaxSlices});
   if (m <= 16) return true;
   const int64_t cps = (chunks + *nsl - 1) / *nsl;
-  if (g2 > cus) return g2 <= 2 * cus && cps == 1;
-  return cps <= (p->block == 16 ? 2 : m <= kSkRows ? chunks : 4);
+  if (g2 > cus) return g2 <= 2 * cus && cps == 1 && p->k > kSkChunk / 2;
+  return cps <= (p->block == 16 ? 2 : m > kSkRows ? 4 : *nsl >= 4 ? 14 : 8);
 }
 
 int launch_nbits_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
-                        int64_t m, float *d_y, int cw, int nsl) {
+                        int64_t m, float *d_y, int cw, int nsl, bool wrap) {
   if (cw == 1) {
-    if (m <= 8) return launch_skinny<0, 1, 8>(ctx, p, d_a, lda, m, d_y, nsl);
-    if (m <= 16) return launch_skinny<1, 1, 8>(ctx, p, d_a, lda, m, d_y, nsl);
-    return launch_skinny<2, 1, 8>(ctx, p, d_a, lda, m, d_y, nsl);
+    if (m <= 8) return launch_skinny<0, 1, 8>(ctx, p, d_a, lda, m, d_y, nsl, wrap);
+    if (m <= 16) return launch_skinny<1, 1, 8>(ctx, p, d_a, lda, m, d_y, nsl, wrap);
+    return launch_skinny<2, 1, 8>(ctx, p, d_a, lda, m, d_y, nsl, wrap);
   }
-  if (m <= 8) return launch_skinny<0, 2, 4>(ctx, p, d_a, lda, m, d_y, nsl);
-  if (m <= 16) return launch_skinny<1, 2, 4>(ctx, p, d_a, lda, m, d_y, nsl);
-  return launch_skinny<2, 2, 4>(ctx, p, d_a, lda, m, d_y, nsl);
+  if (m <= 8) return launch_skinny<0, 2, 4>(ctx, p, d_a, lda, m, d_y, nsl, wrap);
+  if (m <= 16) return launch_skinny<1, 2, 4>(ctx, p, d_a, lda, m, d_y, nsl, wrap);
+  return launch_skinny<2, 2, 4>(ctx, p, d_a, lda, m, d_y, nsl, wrap);
 }
 
 }  // namespace mmnb

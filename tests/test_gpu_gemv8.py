@@ -52,6 +52,10 @@ def _problem(m, k, n, bits, bs, zp, bias, seed):
     (70, 4160, 300, 8, 64, False, True),   # ... its K slices
     (5, 1000, 301, 4, 32, True, True),     # 4-bit weights with a bias, several rows
     (24, 4096, 100, 4, 128, False, True),
+    (2, 1024, 70, 4, 16, True, True),      # ... through the multi-row GEMV
+    (4, 2048, 77, 4, 32, True, True),
+    (5, 2000, 300, 4, 128, False, True),
+    (2, 1000, 90, 8, 32, True, True),      # 8-bit planes, gathered for it
     (130, 2048, 300, 4, 64, True, True),
     (1, 1000, 301, 4, 32, True, True),     # ... and one
     (1, 4160, 3, 4, 128, False, True),

@@ -40,6 +40,10 @@ CASES = [
     (54, 2001, 64, 128, False),
     (2, 5, 7, 16, True),
     (4, 3, 5, 16, False),          # fewer than four values
+    (5, 2000, 130, 32, True),      # the multi-row GEMV: five rows, and its longest rows
+    (2, 16384, 65, 64, False),
+    (18, 8192, 4100, 64, True),    # beyond a workgroup's chunks: the GEMM
+    (300, 256, 1030, 32, False),
 ]
 
 
