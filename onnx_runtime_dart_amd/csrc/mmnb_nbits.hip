@@ -1850,14 +1850,14 @@ int launch_matmul_nbits_prepared(mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, f
   return gemm_run(ctx, p, m, pl, d_ap, d_exp, d_y, d_part, ctx->d_gemm_cnt);
 }
 
-// Which kernel takes a call.  The GEMM's tuning overrides send every call of
-// several rows to it.
+// Which kernel takes a call.  The GEMM's tuning overrides send to it every call of more
+// than 8 rows (up to 8 rows the other kernels hold the activations in more bits).
 enum NbitsRoute { kRouteGeneric, kRouteGemv, kRouteGemvMulti, kRouteSkinny, kRouteGemm };
 static NbitsRoute nbits_route(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, int *cw,
                               int *nsl) {
   if (p->generic) return kRouteGeneric;
   if (m == 1) return kRouteGemv;
-  if (ctx->gemm_cb || ctx->gemm_ksplit || ctx->gemm_stages != 2) return kRouteGemm;
+  if (m > 8 && (ctx->gemm_cb || ctx->gemm_ksplit || ctx->gemm_stages != 2)) return kRouteGemm;
   if (!p->wraps() && gemv_multi_takes(ctx, p, m)) return kRouteGemvMulti;
   return nbits_skinny_plan(ctx, p, m, cw, nsl) ? kRouteSkinny : kRouteGemm;
 }

@@ -63,3 +63,19 @@ def test_forced_launch_shapes(forced_ctx, m, k, n, block, zp):
         np.testing.assert_array_equal(run(), y)
     finally:
         pack.free()
+
+
+@pytest.mark.parametrize("m,k,n", [(2, 1000, 96), (5, 4096, 300), (8, 700, 65)])
+def test_overrides_leave_few_rows_alone(forced_ctx, m, k, n):
+    # up to 8 rows do not take the GEMM whose launch shape is forced: the same bits
+    p = synth.mmnb_problem(m, k, n, 64, True, seed=m + k)
+    y = []
+    for ctx in (forced_ctx, _lib.default_context()):
+        pack = ops.pack_nbits(p.b_q, p.scales, p.zero_points, k=k, n=n, bits=4, block_size=64,
+                              ctx=ctx)
+        try:
+            y.append(np.empty((m, n), np.float32))
+            check(ctx.lib.mmnb_matmul_nbits(ctx.handle, pack.handle, ptr(p.a), m, ptr(y[-1])))
+        finally:
+            pack.free()
+    np.testing.assert_array_equal(*y)
