@@ -86,6 +86,8 @@ struct mmnb_ctx {
   float *d_sk_part = nullptr;
   // Tuning override of the GEMV columns-per-lane R (MMNB_GEMV_R; 0 = auto).
   int gemv_r = 0;
+  // Whether packs hold the few-row kernel's copy of the weights (MMNB_FEW_ROW_COPY).
+  int few_row_copy = 1;
   // Tuning override of the multi-row GEMV column groups per workgroup
   // (MMNB_GEMV_CG; 0 = auto).
   int gemv_cg = 0;
@@ -125,11 +127,11 @@ struct mmnb_pack {
   int64_t k64 = 0;        // k padded to a multiple of 64 (and >= n_blocks*block)
   int64_t col_bytes = 0;  // bytes per column in d_w (= k64 / 2)
   uint8_t *d_w = nullptr;
-  // the same weights for the matrix-core kernels, a second copy in their
-  // operand order: 1 KB units [ceil(n / 32)][k64 / 64], lane l of a unit
-  // holding the 16-byte half l / 32 of column l % 32's segment (zeros past
-  // column n).  In d_w, where a column is one run, a wave's operand load
-  // touches 64 lines for 16 bytes each.
+  // the same weights for the few-row kernel, a second copy behind d_w in its operand
+  // order (null: none, and calls of few rows take the other kernels): 1 KB units
+  // [ceil(n / 32)][k64 / 64], lane l of a unit holding the 16-byte half l / 32 of column
+  // l % 32's segment (zeros past column n).  In d_w, where a column is one run, a wave's
+  // operand load touches 64 lines for 16 bytes each; the GEMVs want the run.
   uint8_t *d_wt = nullptr;
   float *d_scales = nullptr;
   uint8_t *d_zp = nullptr;  // packed uint4; 0x88 filler when the op has none
@@ -312,6 +314,7 @@ bool nbits_block_native(int64_t bs);
 // MatMulNBits of a few rows in one launch (no scratch; K-slice partials and
 // counters of the context): whether a call should take it, with its column
 // waves cw and K slices nsl, and the launch.
+bool nbits_skinny_sizes(const mmnb_pack *p);  // whether its indices fit the weight
 bool nbits_skinny_plan(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, int *cw, int *nsl);
 // wrap: rows of the weight from k / 2 on read A from column 0 again (8-bit planes).
 int launch_nbits_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,

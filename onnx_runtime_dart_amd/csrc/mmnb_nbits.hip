@@ -1859,6 +1859,9 @@ static NbitsRoute nbits_route(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m
   if (m == 1) return kRouteGemv;
   if (m > 8 && (ctx->gemm_cb || ctx->gemm_ksplit || ctx->gemm_stages != 2)) return kRouteGemm;
   if (!p->wraps() && gemv_multi_takes(ctx, p, m)) return kRouteGemvMulti;
+  // without the few-row kernel's copy of the weights: four rows at a time
+  if (!p->d_wt && !p->wraps() && m <= 8 && gemv_multi_fits(ctx, p, std::min<int64_t>(m, 4)))
+    return kRouteGemvMulti;
   return nbits_skinny_plan(ctx, p, m, cw, nsl) ? kRouteSkinny : kRouteGemm;
 }
 
@@ -1875,7 +1878,17 @@ static bool launch_no_scratch(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_
   switch (nbits_route(ctx, p, m, &cw, &nsl)) {
     case kRouteGeneric: *rc = launch_nbits_generic(ctx, p, d_a, lda, m, d_y); return true;
     case kRouteGemv: *rc = launch_gemv<false>(ctx, p, d_a, lda, d_y); return true;
-    case kRouteGemvMulti: *rc = launch_gemv_multi(ctx, p, d_a, lda, m, d_y); return true;
+    case kRouteGemvMulti:
+      *rc = MMNB_OK;
+      for (int64_t r = 0, c; r < m && *rc == MMNB_OK; r += c) {
+        c = m <= 5 && gemv_multi_fits(ctx, p, m) ? m : std::min<int64_t>(m - r, 4);
+        const float *a = d_a + r * lda;
+        float *y = d_y + r * p->n;
+        *rc = c > 1              ? launch_gemv_multi(ctx, p, a, lda, c, y)
+              : p->direct_bias() ? launch_gemv<true>(ctx, p, a, lda, y)
+                                 : launch_gemv<false>(ctx, p, a, lda, y);
+      }
+      return true;
     case kRouteSkinny:
       *rc = launch_nbits_skinny(ctx, p, d_a, lda, m, d_y, cw, nsl, p->wraps());
       return true;

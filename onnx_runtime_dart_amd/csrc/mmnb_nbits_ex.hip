@@ -326,7 +326,13 @@ static int launch_gemv8(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int
 int run_matmul_nbits(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,
                      int64_t m, float *d_y) {
   if (!p->ext) return launch_matmul_nbits(ctx, p, d_a, lda, m, d_y);
-  if (m == 1 && p->bytes8) return launch_gemv8(ctx, p, d_a, lda, d_y);
+  // (several rows one by one where there is no few-row kernel)
+  if (p->bytes8 && (m == 1 || (m <= 8 && !p->d_wt))) {
+    int rc = MMNB_OK;
+    for (int64_t r = 0; r < m && rc == MMNB_OK; r++)
+      rc = launch_gemv8(ctx, p, d_a + r * lda, lda, d_y + r * p->n);
+    return rc;
+  }
   // without gather and correction the kernels take A and the bias themselves (us a
   // call with the passes and without, block 128: 8 bits, bias, M = 8, 4096^2 34.2 and
   // 12.0; M = 24 39.2 and 18.4; M = 512 120 and 78; M = 24, 1024^2 21.2 and 8.9; 4

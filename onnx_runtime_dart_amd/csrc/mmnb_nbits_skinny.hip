@@ -556,9 +556,7 @@ static int launch_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, in
 // 13.2).  Blocks of 16 fill the registers of the two-pass layout: two chunks at most (M
 // = 24, 4096^2: 18.2 against 22.8; M = 64, four chunks: 30.2 against 23.6).
 bool nbits_skinny_plan(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, int *cw, int *nsl) {
-  // 31-bit column offsets, 32-bit unit offsets, grid.y
-  if (p->generic || m < 2 || p->n > ((int64_t)1 << 21) || p->k64 > ((int64_t)1 << 26))
-    return false;
+  if (p->generic || m < 2 || !p->d_wt) return false;
   const int64_t cus = ctx->cu_count, chunks = (p->k + kSkChunk - 1) / kSkChunk;
   const int64_t rows = (m + kSkRows - 1) / kSkRows;
   const int64_t g1 = (p->n + 31) / 32 * rows, g2 = (p->n + 63) / 64 * rows;
@@ -570,6 +568,11 @@ bool nbits_skinny_plan(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, int *
   const int64_t cps = (chunks + *nsl - 1) / *nsl;
   if (g2 > cus) return g2 <= 2 * cus && cps == 1 && p->k > kSkChunk / 2;
   return cps <= (p->block == 16 ? 2 : m > kSkRows ? 4 : *nsl >= 4 ? 14 : 8);
+}
+
+bool nbits_skinny_sizes(const mmnb_pack *p) {
+  // 31-bit column offsets, 32-bit unit offsets, grid.y
+  return p->n <= ((int64_t)1 << 21) && p->k64 <= ((int64_t)1 << 26);
 }
 
 int launch_nbits_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_t lda,

@@ -125,6 +125,10 @@ int mmnb_init(int device, mmnb_ctx **out) {
     const int v = std::atoi(r);
     if (v >= 1 && v <= 8) ctx->gemv_cg = v;
   }
+  if (const char *r = std::getenv("MMNB_FEW_ROW_COPY")) {
+    const int v = std::atoi(r);
+    if (v == 0 || v == 1) ctx->few_row_copy = v;
+  }
   if (const char *r = std::getenv("MMNB_ATTN_MFMA")) {
     const int v = std::atoi(r);
     if (v == 0 || v == 1) ctx->attn_mfma = v;
@@ -236,8 +240,7 @@ int mmnb::pack_nbits_core(mmnb_ctx *ctx, const uint8_t *b_q, const float *scales
   p->k64 = (kp + kSegK - 1) / kSegK * kSegK;
   p->col_bytes = p->k64 / 2;
   auto cleanup = [&](int code) {
-    if (p->d_w) (void)hipFree(p->d_w);
-    if (p->d_wt) (void)hipFree(p->d_wt);
+    if (p->d_w) (void)hipFree(p->d_w);  // d_wt lies behind it
     if (p->d_scales) (void)hipFree(p->d_scales);
     if (p->d_zp) (void)hipFree(p->d_zp);
     if (p->d_st) (void)hipFree(p->d_st);  // d_zt lies inside it
@@ -245,9 +248,19 @@ int mmnb::pack_nbits_core(mmnb_ctx *ctx, const uint8_t *b_q, const float *scales
     return code;
   };
   const size_t wbytes = (size_t)(n * p->col_bytes);
-  if ((rc = device_alloc(wbytes, (void **)&p->d_w))) return cleanup(rc);
-  const size_t wtbytes = (size_t)((n + 31) / 32 * 32 * p->col_bytes);
-  if ((rc = device_alloc(wtbytes, (void **)&p->d_wt))) return cleanup(rc);
+  // with the few-row kernel's copy of the weights behind them, if its sizes allow the
+  // kernel and the memory is there
+  size_t wtbytes = (size_t)((n + 31) / 32 * 32 * p->col_bytes);
+  const size_t wtoff = (wbytes + kTailPad + 255) / 256 * 256;
+  if (ctx->few_row_copy && nbits_skinny_sizes(p) &&
+      hipMalloc((void **)&p->d_w, wtoff + wtbytes + kTailPad) == hipSuccess) {
+    p->d_wt = p->d_w + wtoff;
+  } else {
+    (void)hipGetLastError();  // of the attempt
+    p->d_w = nullptr;
+    wtbytes = 0;
+    if ((rc = device_alloc(wbytes, (void **)&p->d_w))) return cleanup(rc);
+  }
   if ((rc = device_alloc((size_t)(n * nb) * 4, (void **)&p->d_scales))) return cleanup(rc);
   p->has_zp = zero_points != nullptr || zp_fill != 0x88;
   if ((rc = device_alloc((size_t)zp_need, (void **)&p->d_zp))) return cleanup(rc);
@@ -629,8 +642,7 @@ int mmnb_pack_free(mmnb_pack *p) {
     CtxLock lk(ctx);
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
-    if (p->d_w) (void)hipFree(p->d_w);
-    if (p->d_wt) (void)hipFree(p->d_wt);
+    if (p->d_w) (void)hipFree(p->d_w);  // d_wt lies behind it
     if (p->d_scales) (void)hipFree(p->d_scales);
     if (p->d_zp) (void)hipFree(p->d_zp);
     if (p->d_st) (void)hipFree(p->d_st);  // d_zt lies inside it

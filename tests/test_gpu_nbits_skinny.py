@@ -7,10 +7,12 @@ Bar as in test_gpu_mmnb.py: normwise 1e-5 against the oracle and
 gamma_{K+2} sum|a||W| against the 64-bit product; reruns give the same bits.
 """
 import ctypes
+import os
 
 import numpy as np
 import pytest
 
+from oracle import nbits_ex as X
 from oracle import refcpu
 from onnx_runtime_dart_amd import _lib, ops, synth
 from onnx_runtime_dart_amd._lib import check
@@ -113,3 +115,61 @@ def test_magnitudes_of_any_range_in_a_row(m, k, n, block, zp, ratios):
     y64, absdot = refcpu.matmul_nbits_f64(p.a, p.b_q, p.scales, p.zero_points, k, n, block)
     gam = (k + 2) * U / (1 - (k + 2) * U)
     assert np.all(np.abs(y - y64) <= gam * absdot + 1e-30)
+
+
+@pytest.fixture(scope="module")
+def lean_ctx():
+    # packs without the few-row kernel's copy of the weights
+    saved = os.environ.get("MMNB_FEW_ROW_COPY")
+    os.environ["MMNB_FEW_ROW_COPY"] = "0"
+    try:
+        c = _lib.Context(0)
+    finally:
+        if saved is None:
+            os.environ.pop("MMNB_FEW_ROW_COPY", None)
+        else:
+            os.environ["MMNB_FEW_ROW_COPY"] = saved
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("m,k,n,bits,block,zp,bias", [
+    (2, 1000, 65, 4, 32, True, False),
+    (5, 9000, 40, 4, 64, False, False),    # five rows do not fit LDS
+    (8, 4096, 130, 4, 128, True, True),
+    (7, 512, 33, 4, 16, False, True),      # 4 + 3
+    (9, 2048, 70, 4, 32, True, False),     # the GEMM
+    (6, 1000, 50, 8, 32, False, True),
+    (3, 700, 41, 8, 64, True, True),
+    (20, 640, 64, 8, 32, False, False),
+])
+def test_packs_without_the_copy(lean_ctx, m, k, n, bits, block, zp, bias):
+    rng = np.random.default_rng(m + k)
+    nb = -(-k // block)
+    b = rng.integers(0, 256, (n, nb, block * bits // 8)).astype(np.uint8)
+    s = rng.uniform(0.002, 0.02, n * nb).astype(np.float32)
+    z = rng.integers(0, 256, n * nb if bits == 8 else (n * nb + 1) // 2).astype(np.uint8)
+    z = z if zp else None
+    bv = rng.standard_normal(n).astype(np.float32) if bias else None
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    y, size = [], []
+    for ctx in (lean_ctx, _lib.default_context()):
+        pack = ops.pack_nbits_ex(b, s, z, None, bv, k=k, n=n, bits=bits, block_size=block, ctx=ctx)
+        try:
+            y.append(np.empty((m, n), np.float32))
+            check(ctx.lib.mmnb_matmul_nbits(ctx.handle, pack.handle, _lib.ptr(a), m,
+                                            _lib.ptr(y[-1])))
+            size.append(pack.device_bytes)
+        finally:
+            pack.free()
+    assert size[1] - size[0] >= n * nb * block * bits // 8
+    y64, _ = X.matmul_nbits_ex_f64(a, b, s, z, None, bv, k, n, bits, block)
+    q = X.unpack_q(b, k, n, bits, block).astype(np.float64)
+    gi = np.arange(k) // block
+    # the bound of tests/test_gpu_nbits_ex.py (8 bits: planes of 16 hi and lo)
+    part = np.abs(q) + np.abs(X.zero_points_per_block(z, n, nb, bits)[:, gi])
+    part = (part + (272.0 if bits == 8 else 0.0)) * s.astype(np.float64).reshape(n, nb)[:, gi]
+    kk = (2 if bits == 8 else 1) * k + nb + 4
+    scale = np.abs(a.astype(np.float64)) @ part.T + (0 if bv is None else np.abs(bv.astype(float)))
+    for v in y:
+        assert np.all(np.abs(v - y64) <= kk * U / (1 - kk * U) * scale + 1e-30)
