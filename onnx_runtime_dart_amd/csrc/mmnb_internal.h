@@ -199,7 +199,7 @@ int check_hip(hipError_t e, const char *what);
 
 // Kernel ids reported by the timing mode (see mmnb_kernel_name).
 enum KernelId {
-  kKernGemv = 0,
+  kKernGemv = 0,         // MatMulNBits of one row
   kKernPrep = 1,
   kKernGemm = 2,
   kKernDqlMinmax = 3,
@@ -218,7 +218,10 @@ enum KernelId {
   kKernConv = 16,        // convolutions
   kKernNbitsEx = 17,     // extended MatMulNBits: A gather, block sums, correction
   kKernNbitsAny = 18,    // MatMulNBits of a block size the fast kernels do not take
-  kKernCount = 19
+  kKernSkinny = 19,      // MatMulNBits of a few rows on the matrix cores
+  kKernGemv8 = 20,       // ... of one row with 8-bit weights
+  kKernGemvMulti = 21,   // ... of two to five rows on the vector units
+  kKernCount = 22
 };
 
 // Launch `kern` on the context stream; in timing mode the dispatch records

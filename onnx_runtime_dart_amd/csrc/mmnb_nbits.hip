@@ -858,7 +858,8 @@ static int launch_gemv_lds_mr(mmnb_ctx *ctx, int nbpc, dim3 grid, dim3 block, si
                                           (int)shmem);                                       \
       if (e_ != hipSuccess) return check_hip(e_, "hipFuncSetAttribute");                     \
     }                                                                                        \
-    return launch(ctx, kKernGemv, kern, grid, block, shmem, A, lda, p->d_w, p->col_bytes,   \
+    return launch(ctx, kKernGemvMulti, kern, grid, block, shmem, A, lda, p->d_w,            \
+                  p->col_bytes,                                                              \
                   p->d_scales, p->d_zp, nb, bs_log2, K, N, Y, p->direct_bias(), C, kw,      \
                   iters, groups, vec);                                                       \
   }

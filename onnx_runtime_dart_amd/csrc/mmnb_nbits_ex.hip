@@ -300,7 +300,7 @@ static int launch_gemv8_r(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, b
   while ((int64_t(1) << bs_log2) < p->block) bs_log2++;
   const float *bias = p->d_bias ? p->d_bias : p->d_scales;
 #define MMNB_GEMV8(ZP, F)                                                                     \
-  return launch(ctx, kKernGemv, k_gemv8<R, NBPC, ZP, F>, grid, block, 0, d_a, p->d_w,         \
+  return launch(ctx, kKernGemv8, k_gemv8<R, NBPC, ZP, F>, grid, block, 0, d_a, p->d_w,         \
                 p->col_bytes, p->d_scales, p->d_z8, bias, (int)p->nb8, bs_log2,               \
                 (int)p->k_in, (int)n, d_y, C, iters, (int)p->n_blocks)
   if (p->d_z8) {

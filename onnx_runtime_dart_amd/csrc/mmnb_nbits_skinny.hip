@@ -515,11 +515,12 @@ static int launch_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, in
   const size_t shmem = std::max<size_t>((size_t)R::kUnits * 1024, red);  // 64 KB at most
   int bs_log2 = 0;
   while ((int64_t(1) << (bs_log2 + 1)) <= p->block) bs_log2++;
+  const dim3 grid((unsigned)nsl, (unsigned)tiles, (unsigned)((m + R::kMax - 1) / R::kMax));
 #define MMNB_SKINNY(Q)                                                                        \
   {                                                                                           \
     auto kern = k_nbits_skinny<V, CW, KW, Q>;                                                 \
-    return launch(ctx, kKernGemv, kern, dim3((unsigned)nsl, (unsigned)tiles, (unsigned)((m + R::kMax - 1) / R::kMax)), dim3(kSkThreads),      \
-                  shmem, d_a, lda, (const uint8_t *)p->d_wt,                     \
+    return launch(ctx, kKernSkinny, kern, grid, dim3(kSkThreads), shmem, d_a, lda,            \
+                  (const uint8_t *)p->d_wt,                                                   \
                   (const float *)p->d_st, (int)p->ldsz, (int)p->n_blocks, bs_log2,            \
                   (int)(p->k64 / kSegK), k, kwrap, (int)m, (int)n,                             \
                   d_y, p->direct_bias(), nchunks, cps, nsl, tiles, ctx->d_sk_part,            \
