@@ -50,6 +50,16 @@ def fixture_float_ok(have, want, tol=2e-5):
     return ok, max_abs, cos
 
 
+def kernels_of(ctx, call):
+    """Names of the library's kernels that call() launches."""
+    ctx.kernel_timing(True, max_launches=4096)
+    try:
+        call()
+        return set(ctx.kernel_timing_read())
+    finally:
+        ctx.kernel_timing(False)
+
+
 def normwise_rel_err(have, want):
     """max|have - want| / max|want| (the float parity metric of the path)."""
     w = np.asarray(want, dtype=np.float64)

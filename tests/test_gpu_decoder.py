@@ -32,7 +32,7 @@ from oracle import decoder as D
 from oracle import refcpu  # noqa: F401  (builds the oracle library)
 from onnx_runtime_dart_amd import _lib
 from onnx_runtime_dart_amd import decoder as G
-from tests.helpers import fixture_float_ok, load_golden, node_arg, normwise_rel_err
+from tests.helpers import fixture_float_ok, kernels_of, load_golden, node_arg, normwise_rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -373,8 +373,11 @@ def unfused_ctx():
     c.close()
 
 
-@pytest.mark.parametrize("cfg,prompt_len", [(SMALL, 20), (QWEN_HEADS, 48), (QWEN_HEADS, 70)],
-                         ids=["small", "qwen_heads", "qwen_heads_two_row_tiles"])
+# (20 rows take the few-row kernel, which reads fp32 rows, in both contexts)
+@pytest.mark.parametrize("cfg,prompt_len", [(SMALL, 20), (QWEN_HEADS, 48), (QWEN_HEADS, 70),
+                                            (SMALL, 40)],
+                         ids=["small", "qwen_heads", "qwen_heads_two_row_tiles",
+                              "small_two_row_tiles"])
 def test_prefill_fused_prep_bit_identical(ctx, unfused_ctx, cfg, prompt_len):
     # The norms and SwiGLU that write the GEMM's prepared activations compute
     # the same fp32 values as the separate kernels + k_prep_a: same logits,
@@ -392,6 +395,36 @@ def test_prefill_fused_prep_bit_identical(ctx, unfused_ctx, cfg, prompt_len):
     assert out[0][0] == out[1][0]
     np.testing.assert_array_equal(out[0][1], out[1][1])
     np.testing.assert_array_equal(out[0][2], out[1][2])
+
+
+@pytest.mark.parametrize("copy,prompt_len,gemm", [("1", 8, False), ("1", 20, False),
+                                                  ("1", 33, True), ("0", 20, True),
+                                                  ("0", 9, True)])
+def test_prompt_kernels(copy, prompt_len, gemm):
+    # Up to 32 rows take the few-row kernel (the GEMM with fused preparation from 9 rows on
+    # in packs without its copy of the weights), and the logits match the oracle either way.
+    saved = os.environ.get("MMNB_FEW_ROW_COPY")
+    os.environ["MMNB_FEW_ROW_COPY"] = copy
+    try:
+        c = _lib.Context(0)
+    finally:
+        if saved is None:
+            os.environ.pop("MMNB_FEW_ROW_COPY", None)
+        else:
+            os.environ["MMNB_FEW_ROW_COPY"] = saved
+    try:
+        prompt = np.random.default_rng(prompt_len).integers(0, SMALL.vocab, prompt_len)
+        w = G.random_weights(SMALL, seed=23)
+        dec = G.GpuDecoder(w, c)
+        try:
+            ks = kernels_of(c, lambda: dec.prefill(prompt))
+            assert ("k_gemm_mfma" in ks, "k_nbits_skinny" in ks) == (gemm, not gemm)
+            ref = oracle_model(w).forward(prompt)[-1]
+            assert normwise_rel_err(dec.logits(), ref) <= DEC_TOL
+        finally:
+            dec.free()
+    finally:
+        c.close()
 
 
 def prune_matrix(m, rng, dead_cols=0.125, keep=0.01):

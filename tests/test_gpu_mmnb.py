@@ -178,6 +178,9 @@ def test_edge_shapes(ctx, m, k, n, block, zp):
     (256, 2048, 1024, 128, True),  # decoder o projection shape: 4 slices
     (256, 1024, 4096, 128, True),  # decoder q|k|v shape: 2 slices
     (64, 2000, 100, 16, True),     # block 16, K not a multiple of 64
+    (64, 20480, 130, 128, False),  # beyond the few-row kernel, which takes those above
+    (40, 21000, 100, 64, True),
+    (130, 4096, 4096, 32, True),
 ])
 def test_gemm_k_slices(ctx, m, k, n, block, zp):
     # Few tiles: K is split across workgroups and the last slice of each tile

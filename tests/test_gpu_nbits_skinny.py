@@ -16,7 +16,7 @@ from oracle import nbits_ex as X
 from oracle import refcpu
 from onnx_runtime_dart_amd import _lib, ops, synth
 from onnx_runtime_dart_amd._lib import check
-from tests.helpers import normwise_rel_err
+from tests.helpers import kernels_of, normwise_rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -173,3 +173,28 @@ def test_packs_without_the_copy(lean_ctx, m, k, n, bits, block, zp, bias):
     scale = np.abs(a.astype(np.float64)) @ part.T + (0 if bv is None else np.abs(bv.astype(float)))
     for v in y:
         assert np.all(np.abs(v - y64) <= kk * U / (1 - kk * U) * scale + 1e-30)
+
+
+@pytest.mark.parametrize("m,k,n,bits,block,kernel", [
+    (1, 512, 64, 4, 32, "k_gemv_valu"), (1, 512, 64, 8, 32, "k_gemv8"),
+    (2, 2048, 256, 4, 32, "k_gemv_lds"), (5, 2048, 256, 4, 32, "k_gemv_lds"),
+    (2, 8192, 4096, 4, 128, "k_gemv_lds"), (6, 2048, 256, 4, 32, "k_nbits_skinny"),
+    (16, 4096, 4096, 4, 32, "k_nbits_skinny"), (32, 4096, 256, 4, 32, "k_nbits_skinny"),
+    (20, 4096, 256, 4, 16, "k_nbits_skinny"), (20, 8192, 4096, 4, 16, "k_gemm_mfma"),
+    (17, 8192, 16384, 4, 128, "k_gemm_mfma"), (64, 2048, 2048, 4, 32, "k_nbits_skinny"),
+    (256, 64, 4096, 4, 32, "k_gemm_mfma"), (100, 4096, 4096, 4, 32, "k_gemm_mfma"),
+])
+def test_kernel_of_a_call(m, k, n, bits, block, kernel):
+    ctx = _lib.default_context()
+    nb = -(-k // block)
+    pack = ops.pack_nbits_ex(np.full((n, nb, block * bits // 8), 0x77, np.uint8),
+                             np.ones(n * nb, np.float32), k=k, n=n, bits=bits, block_size=block,
+                             ctx=ctx)
+    da, dy = ctx.to_device(np.zeros((m, k), np.float32)), ctx.alloc(m * n * 4)
+    try:
+        assert kernel in kernels_of(ctx, lambda: check(ctx.lib.mmnb_matmul_nbits_dev(
+            ctx.handle, pack.handle, da.ptr, m, dy.ptr)))
+    finally:
+        da.free()
+        dy.free()
+        pack.free()

@@ -3,12 +3,13 @@ against mmnb_matmul_nbits_dev, through the C ABI: the same kernels on a
 fixed workspace instead of the context's grow-only scratch, so the results
 must be identical bit for bit.  Two calls in a row per case, the second with
 a smaller input (the workspace keeps the first call's contents), and the
-GEMV, the plain GEMM and the K-sliced GEMM (whose tile counters live in the
-workspace) all covered."""
+GEMVs, the few-row kernel, the plain GEMM and the K-sliced GEMM (whose tile
+counters live in the workspace) all covered."""
 import numpy as np
 import pytest
 
 from onnx_runtime_dart_amd import _lib, ops, synth
+from tests.helpers import kernels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -33,10 +34,11 @@ def _run(ctx, fn, pack, a):
 
 @pytest.mark.parametrize("k,n,block,zp,ms", [
     (4096, 4096, 32, True, (512, 130)),    # GEMM, then a smaller GEMM
-    (4096, 512, 32, True, (100, 40)),      # K-sliced GEMM (8 tiles), then fewer rows
-    (1024, 3072, 128, False, (64, 1)),     # GEMM, then the M = 1 GEMV
-    (3000, 700, 64, True, (8, 3)),         # multi-row GEMV, K not a multiple of 64
-    (8192, 40, 64, True, (8, 5)),          # rows too long for the GEMV's LDS: the GEMM
+    (4096, 512, 32, True, (100, 40)),      # few-row kernel with K slices and row groups
+    (1024, 3072, 128, False, (64, 1)),     # ... then the M = 1 GEMV
+    (3000, 700, 64, True, (8, 3)),         # ... then the multi-row GEMV, K % 64 != 0
+    (8192, 40, 64, True, (8, 5)),          # ... rows too long for the multi-row GEMV's LDS
+    (20480, 512, 32, True, (100, 40)),     # K-sliced GEMM, then fewer rows
 ])
 def test_noalloc_matches_dev_entry_point(ctx, k, n, block, zp, ms):
     p = synth.mmnb_problem(max(ms), k, n, block, zp, seed=k + n)
@@ -53,13 +55,20 @@ def test_noalloc_matches_dev_entry_point(ctx, k, n, block, zp, ms):
         pack.free()
 
 
-def test_noalloc_repeat_calls_identical(ctx):
+@pytest.mark.parametrize("m,k,n,kernel", [
+    (64, 3072, 1024, "k_nbits_skinny"),   # counters and partials of the context
+    (130, 4096, 4096, "k_gemm_mfma"),     # ... of the workspace
+    (64, 20480, 512, "k_gemm_mfma"),
+])
+def test_noalloc_repeat_calls_identical(ctx, m, k, n, kernel):
     # K slices: the counters the last slice resets must start the next call
     # at zero, so back-to-back calls give the same bits
-    p = synth.mmnb_problem(64, 3072, 1024, 128, False, seed=7)
-    pack = ops.pack_nbits(p.b_q, p.scales, None, k=3072, n=1024, bits=4, block_size=128, ctx=ctx)
+    p = synth.mmnb_problem(m, k, n, 128, False, seed=7)
+    pack = ops.pack_nbits(p.b_q, p.scales, None, k=k, n=n, bits=4, block_size=128, ctx=ctx)
     try:
         first = _run(ctx, ctx.lib.mmnb_matmul_nbits_dev_noalloc, pack, p.a)
+        assert kernel in kernels_of(ctx, lambda: _run(
+            ctx, ctx.lib.mmnb_matmul_nbits_dev_noalloc, pack, p.a))
         for _ in range(3):
             np.testing.assert_array_equal(
                 _run(ctx, ctx.lib.mmnb_matmul_nbits_dev_noalloc, pack, p.a), first)
@@ -99,15 +108,15 @@ def test_noalloc_rejects_oversized_and_extended(ctx):
 
 def test_noalloc_first_call_inside_graph_capture():
     # A fresh context (no scratch ever grown) whose FIRST MatMulNBits calls
-    # are made under HIP graph capture through the no-alloc entry point: a
-    # K-sliced GEMM (tile counters in the workspace, cleared by the prep
-    # kernel) and an M <= 8 call that falls back to the GEMM (rows too long
-    # for the multi-row GEMV's LDS; a GEMM of more than 64 KB of LDS, so a
+    # are made under HIP graph capture through the no-alloc entry point: few-row
+    # calls with K slices, and K-sliced GEMMs (tile counters in the workspace,
+    # cleared by the prep kernel; more than 64 KB of LDS, so a
     # hipFuncSetAttribute while capturing).  Nothing may allocate during capture; every replay,
     # with eager work and synchronisations in between, must give the bits of
     # mmnb_matmul_nbits_dev run outside capture.
     c = _lib.Context(0)
-    cases = [(100, 4096, 512, 32, True), (5, 8192, 40, 64, True)]
+    cases = [(100, 4096, 512, 32, True), (5, 8192, 40, 64, True), (130, 4096, 4096, 32, True),
+             (64, 20480, 512, 128, False)]
     packs, bufs = [], []
     try:
         for m, k, n, block, zp in cases:
@@ -128,6 +137,10 @@ def test_noalloc_first_call_inside_graph_capture():
             for pk, (m, n, da, dy) in zip(packs, bufs):
                 want.append(_run(c, c.lib.mmnb_matmul_nbits_dev, pk, da.numpy(np.float32,
                                                                               (m, pk.k))))
+                assert kernels_of(c, lambda: _run(
+                    c, c.lib.mmnb_matmul_nbits_dev, pk, da.numpy(np.float32, (m, pk.k)))) == (
+                        {"k_prep_a", "k_gemm_mfma"} if m == 130 or pk.k == 20480
+                        else {"k_nbits_skinny"})
             for rep in range(3):
                 for (m, n, da, dy) in bufs:
                     dy.upload(np.full((m, n), np.nan, np.float32))
@@ -136,8 +149,9 @@ def test_noalloc_first_call_inside_graph_capture():
                 for w, (m, n, da, dy) in zip(want, bufs):
                     np.testing.assert_array_equal(dy.numpy(np.float32, (m, n)), w, err_msg=str(rep))
                 # eager work between replays (the entry points outside the graph)
-                _run(c, c.lib.mmnb_matmul_nbits_dev_noalloc, packs[0],
-                     bufs[0][2].numpy(np.float32, (bufs[0][0], packs[0].k)))
+                for i in (0, 2):
+                    _run(c, c.lib.mmnb_matmul_nbits_dev_noalloc, packs[i],
+                         bufs[i][2].numpy(np.float32, (bufs[i][0], packs[i].k)))
         finally:
             c.graph_destroy(g)
     finally:
