@@ -165,6 +165,9 @@ struct mmnb_pack {
   bool bytes8 = false;
   int64_t nb8 = 0;
   uint8_t *d_z8 = nullptr;
+  // Whether the few-row kernel can take the pack: its copy of the weights is there, and
+  // a row has the four values that it loads at once.
+  bool few_rows() const { return d_wt && k_in >= 4; }
   // Whether the kernels take the operator's own A and bias (no gather, no correction
   // pass).  Rows past k_wrap() are then A's from column 0 again, and A has k_read()
   // columns.

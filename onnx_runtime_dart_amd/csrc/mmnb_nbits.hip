@@ -1860,8 +1860,8 @@ static NbitsRoute nbits_route(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m
   if (m == 1) return kRouteGemv;
   if (m > 8 && (ctx->gemm_cb || ctx->gemm_ksplit || ctx->gemm_stages != 2)) return kRouteGemm;
   if (!p->wraps() && gemv_multi_takes(ctx, p, m)) return kRouteGemvMulti;
-  // without the few-row kernel's copy of the weights: four rows at a time
-  if (!p->d_wt && !p->wraps() && m <= 8 && gemv_multi_fits(ctx, p, std::min<int64_t>(m, 4)))
+  // where the few-row kernel cannot: four rows at a time
+  if (!p->few_rows() && !p->wraps() && m <= 8 && gemv_multi_fits(ctx, p, std::min<int64_t>(m, 4)))
     return kRouteGemvMulti;
   return nbits_skinny_plan(ctx, p, m, cw, nsl) ? kRouteSkinny : kRouteGemm;
 }

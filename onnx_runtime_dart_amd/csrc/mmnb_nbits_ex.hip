@@ -327,7 +327,7 @@ int run_matmul_nbits(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, int64_
                      int64_t m, float *d_y) {
   if (!p->ext) return launch_matmul_nbits(ctx, p, d_a, lda, m, d_y);
   // (several rows one by one where there is no few-row kernel)
-  if (p->bytes8 && (m == 1 || (m <= 8 && !p->d_wt))) {
+  if (p->bytes8 && (m == 1 || (m <= 8 && !p->few_rows()))) {
     int rc = MMNB_OK;
     for (int64_t r = 0; r < m && rc == MMNB_OK; r++)
       rc = launch_gemv8(ctx, p, d_a + r * lda, lda, d_y + r * p->n);

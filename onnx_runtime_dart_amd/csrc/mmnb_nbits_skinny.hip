@@ -44,9 +44,9 @@
 // serial chain of staging, barrier, LDS reads and MFMAs of two waves per
 // SIMD, 1.4 (M <= 8) to 3.2 us (M <= 32) long; the slice exchange ~2.5 us.
 // us per call back to back, before (k_gemv_lds for M <= 8, else k_prep_a and
-// the GEMM) and now: M = 8, K = N = 4096 13.9 -> 9.0; N = 14336 48.4 -> 15.8;
-// (1024, 6144) 7.6 -> 5.0; M = 12, 4096^2 20.9 -> 10.0; M = 24 21.2 -> 12.6;
-// M = 32 and 256, 1024^2 13.2 -> 7.5 and 14.9 -> 7.8.
+// the GEMM) and now: M = 8, K = N = 4096 13.9 -> 8.8; N = 14336 48.4 -> 14.8;
+// (1024, 6144) 7.6 -> 5.0; M = 12, 4096^2 20.9 -> 9.8; M = 24 21.2 -> 12.6;
+// M = 32 and 256, 1024^2 13.2 -> 6.9 and 14.9 -> 7.8.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -90,8 +90,15 @@ __device__ __forceinline__ void sk_lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+__device__ __forceinline__ uint32_t sk_move(uint32_t v) {
+  uint32_t r;
+  asm volatile("v_mov_b32 %0, %1" : "=v"(r) : "v"(v));
+  return r;
+}
+
 typedef float f2vec __attribute__((ext_vector_type(2)));
 typedef float f4vec __attribute__((ext_vector_type(4)));
+typedef int i4vec __attribute__((ext_vector_type(4)));
 
 // max over the 64 lanes, wave-uniform.
 template <int CTRL>
@@ -200,28 +207,19 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
     // length and start.  Value by value where K % 8 or a row's alignment forbade the
     // aligned form, M = 54, (1999, 4083) took 36.3 us, M = 3, (859, 2142) 6.7; now
     // 15.2 and 4.7.)
-    if (K >= 4) {  // uniform
-      // four values that end past the row's end are read from its last four, and
-      // moved to their places in stage(), which also drops those past the end
-      const uint32_t off0 = 4u * (uint32_t)min(k0, K - 4);
-      const uint32_t off1 = 4u * (uint32_t)min(k0 + 4, K - 4);
+    // four values that end past the row's end are read from its last four, and
+    // moved to their places in trim(), which also drops those past the end (K >= 4)
+    const uint32_t off0 = 4u * (uint32_t)min(k0, K - 4);
+    const uint32_t off1 = 4u * (uint32_t)min(k0 + 4, K - 4);
 #pragma unroll
-      for (int i = 0; i < R::kPer; i++) {
-        const __amdgpu_buffer_rsrc_t rs = buf_rsrc(A + (int64_t)min(wid + 8 * i, M - 1) * lda);
-        const f4vec x0 =
-            __builtin_bit_cast(f4vec, __builtin_amdgcn_raw_buffer_load_b128(rs, off0, 0, 0));
-        const f4vec x1 =
-            __builtin_bit_cast(f4vec, __builtin_amdgcn_raw_buffer_load_b128(rs, off1, 0, 0));
-        av[i][0] = x0.x; av[i][1] = x0.y; av[i][2] = x0.z; av[i][3] = x0.w;
-        av[i][4] = x1.x; av[i][5] = x1.y; av[i][6] = x1.z; av[i][7] = x1.w;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < R::kPer; i++) {
-        const float *ar = A + (int64_t)min(wid + 8 * i, M - 1) * lda;
-#pragma unroll
-        for (int e = 0; e < 8; e++) av[i][e] = ar[min(k0 + e, K - 1)];
-      }
+    for (int i = 0; i < R::kPer; i++) {
+      const __amdgpu_buffer_rsrc_t rs = buf_rsrc(A + (int64_t)min(wid + 8 * i, M - 1) * lda);
+      const f4vec x0 =
+          __builtin_bit_cast(f4vec, __builtin_amdgcn_raw_buffer_load_b128(rs, off0, 0, 0));
+      const f4vec x1 =
+          __builtin_bit_cast(f4vec, __builtin_amdgcn_raw_buffer_load_b128(rs, off1, 0, 0));
+      av[i][0] = x0.x; av[i][1] = x0.y; av[i][2] = x0.z; av[i][3] = x0.w;
+      av[i][4] = x1.x; av[i][5] = x1.y; av[i][6] = x1.z; av[i][7] = x1.w;
     }
   };
   // A chunk's pieces to LDS: lane l holds k = 8l .. 8l + 7, i.e. half l & 1 of
@@ -234,7 +232,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
     if (c * kSkChunk + kSkChunk > K) {                // uniform
 #pragma unroll
       for (int i = 0; i < R::kPer; i++) {
-        if (K >= 4 && (K & 3)) {  // uniform: else no four values straddle the end
+        if (K & 3) {  // uniform: else no four values straddle the end
 #pragma unroll
           for (int q = 0; q < 8; q += 4) {  // values q .. q + 3 were read 4 - n further on
             const int n = left - q;
@@ -255,12 +253,15 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
 #pragma unroll
     for (int i = 0; i < R::kPer; i++) {
       const int row = wid + 8 * i;  // wave-uniform
-      // largest magnitude as an integer (NaN and infinities above every
-      // finite value), over the wave's 64 lanes
-      uint32_t mu = 0;
+      // largest and (layout 0) smallest magnitude, NaN from a NaN; then the largest of
+      // the wave's 64 lanes as an integer (NaN and infinities above every finite value)
+      float mxa = fabsf(av[i][0]), mna = mxa;
 #pragma unroll
-      for (int e = 0; e < 8; e++)
-        mu = max(mu, __builtin_bit_cast(uint32_t, av[i][e]) & 0x7FFFFFFFu);
+      for (int e = 1; e < 8; e++) {
+        mxa = __builtin_elementwise_maximum(mxa, fabsf(av[i][e]));
+        if constexpr (V == 0 && !REST) mna = __builtin_elementwise_minimum(mna, fabsf(av[i][e]));
+      }
+      uint32_t mu = __builtin_bit_cast(uint32_t, mxa);
       bool fin = true;
       mu = wave_max_u32(mu);
       if (mu >= 0x7F800000u) {  // uniform: scale by the largest finite magnitude
@@ -303,14 +304,14 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
       }
       if constexpr (V == 0 && !REST) {
         // whether the terms miss anything: a value other than 0 below the window
-        // (as integers without sign and less 1, in which 0 is the largest)
-        uint32_t mn = 0xFFFFFFFFu;
+        const float lim = ldexpf(1.0f, kSkWindow - ex);
+        // (lanes past the row's end hold zeros only)
+        if (fin && __builtin_amdgcn_ballot_w64((mna < lim) & (mxa > 0.0f)) != 0) {  // wave-uniform
+          bool miss = false;
 #pragma unroll
-        for (int e = 0; e < 8; e++)
-          mn = min(mn, (__builtin_bit_cast(uint32_t, av[i][e]) << 1) - 1u);
-        const uint32_t lim = __builtin_bit_cast(uint32_t, ldexpf(1.0f, kSkWindow - ex)) << 1;
-        if (__builtin_amdgcn_ballot_w64(mn < max(lim, 1u) - 1u) != 0 && lane == 0)
-          srest[wid] = row < M;
+          for (int e = 0; e < 8; e++) miss |= fabsf(av[i][e]) < lim && av[i][e] != 0.0f;
+          if (__builtin_amdgcn_ballot_w64(miss) != 0 && lane == 0) srest[wid] = row < M;
+        }
       }
       if (!STORE) continue;
       if (row < M) {  // wave-uniform
@@ -394,6 +395,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
   const std::true_type yes;
   const std::false_type no;
   if (V == 0 && lane == 0) srest[wid] = 0;
+  i4vec r0 = {}, r1 = {};
   Weights w0;
   load_a(c0);
   load_w(w0, c0);
@@ -404,21 +406,41 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
     // activations first: the next stage() waits for them alone.  (The weights are
     // moved, not alternated between two copies of the loop's code: M = 8, (4096,
     // 14336) 16.4 -> 14.6 us, (1024, 1024) 4.75 -> 4.6.)
-    const Weights wc = w0;
+    Weights wc;
+    // (explicit moves, before the loads: the compiler puts its own behind them, with a
+    // wait for them)
+    auto move_w = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < kWS; i++) {
+#pragma unroll
+        for (int d = 0; d < 4; d++) wc.w[i][d] = sk_move(w0.w[i][d]);
+#pragma unroll
+        for (int q = 0; q < NBPS; q++) {
+          wc.s[i][q] =
+              __builtin_bit_cast(float, sk_move(__builtin_bit_cast(uint32_t, w0.s[i][q])));
+          wc.z[i][q] = sk_move(w0.z[i][q]);
+        }
+      }
+    };
     if (c + 1 < c1) {  // uniform
       load_a(c + 1);
+      move_w();
       load_w(w0, c + 1);
+    } else {
+      move_w();
     }
     sk_lds_barrier();
+    if constexpr (V == 0) {  // (read here, needed after the last chunk)
+      r0 = *(const i4vec *)srest;
+      r1 = *(const i4vec *)(srest + 4);
+    }
     multiply(c, wc);
     sk_lds_barrier();  // every wave is done with the staged chunk
   }
   if constexpr (V == 0) {
     auto any_rest = [&]() __attribute__((always_inline)) {
-      int r = 0;
-#pragma unroll
-      for (int q = 0; q < 8; q++) r |= srest[q];
-      return __builtin_amdgcn_readfirstlane(r) != 0;  // of the workgroup
+      const i4vec r = r0 | r1;
+      return __builtin_amdgcn_readfirstlane((r.x | r.y) | (r.z | r.w)) != 0;  // of the workgroup
     };
     if (__builtin_expect(any_rest(), 0)) {
       for (int c = c0; c < c1; c++) {
@@ -433,6 +455,8 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
           sk_lds_barrier();  // every wave has read srest
           if (lane == 0) srest[wid] = nz;
           sk_lds_barrier();
+          r0 = *(const i4vec *)srest;
+          r1 = *(const i4vec *)(srest + 4);
           if (!any_rest()) break;
           stage(yes, yes);  // (zeros in the rows with nothing left)
           load_w(w0, c);
@@ -557,7 +581,7 @@ static int launch_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, in
 // 13.2).  Blocks of 16 fill the registers of the two-pass layout: two chunks at most (M
 // = 24, 4096^2: 18.2 against 22.8; M = 64, four chunks: 30.2 against 23.6).
 bool nbits_skinny_plan(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, int *cw, int *nsl) {
-  if (p->generic || m < 2 || !p->d_wt) return false;
+  if (p->generic || m < 2 || !p->few_rows()) return false;
   const int64_t cus = ctx->cu_count, chunks = (p->k + kSkChunk - 1) / kSkChunk;
   const int64_t rows = (m + kSkRows - 1) / kSkRows;
   const int64_t g1 = (p->n + 31) / 32 * rows, g2 = (p->n + 63) / 64 * rows;

@@ -56,6 +56,9 @@ def _problem(m, k, n, bits, bs, zp, bias, seed):
     (4, 2048, 77, 4, 32, True, True),
     (5, 2000, 300, 4, 128, False, True),
     (2, 1000, 90, 8, 32, True, True),      # 8-bit planes, gathered for it
+    (4, 3, 9, 8, 16, False, True),         # fewer than four values: row by row, the GEMM
+    (11, 2, 9, 8, 16, True, False),
+    (9, 3, 9, 4, 16, True, True),
     (130, 2048, 300, 4, 64, True, True),
     (1, 1000, 301, 4, 32, True, True),     # ... and one
     (1, 4160, 3, 4, 128, False, True),
