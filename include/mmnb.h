@@ -117,6 +117,8 @@ int mmnb_matmul_nbits_dev(mmnb_ctx *ctx, const mmnb_pack *pack,
  * counters) comes from a fixed device array of
  * mmnb_noalloc_workspace_bytes() bytes per GPU (64 MiB, held from library
  * load until the process ends) instead of the context's grow-only buffers.
+ * (Calls of few rows need none of it: their partials and counters are
+ * allocated with the context in either form.)
  * Calls whose scratch would exceed it return MMNB_ERR_UNSUPPORTED (M x K up
  * to 2048 x 4096 fits); packs from mmnb_pack_nbits_ex with g_idx, bias,
  * bits 8 or float zero points return MMNB_ERR_UNSUPPORTED.  All calls on one
@@ -245,7 +247,8 @@ int mmnb_dynamic_matmul_dev(mmnb_ctx *ctx, const mmnb_pack *pack,
                             float *d_y);
 
 /* ---- QLinearMatMul, ConvInteger, QLinearConv ----------------------------
- * The integer products run on the MatMulInteger kernels (exact int32);
+ * The integer products are exact (int32), QLinearMatMul's on the
+ * MatMulInteger kernels and the convolutions' on kernels of their own;
  * 8-bit outputs are int8 when *_is_signed, else uint8.  The reference
  * returns these as Tensor.int64 (the Dart binding widens). */
 
@@ -322,7 +325,7 @@ int mmnb_qlinear_conv(mmnb_ctx *ctx, const mmnb_pack *w, const void *x,
                       int y_is_signed, const int32_t *bias,
                       const mmnb_conv_params *prm, void *y);
 /* Device form: d_x / d_y device buffers; w_scale and bias stay host arrays
- * (uploaded per call, so this call is not capturable). */
+ * that every call reads anew, so this call is not capturable. */
 int mmnb_qlinear_conv_dev(mmnb_ctx *ctx, const mmnb_pack *w, const void *d_x,
                           int x_is_signed, int64_t n, int64_t c, int64_t h,
                           int64_t wd, int64_t x_zero_point, float x_scale,
@@ -461,7 +464,11 @@ int mmnb_decoder_free(mmnb_decoder *dec);
  * (OnnxModel.dispose / a NativeFinalizer on the Dart side). */
 int mmnb_pack_free(mmnb_pack *pack);
 
-/* Device bytes held by a pack. */
+/* Device bytes held by a pack.  A 4-bit MatMulNBits pack holds its weights
+ * twice where calls of 2 to 32 rows can use the second copy (one byte per
+ * weight in all, besides scales and zero points); MMNB_FEW_ROW_COPY=0 at
+ * mmnb_init leaves the copy out, and a pack that memory does not hold both
+ * of does without. */
 int64_t mmnb_pack_device_bytes(const mmnb_pack *pack);
 
 /* The operator shape a pack serves: k = A's last dimension (MatMulNBits,

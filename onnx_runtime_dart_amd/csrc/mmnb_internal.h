@@ -62,11 +62,11 @@ struct mmnb_ctx {
   int lds_max = 65536;
   // Device staging/scratch buffers, grown on demand and kept for reuse:
   //  0: activations in (fp32 / uint8), 1: outputs, 2: prepared activations
-  //  (fp16 hi/lo), 3: small reductions, 4: raw weights while packing,
-  //  5: small uploads (zero points), 6: unused, 7: block
-  //  sums / the convolution's input zero point, 8: QLinearConv per-channel
-  //  parameters, 9: gathered activations of an extended MatMulNBits pack,
-  //  10: the prefill GEMM's K-slice partial tiles.
+  //  (fp16 hi/lo), 3: their row exponents / small reductions, 4: raw weights while
+  //  packing, 5: small uploads (zero points), 6: unused, 7: block sums of an extended
+  //  MatMulNBits pack, 8: QLinearConv parameters of more channels than its arguments
+  //  hold, 9: gathered activations of an extended MatMulNBits pack, 10: the prefill
+  //  GEMM's K-slice partial tiles.
   mmnb::Scratch scratch[11];
   int live_packs = 0;
   // Kernel timing mode: launches go through hipExtLaunchKernelGGL with a
@@ -78,8 +78,9 @@ struct mmnb_ctx {
   // 4 KB device page: 1 KB of 0x00 and 1 KB of 0x80 (int8 padding), then a
   // 2 KB sink for the calibration kernels.
   void *d_pad = nullptr;
-  // Per-tile arrival counters of the prefill GEMM's K slices (kGemmMaxSplitTiles
-  // ints, zero at rest: the last slice of a tile resets its counter).
+  // Per-tile arrival counters of the K slices of the prefill GEMM and of the few-row
+  // kernel (kGemmMaxSplitTiles ints, zero at rest: the last slice of a tile resets its
+  // counter).
   int *d_gemm_cnt = nullptr;
   // K-slice partials of the few-row products (kSkMaxGroups tiles of kSkTile
   // floats, 8 MB), allocated with the context: those calls never grow scratch.
@@ -88,8 +89,8 @@ struct mmnb_ctx {
   int gemv_r = 0;
   // Whether packs hold the few-row kernel's copy of the weights (MMNB_FEW_ROW_COPY).
   int few_row_copy = 1;
-  // Tuning override of the multi-row GEMV column groups per workgroup
-  // (MMNB_GEMV_CG; 0 = auto).
+  // Tuning override of the column groups per workgroup of the multi-row GEMV
+  // (MMNB_GEMV_CG; 0 = auto; that kernel takes 2 to 5 rows).
   int gemv_cg = 0;
   // Prefill attention on the matrix cores (MMNB_ATTN_MFMA: 0 selects the
   // vector-ALU kernel; on by default).
@@ -101,7 +102,8 @@ struct mmnb_ctx {
   // (MMNB_DEC_ATTN_DEFER: 0 keeps the attention launch's own count and
   // merge; on by default where the merge fits).
   int dec_attn_defer = 1;
-  // Prefill GEMM LDS stages (2 or 3; MMNB_GEMM_STAGES tuning override).
+  // Prefill GEMM LDS stages (2 or 3; MMNB_GEMM_STAGES tuning override; like the next two
+  // it sends every call of more than 8 rows to the GEMM, and none of fewer).
   int gemm_stages = 2;
   // Prefill GEMM 128-column blocks per tile (MMNB_GEMM_CB: 1 or 2; 0 = auto).
   int gemm_cb = 0;

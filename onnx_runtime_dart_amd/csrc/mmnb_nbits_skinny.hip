@@ -98,7 +98,6 @@ __device__ __forceinline__ uint32_t sk_move(uint32_t v) {
 
 typedef float f2vec __attribute__((ext_vector_type(2)));
 typedef float f4vec __attribute__((ext_vector_type(4)));
-typedef int i4vec __attribute__((ext_vector_type(4)));
 
 // max over the 64 lanes, wave-uniform.
 template <int CTRL>
@@ -153,7 +152,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
   constexpr int kJB = 4 / NBPS;       // 16-k steps per quantisation block
   extern __shared__ u4vec sk_smem[];  // operand units, then (reused) the k waves' tiles
   __shared__ int sex[R::kMax];        // piece exponents of the staged chunk
-  __shared__ __align__(16) int srest[8];  // waves whose terms miss something (layout 0)
+  __shared__ int srest[8];            // waves whose terms miss something (layout 0)
   kernarg_fence(Aall, lda, Wt, ST, ldsz, nb, bs_log2, segs, K, kwrap, Mall, N, Yall, bias, nchunks,
                 cps, nsl, gy, part, tile_cnt);
   const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -261,6 +260,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
         mxa = __builtin_elementwise_maximum(mxa, fabsf(av[i][e]));
         if constexpr (V == 0 && !REST) mna = __builtin_elementwise_minimum(mna, fabsf(av[i][e]));
       }
+      if constexpr (V == 0 && !REST) asm volatile("" : "+v"(mna));  // here, not where it is used
       uint32_t mu = __builtin_bit_cast(uint32_t, mxa);
       bool fin = true;
       mu = wave_max_u32(mu);
@@ -284,10 +284,6 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
           const float up = 1 << kUp[p];
           x.x = fmaf((float)t[p - 1][e].x, -up, x.x * up);
           x.y = fmaf((float)t[p - 1][e].y, -up, x.y * up);
-          if (!fin) {  // the first term alone, so that the sums follow IEEE
-            x.x = x.x == x.x ? x.x : 0.0f;
-            x.y = x.y == x.y ? x.y : 0.0f;
-          }
           t[p][e] = __builtin_convertvector(x, half2_t);
         }
         if constexpr (REST) {
@@ -302,19 +298,19 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
           av[i][e + 4] = fin ? av[i][e + 4] : 0.0f;
         }
       }
-      if constexpr (V == 0 && !REST) {
-        // whether the terms miss anything: a value other than 0 below the window
-        const float lim = ldexpf(1.0f, kSkWindow - ex);
-        // (lanes past the row's end hold zeros only)
-        if (fin && __builtin_amdgcn_ballot_w64((mna < lim) & (mxa > 0.0f)) != 0) {  // wave-uniform
-          bool miss = false;
+      // of an infinity or NaN the first term alone, so that the sums follow IEEE (the
+      // others, formed with it, are NaN)
+      if (__builtin_expect(!fin, 0)) {  // uniform
+        asm volatile("");  // a branch, not two selects a term in every piece
 #pragma unroll
-          for (int e = 0; e < 8; e++) miss |= fabsf(av[i][e]) < lim && av[i][e] != 0.0f;
-          if (__builtin_amdgcn_ballot_w64(miss) != 0 && lane == 0) srest[wid] = row < M;
-        }
+        for (int p = 1; p < R::kParts; p++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            t[p][e].x = t[p][e].x == t[p][e].x ? t[p][e].x : (_Float16)0.0f;
+            t[p][e].y = t[p][e].y == t[p][e].y ? t[p][e].y : (_Float16)0.0f;
+          }
       }
-      if (!STORE) continue;
-      if (row < M) {  // wave-uniform
+      if (STORE && row < M) {  // wave-uniform
         if (lane == 0) sex[row] = ex;
 #pragma unroll
         for (int p = 0; p < R::kParts; p++) {
@@ -323,6 +319,18 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
           const int trow = V == 0 ? 8 * p + row : V == 1 ? 16 * p + row : row;
           const int unit = V == 2 ? u * 2 + p : u;
           sk_smem[unit * 64 + 32 * gg + (trow ^ u)] = __builtin_bit_cast(u4vec, h);
+        }
+      }
+      if constexpr (V == 0 && !REST) {
+        // whether the terms miss anything: a value other than 0 below the window (looked
+        // at while the stores are under way)
+        const float lim = ldexpf(1.0f, kSkWindow - ex);
+        // (lanes past the row's end hold zeros only)
+        if (fin && __builtin_amdgcn_ballot_w64((mna < lim) & (mxa > 0.0f)) != 0) {  // wave-uniform
+          bool miss = false;
+#pragma unroll
+          for (int e = 0; e < 8; e++) miss |= fabsf(av[i][e]) < lim && av[i][e] != 0.0f;
+          if (__builtin_amdgcn_ballot_w64(miss) != 0 && lane == 0) srest[wid] = row < M;
         }
       }
     }
@@ -395,7 +403,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
   const std::true_type yes;
   const std::false_type no;
   if (V == 0 && lane == 0) srest[wid] = 0;
-  i4vec r0 = {}, r1 = {};
+  int rest = 0;  // srest of wave lane % 8
   Weights w0;
   load_a(c0);
   load_w(w0, c0);
@@ -431,16 +439,14 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
     }
     sk_lds_barrier();
     if constexpr (V == 0) {  // (read here, needed after the last chunk)
-      r0 = *(const i4vec *)srest;
-      r1 = *(const i4vec *)(srest + 4);
+      rest = srest[lane & 7];
     }
     multiply(c, wc);
     sk_lds_barrier();  // every wave is done with the staged chunk
   }
   if constexpr (V == 0) {
-    auto any_rest = [&]() __attribute__((always_inline)) {
-      const i4vec r = r0 | r1;
-      return __builtin_amdgcn_readfirstlane((r.x | r.y) | (r.z | r.w)) != 0;  // of the workgroup
+    auto any_rest = [&]() __attribute__((always_inline)) {  // of the workgroup
+      return __builtin_amdgcn_ballot_w64(rest != 0) != 0;
     };
     if (__builtin_expect(any_rest(), 0)) {
       for (int c = c0; c < c1; c++) {
@@ -455,8 +461,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
           sk_lds_barrier();  // every wave has read srest
           if (lane == 0) srest[wid] = nz;
           sk_lds_barrier();
-          r0 = *(const i4vec *)srest;
-          r1 = *(const i4vec *)(srest + 4);
+          rest = srest[lane & 7];
           if (!any_rest()) break;
           stage(yes, yes);  // (zeros in the rows with nothing left)
           load_w(w0, c);

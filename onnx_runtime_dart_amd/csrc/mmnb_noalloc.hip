@@ -6,7 +6,9 @@
 // grow-only buffers, which call hipMalloc the first time a shape needs more.
 // mmnb_matmul_nbits_dev_noalloc runs the same kernels on a fixed workspace
 // instead: the file-scope device array `scratch` below, kNoAllocBytes per
-// GPU, held from module load until the process ends.
+// GPU, held from module load until the process ends.  (Calls of few rows need
+// neither: their partial tiles and counters are the context's own, allocated
+// with it, and two such calls on different contexts do not meet.)
 //
 // In host code `scratch` names a host-side stand-in, not device memory: its
 // device address comes from hipGetSymbolAddress, taken once per context at

@@ -1,11 +1,12 @@
-// QLinearMatMul, ConvInteger and QLinearConv on the MatMulInteger kernels.
+// QLinearMatMul, ConvInteger and QLinearConv.
 //
 // QLinearMatMul (onnx_qlinear_ops.dart:83-106) is MatMulInteger with an
-// 8-bit requantising epilogue.  A convolution (:157-308) is one launch
-// (k_conv) of the product A[p][kc] * w^T per image and group (p an output
-// position, kc = (c*kh + ky)*kw + kx, out-of-image taps set to the input zero
-// point so that (x - x_zp) = 0 there, which is the reference's skipping of
-// them): the weight w[m][c/g][kh][kw] is a MatMulInteger pack of B^T per
+// 8-bit requantising epilogue, on its kernels.  A convolution (:157-308) is the
+// product A[p][kc] * w^T per image and group (p an output position, kc =
+// (c*kh + ky)*kw + kx, out-of-image taps set to the input zero point so that
+// (x - x_zp) = 0 there, which is the reference's skipping of them), in one
+// launch of k_conv (matrix cores) or k_conv_taps (few channels), or a few
+// where the grid would pass its limits: the weight w[m][c/g][kh][kw] is a MatMulInteger pack of B^T per
 // group (batch = group), and the epilogue stores channel-major y[m][oy][ox],
 // requantising per output channel for QLinearConv.
 #include <cmath>
@@ -917,7 +918,7 @@ int mmnb_qlinear_conv_dev(mmnb_ctx *ctx, const mmnb_pack *w, const void *d_x, in
                           float y_scale, int64_t y_zero_point, int y_is_signed,
                           const int32_t *bias, const mmnb_conv_params *prm, void *d_y) {
   MMNB_GUARD_CTX(ctx);
-  if (ctx->capturing) return fail(MMNB_ERR_ARG, "QLinearConv uploads its parameters: not capturable");
+  if (ctx->capturing) return fail(MMNB_ERR_ARG, "QLinearConv reads host arrays at the call: not capturable");
   ConvShape s;
   int rc = conv_shape(w, n, c, h, wd, prm, &s);
   if (rc) return rc;
