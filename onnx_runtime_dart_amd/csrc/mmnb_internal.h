@@ -90,7 +90,7 @@ struct mmnb_ctx {
   // Whether packs hold the few-row kernel's copy of the weights (MMNB_FEW_ROW_COPY).
   int few_row_copy = 1;
   // Tuning override of the column groups per workgroup of the multi-row GEMV
-  // (MMNB_GEMV_CG; 0 = auto; that kernel takes 2 to 5 rows).
+  // (MMNB_GEMV_CG; 0 = auto; that kernel takes 2 to 4 rows).
   int gemv_cg = 0;
   // Prefill attention on the matrix cores (MMNB_ATTN_MFMA: 0 selects the
   // vector-ALU kernel; on by default).

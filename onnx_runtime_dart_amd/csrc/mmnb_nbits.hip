@@ -636,7 +636,7 @@ int launch_dec_gemv_attn(mmnb_ctx *ctx, const mmnb_pack *p, const DecAttnPartial
 }
 
 // ---------------------------------------------------------------------------
-// Decode-shape GEMV for 2 <= M <= 5 and small weights (gemv_multi_takes),
+// Decode-shape GEMV for 2 <= M <= 4 and small weights (gemv_multi_takes),
 // activations staged in LDS.
 //
 // Holding a chunk's 32 activations per row in registers (the M = 1 kernel)
@@ -911,40 +911,41 @@ static bool gemv_multi_fits(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m) 
   return gemv_multi_lds(p, m, nullptr, nullptr) + 8 * 8 * 8 * 4 <= (size_t)ctx->lds_max;
 }
 
-// Whether a call of 2 <= M <= 5 rows takes the multi-row GEMV instead of the few-row
+// Whether a call of 2 <= M <= 4 rows takes the multi-row GEMV instead of the few-row
 // matrix-core kernel (us there and here, block 128 if not said otherwise).  It wins
-// on small weights with K longer than two chunks of that kernel (M = 2, (2048, 4096) 6.7
-// and 5.1; M = 4, (2048, 2048) 5.8 and 5.5; M = 5, (2048, 4096) 6.8 and 6.3; but M = 3,
-// (3072, 8192) 9.5 and 11.4), and loses with every row more.  Larger weights:
+// on small weights with K longer than two chunks of that kernel (M = 2, (2048, 4096) 5.9
+// and 4.5; M = 3, 4096^2 8.2 and 6.9; M = 4, (2048, 2048) 5.9 and 5.0, but 4096^2 in block
+// 32 8.6 and 8.6), and loses with every row more (M = 5, (2048, 4096) 6.1 and 6.1, (2000,
+// 3000) 6.5 and 12.3).  Larger weights, up to the columns that the few-row kernel takes
+// in one slice on three quarters of the CUs (M = 2, K = 4096, N = 12288 12.8 and 11.4, N =
+// 14336 12.8 and 13.4):
 //   two rows, where K is a multiple of 4096, so that its waves' chunks come out even:
-//     K = 4096, N = 6144 10.2 and 7.7; K = 8192, N = 4096 10.7 and 9.1, N = 12288 22.9
-//     and 18.5, but N = 16384 23.2 and 23.1 (K = 5120, N = 5120 10.0 and 11.7); beyond,
-//     K = 16384, N = 4096 15.9 and 15.0, N = 8192 26.7 and 28.8 and, where the few-row
-//     kernel has one slice on up to three quarters of the CUs, N = 10240 43.7 and 41.9;
-//     other K where its workgroups are just one round, K = 5120, N = 4096 9.6 and 8.4,
-//     K = 11008 13.5 and 12.5, but in block 32 14.7 and 14.5;
-//   three and four rows, K = 4096, N = 8192 11.5 and 9.5, 11.6 and 11.0 (block 32 12.4
-//     and 11.0; N = 4096, four rows 9.0 and 8.6).
-// K = 1024: M = 2, N = 2048 4.2 and 4.0, block 16 4.8 and 4.3; M = 3, block 16 4.8 and
-// 4.5.
+//     K = 4096, N = 6144 10.3 and 7.7; K = 8192, N = 4096 10.6 and 9.1, N = 12288 23.2
+//     and 18.6 (K = 5120, N = 5120 10.0 and 11.7), in block 16 up to 4096 columns (N =
+//     4096 13.1 and 12.3, N = 5120 16.1 and 22.2); beyond, in long blocks, K = 16384, N =
+//     4096 16.0 and 14.8, N = 8192 26.7 and 28.8 and, where the few-row kernel has one
+//     slice on more than half of the CUs, N = 10240 44.7 and 41.8 (block 32 50.2 and 50.9);
+//     other K where its workgroups are just one round, K = 5120, N = 4096 9.5 and 8.2,
+//     K = 11008 13.4 and 12.3, but in block 32 14.7 and 14.5;
+//   three rows, K = 4096, where the few-row kernel has less than three slices: N = 8192
+//     11.2 and 9.4, N = 5120 8.7 and 9.1, and in block 16 N = 8192 13.5 and 16.9.
+// K = 1024: M = 2, N = 2048 4.0 and 4.0, block 16 4.7 and 4.3.
 static bool gemv_multi_takes(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m) {
-  if (m < 2 || m > 5 || p->k64 < 1024 || !gemv_multi_fits(ctx, p, m)) return false;
+  if (m < 2 || m > 4 || p->k64 < 1024 || !gemv_multi_fits(ctx, p, m)) return false;
   const int64_t bytes = p->n * p->col_bytes, k = p->k64;
   const int64_t mb = (bytes + (1 << 20) - 1) >> 20;
-  if (k <= 1024) return mb <= 2 && (m == 2 || (m == 3 && p->block == 16));
-  if (m == 5) return k <= 2048 && mb <= 4;
+  if (k <= 1024) return mb <= 2 && m == 2;
   if (mb <= (m <= 3 ? 8 : 4)) return true;
   if (m == 2 && k <= 11264 && p->n > 3072 && p->n <= 4096 && (p->block >= 64 || k <= 5120))
     return true;
-  if (k % 4096 != 0) return false;
-  if (m >= 3) return k == 4096 && mb <= (m == 3 || p->block >= 64 ? 16 : 8);
   const int64_t wgs = (p->n + 63) / 64;  // the few-row kernel's, in one slice
-  return k <= 8192 ? mb <= 48
-                   : (mb <= 32 && p->block >= 64) ||
-                         (2 * wgs > ctx->cu_count && 4 * wgs <= 3 * ctx->cu_count);
+  if (k % 4096 != 0 || 4 * wgs > 3 * ctx->cu_count || m == 4) return false;
+  if (m == 3) return k == 4096 && p->block >= 32 && 3 * wgs > ctx->cu_count && mb <= 16;
+  if (k <= 8192) return p->block >= 32 || p->n <= 4096;
+  return p->block >= 64 && (2 * wgs > ctx->cu_count || (p->n > 3072 && p->n <= 4096));
 }
 
-// 2 <= M <= 5 (gemv_multi_takes).
+// 2 <= M <= 4.
 static int launch_gemv_multi(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a,
                              int64_t lda, int64_t m, float *d_y) {
   const int C = (int)(p->col_bytes / 16);
@@ -973,7 +974,6 @@ static int launch_gemv_multi(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a
     MMNB_CASE(2)
     MMNB_CASE(3)
     MMNB_CASE(4)
-    MMNB_CASE(5)
 #undef MMNB_CASE
     default:
       return fail(MMNB_ERR_ARG, "GEMV: M out of range");
@@ -1882,7 +1882,7 @@ static bool launch_no_scratch(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_
     case kRouteGemvMulti:
       *rc = MMNB_OK;
       for (int64_t r = 0, c; r < m && *rc == MMNB_OK; r += c) {
-        c = m <= 5 && gemv_multi_fits(ctx, p, m) ? m : std::min<int64_t>(m - r, 4);
+        c = std::min<int64_t>(m - r, 4);
         const float *a = d_a + r * lda;
         float *y = d_y + r * p->n;
         *rc = c > 1              ? launch_gemv_multi(ctx, p, a, lda, c, y)

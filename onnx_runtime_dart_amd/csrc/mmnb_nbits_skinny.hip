@@ -575,16 +575,17 @@ static int launch_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, in
 // It takes all calls of up to 16 rows that the multi-row GEMV does not (M = 12, (4096,
 // 28672): 37.5 against the GEMM's 39.5; M = 16, (28672, 8192) 63 against 64).  Up to
 // 32 rows while one round of the CUs holds the columns (M = 20, N = 14336 26.7 against
-// 29.2, but M = 17, N = 28672 49.6 against 40.0) and a workgroup has at most 8 chunks
-// (M = 32, (4096, 14336) 26.2 against 25.4, (5120, 13824), 10 chunks, 32.0 against 28.8,
-// (16384, 16384), 32 chunks, 100 against 73) or, of four slices and more, whose columns
-// the GEMM's tiles leave CUs idle for, 14 ((28672, 4096) 48.7 against 48.0).  With more
-// rows, i.e. several row groups, for at most 4 chunks of one round (M = 64, 4096^2: 20.8
+// 29.2, but M = 17, N = 28672 49.6 against 40.0) and a workgroup has at most 8 chunks,
+// 10 where its columns fill three quarters of the CUs (M = 32, (4608, 13824) 26.8 against
+// 29.0, (5120, 13824) 29.4 against 30.4, but (5120, 10240) 28.8 against 27.3, (16384,
+// 16384), 32 chunks, 92 against 77), or, of four slices and more, whose columns the GEMM's
+// tiles leave CUs idle for, 14 ((28672, 4096), block 16 54 against 59).  With more rows, i.e. several row groups, for at most 4 chunks of one round (M = 64, 4096^2: 20.8
 // against 22.3; 28 with the 8 chunks of one slice) or one chunk, more than half filled,
 // of two (M = 2048, 512^2: 12.5 against 20.8; M = 256, N = 4096, K = 384 10.8 against
 // 11.3, K = 256 10.8 against 10.0; four rounds, M = 100, (512, 14336): 19.6 against
-// 13.2).  Blocks of 16 fill the registers of the two-pass layout: two chunks at most (M
-// = 24, 4096^2: 18.2 against 22.8; M = 64, four chunks: 30.2 against 23.6).
+// 13.2).  Blocks of 16 fill the registers of the two-pass layout: of more than 32 rows
+// two chunks at most (M = 64, four chunks: 30.2 against 23.6; but M = 32, (4096, 14336),
+// eight, 29.6 against 32.5).
 bool nbits_skinny_plan(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, int *cw, int *nsl) {
   if (p->generic || m < 2 || !p->few_rows()) return false;
   const int64_t cus = ctx->cu_count, chunks = (p->k + kSkChunk - 1) / kSkChunk;
@@ -597,7 +598,8 @@ bool nbits_skinny_plan(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, int *
   if (m <= 16) return true;
   const int64_t cps = (chunks + *nsl - 1) / *nsl;
   if (g2 > cus) return g2 <= 2 * cus && cps == 1 && p->k > kSkChunk / 2;
-  return cps <= (p->block == 16 ? 2 : m > kSkRows ? 4 : *nsl >= 4 ? 14 : 8);
+  if (m > kSkRows) return cps <= (p->block == 16 ? 2 : 4);
+  return cps <= (*nsl >= 4 ? 14 : 4 * g2 > 3 * cus ? 10 : 8);
 }
 
 bool nbits_skinny_sizes(const mmnb_pack *p) {

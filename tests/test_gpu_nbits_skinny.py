@@ -42,9 +42,11 @@ CASES = [
     (54, 2001, 64, 128, False),
     (2, 5, 7, 16, True),
     (4, 3, 5, 16, False),          # fewer than four values
-    (5, 2000, 130, 32, True),      # the multi-row GEMV: five rows, and its longest rows
+    (5, 2000, 130, 32, True),
+    (4, 2000, 130, 32, True),      # the multi-row GEMV: four rows, and its longest rows
     (2, 16384, 65, 64, False),
-    (18, 8192, 4100, 64, True),    # beyond a workgroup's chunks: the GEMM
+    (18, 8192, 4100, 64, True),    # six chunks a slice
+    (18, 4700, 8260, 64, True),    # beyond a workgroup's chunks: the GEMM
     (300, 256, 1030, 32, False),
 ]
 
@@ -177,10 +179,12 @@ def test_packs_without_the_copy(lean_ctx, m, k, n, bits, block, zp, bias):
 
 @pytest.mark.parametrize("m,k,n,bits,block,kernel", [
     (1, 512, 64, 4, 32, "k_gemv_valu"), (1, 512, 64, 8, 32, "k_gemv8"),
-    (2, 2048, 256, 4, 32, "k_gemv_lds"), (5, 2048, 256, 4, 32, "k_gemv_lds"),
-    (2, 8192, 4096, 4, 128, "k_gemv_lds"), (6, 2048, 256, 4, 32, "k_nbits_skinny"),
+    (2, 2048, 256, 4, 32, "k_gemv_lds"), (4, 2048, 256, 4, 32, "k_gemv_lds"),
+    (2, 8192, 4096, 4, 128, "k_gemv_lds"), (5, 2048, 256, 4, 32, "k_nbits_skinny"),
+    (3, 4096, 8192, 4, 16, "k_nbits_skinny"), (2, 4096, 14336, 4, 32, "k_nbits_skinny"),
     (16, 4096, 4096, 4, 32, "k_nbits_skinny"), (32, 4096, 256, 4, 32, "k_nbits_skinny"),
-    (20, 4096, 256, 4, 16, "k_nbits_skinny"), (20, 8192, 4096, 4, 16, "k_gemm_mfma"),
+    (20, 4096, 256, 4, 16, "k_nbits_skinny"), (20, 8192, 4096, 4, 16, "k_nbits_skinny"),
+    (20, 8192, 8320, 4, 16, "k_gemm_mfma"),
     (17, 8192, 16384, 4, 128, "k_gemm_mfma"), (64, 2048, 2048, 4, 32, "k_nbits_skinny"),
     (256, 64, 4096, 4, 32, "k_gemm_mfma"), (100, 4096, 4096, 4, 32, "k_gemm_mfma"),
 ])
