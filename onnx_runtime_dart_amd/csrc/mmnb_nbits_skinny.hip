@@ -252,6 +252,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
 #pragma unroll
     for (int i = 0; i < R::kPer; i++) {
       const int row = wid + 8 * i;  // wave-uniform
+      if (row >= M) break;
       // largest and (layout 0) smallest magnitude, NaN from a NaN; then the largest of
       // the wave's 64 lanes as an integer (NaN and infinities above every finite value)
       float mxa = fabsf(av[i][0]), mna = mxa;
@@ -310,7 +311,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
             t[p][e].y = t[p][e].y == t[p][e].y ? t[p][e].y : (_Float16)0.0f;
           }
       }
-      if (STORE && row < M) {  // wave-uniform
+      if (STORE) {
         if (lane == 0) sex[row] = ex;
 #pragma unroll
         for (int p = 0; p < R::kParts; p++) {
@@ -330,7 +331,7 @@ __global__ __launch_bounds__(kSkThreads) void k_nbits_skinny(
           bool miss = false;
 #pragma unroll
           for (int e = 0; e < 8; e++) miss |= fabsf(av[i][e]) < lim && av[i][e] != 0.0f;
-          if (__builtin_amdgcn_ballot_w64(miss) != 0 && lane == 0) srest[wid] = row < M;
+          if (__builtin_amdgcn_ballot_w64(miss) != 0 && lane == 0) srest[wid] = 1;
         }
       }
     }
