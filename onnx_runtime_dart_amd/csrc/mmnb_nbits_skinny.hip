@@ -42,11 +42,11 @@
 //
 // Bound: the launch, one pass of the weights and then latency: a chunk is a
 // serial chain of staging, barrier, LDS reads and MFMAs of two waves per
-// SIMD, 1.4 (M <= 8) to 3.2 us (M <= 32) long; the slice exchange ~2.5 us.
-// us per call back to back, before (k_gemv_lds for M <= 8, else k_prep_a and
-// the GEMM) and now: M = 8, K = N = 4096 13.9 -> 8.8; N = 14336 48.4 -> 14.8;
-// (1024, 6144) 7.6 -> 5.0; M = 12, 4096^2 20.9 -> 9.8; M = 24 21.2 -> 12.6;
-// M = 32 and 256, 1024^2 13.2 -> 6.9 and 14.9 -> 7.8.
+// SIMD, 1.3 (M <= 8) to 2.6 us (M <= 32) long; the slice exchange ~2.5 us.
+// us per call back to back, block 128, before (k_gemv_lds for M <= 8, else
+// k_prep_a and the GEMM) and now: M = 8, K = N = 4096 12.4 -> 8.6; N = 14336
+// 45.9 -> 13.4; (1024, 6144) 6.8 -> 4.3; M = 12, 4096^2 19.3 -> 9.3; M = 24
+// 19.6 -> 11.4; M = 32 and 256, 1024^2 12.5 -> 6.3 and 14.1 -> 6.9.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -50,9 +50,9 @@ namespace mmnb {
 //
 // Against an im2col launch and the MatMulInteger kernel (ConvInteger, us per call, u8
 // x i8, back to back; QLinearConv took 13 us more there for the parameters): 64
-// channels of 56 x 56, 3 x 3 to 64 11.6 -> 6.3; 256 of 14 x 14 to 256 12.9 -> 10.8; 512
-// of 7 x 7 to 512 18.7 -> 16.3; 512 of 28 x 28 to 512 29.0 -> 27.2; 256 of 112 x 112 to
-// 256 104 -> 34.9; 512 of 112 x 112 to 512 243 -> 126.
+// channels of 56 x 56, 3 x 3 to 64 11.5 -> 6.6; 256 of 14 x 14 to 256 12.8 -> 10.7; 512
+// of 7 x 7 to 512 18.9 -> 16.7; 512 of 28 x 28 to 512 28.9 -> 27.4; 256 of 112 x 112 to
+// 256 103 -> 35.0; 512 of 112 x 112 to 512 234 -> 125.
 // ---------------------------------------------------------------------------
 typedef int conv_i4 __attribute__((ext_vector_type(4)));
 typedef uint32_t conv_u4 __attribute__((ext_vector_type(4)));

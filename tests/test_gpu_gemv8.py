@@ -54,7 +54,7 @@ def _problem(m, k, n, bits, bs, zp, bias, seed):
     (24, 4096, 100, 4, 128, False, True),
     (2, 1024, 70, 4, 16, True, True),      # ... through the multi-row GEMV
     (4, 2048, 77, 4, 32, True, True),
-    (5, 2000, 300, 4, 128, False, True),
+    (5, 2000, 300, 4, 128, False, True),   # five rows: the few-row kernel
     (2, 1000, 90, 8, 32, True, True),      # 8-bit planes, gathered for it
     (4, 3, 9, 8, 16, False, True),         # fewer than four values: row by row, the GEMM
     (11, 2, 9, 8, 16, True, False),
@@ -63,7 +63,7 @@ def _problem(m, k, n, bits, bs, zp, bias, seed):
     (1, 1000, 301, 4, 32, True, True),     # ... and one
     (1, 4160, 3, 4, 128, False, True),
 ])
-def test_one_row_gemvs(m, k, n, bits, bs, zp, bias):
+def test_packs_without_a_correction(m, k, n, bits, bs, zp, bias):
     a, b, s, z, bv, nb = _problem(m, k, n, bits, bs, zp, bias, m + k + n)
     y = ops.op_matmul_nbits_ex(a, b, s, z, None, bv, k=k, n=n, bits=bits, block_size=bs,
                                ctx=_lib.default_context())
