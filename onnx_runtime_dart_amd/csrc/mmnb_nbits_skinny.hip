@@ -569,7 +569,9 @@ static int launch_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, in
 //     workgroups: 14.0 against 9.2);
 //   - three or four chunks: 64 columns with a slice per chunk when all of it
 //     stays below one round of the CUs (M = 2, (2048, 2048): 5.6 against 6.6; M = 5,
-//     (1999, 4083), 256 workgroups: 7.8 against 7.2), else as above;
+//     (1999, 4083), 256 workgroups: 7.8 against 7.2; with more than 16 rows in short
+//     blocks also where it is the round, M = 33, 2048^2, block 32: 10.3 against 11.0),
+//     else as above;
 //   - longer K: 64 columns and the slices that fill the CUs (M = 24, 4096^2:
 //     12.6 with 4 slices, 17.5 with 2, 19.3 with 8; 128-column workgroups 21
 //     and more, their registers spill).
@@ -580,26 +582,29 @@ static int launch_skinny(mmnb_ctx *ctx, const mmnb_pack *p, const float *d_a, in
 // 10 where its columns fill three quarters of the CUs (M = 32, (4608, 13824) 26.8 against
 // 29.0, (5120, 13824) 29.4 against 30.4, but (5120, 10240) 28.8 against 27.3, (16384,
 // 16384), 32 chunks, 92 against 77), or, of four slices and more, whose columns the GEMM's
-// tiles leave CUs idle for, 14 ((28672, 4096), block 16 54 against 59).  With more rows, i.e. several row groups, for at most 4 chunks of one round (M = 64, 4096^2: 20.8
-// against 22.3; 28 with the 8 chunks of one slice) or one chunk, more than half filled,
-// of two (M = 2048, 512^2: 12.5 against 20.8; M = 256, N = 4096, K = 384 10.8 against
-// 11.3, K = 256 10.8 against 10.0; four rounds, M = 100, (512, 14336): 19.6 against
+// tiles leave CUs idle for, 14 ((28672, 4096), block 16 54 against 59).  With more rows,
+// i.e. several row groups, for at most 4 chunks of one round (M = 64, 4096^2: 17.9
+// against 19.9; 28 with the 8 chunks of one slice) or one chunk, more than three eighths
+// filled, of two (M = 2048, 512^2: 10.8 against 20.4; M = 256, N = 4096, K = 256 9.8
+// against 10.0, K = 128 9.8 against 8.7; four rounds, M = 100, (512, 14336): 19.6 against
 // 13.2).  Blocks of 16 fill the registers of the two-pass layout: of more than 32 rows
-// two chunks at most (M = 64, four chunks: 30.2 against 23.6; but M = 32, (4096, 14336),
-// eight, 29.6 against 32.5).
+// two chunks at most in 64-column workgroups (M = 64, 4096^2, four: 30.2 against 23.6; but
+// (2048, 4096), four in 32-column ones, 12.0 against 17.9; M = 32, (4096, 14336), eight,
+// 29.6 against 32.5).
 bool nbits_skinny_plan(const mmnb_ctx *ctx, const mmnb_pack *p, int64_t m, int *cw, int *nsl) {
   if (p->generic || m < 2 || !p->few_rows()) return false;
   const int64_t cus = ctx->cu_count, chunks = (p->k + kSkChunk - 1) / kSkChunk;
   const int64_t rows = (m + kSkRows - 1) / kSkRows;
   const int64_t g1 = (p->n + 31) / 32 * rows, g2 = (p->n + 63) / 64 * rows;
-  *cw = chunks <= 4 && g1 <= cus && (chunks <= 2 || g2 * chunks >= cus) ? 1 : 2;
+  const bool round = m <= 16 || p->block >= 64 ? g2 * chunks >= cus : g2 * chunks > cus;
+  *cw = chunks <= 4 && g1 <= cus && (chunks <= 2 || round) ? 1 : 2;
   *nsl = *cw == 1 || g2 > cus
              ? 1
              : (int)std::min<int64_t>({cus / g2, chunks, (int64_t)kSkMaxSlices});
   if (m <= 16) return true;
   const int64_t cps = (chunks + *nsl - 1) / *nsl;
-  if (g2 > cus) return g2 <= 2 * cus && cps == 1 && p->k > kSkChunk / 2;
-  if (m > kSkRows) return cps <= (p->block == 16 ? 2 : 4);
+  if (g2 > cus) return g2 <= 2 * cus && cps == 1 && p->k > 3 * kSkChunk / 8;
+  if (m > kSkRows) return cps <= (p->block == 16 && *cw == 2 ? 2 : 4);
   return cps <= (*nsl >= 4 ? 14 : 4 * g2 > 3 * cus ? 10 : 8);
 }
 

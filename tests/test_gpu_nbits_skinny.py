@@ -40,6 +40,7 @@ CASES = [
     (3, 859, 33, 128, False),      # rows of no alignment: K % 4 = 3, 2, 1
     (20, 1514, 65, 32, True),
     (54, 2001, 64, 128, False),
+    (40, 2000, 2100, 16, True),    # two row groups, four chunks in 32-column workgroups
     (2, 5, 7, 16, True),
     (4, 3, 5, 16, False),          # fewer than four values
     (5, 2000, 130, 32, True),
@@ -185,8 +186,10 @@ def test_packs_without_the_copy(lean_ctx, m, k, n, bits, block, zp, bias):
     (16, 4096, 4096, 4, 32, "k_nbits_skinny"), (32, 4096, 256, 4, 32, "k_nbits_skinny"),
     (20, 4096, 256, 4, 16, "k_nbits_skinny"), (20, 8192, 4096, 4, 16, "k_nbits_skinny"),
     (20, 8192, 8320, 4, 16, "k_gemm_mfma"),
+    (64, 2048, 4096, 4, 16, "k_nbits_skinny"), (64, 4096, 4096, 4, 16, "k_gemm_mfma"),
     (17, 8192, 16384, 4, 128, "k_gemm_mfma"), (64, 2048, 2048, 4, 32, "k_nbits_skinny"),
-    (256, 64, 4096, 4, 32, "k_gemm_mfma"), (100, 4096, 4096, 4, 32, "k_gemm_mfma"),
+    (256, 64, 4096, 4, 32, "k_gemm_mfma"), (256, 256, 4096, 4, 32, "k_nbits_skinny"),
+    (100, 4096, 4096, 4, 32, "k_gemm_mfma"),
 ])
 def test_kernel_of_a_call(m, k, n, bits, block, kernel):
     ctx = _lib.default_context()
